@@ -28,7 +28,8 @@ PROBE_LIB = os.path.join(LIB_DIR, "libramnet_lds_probe.so")
 PROBE_SOURCE = "lds_probe.hip"
 
 SOURCES = ("topk_addr.hip", "segment_forward.hip", "segment_scan_f32.hip", "segment_scan_f16.hip",
-           "segment_scan_bf16.hip", "segment_backward.hip", "autoregressive.hip", "capi.hip")
+           "segment_scan_bf16.hip", "segment_level_f32.hip", "segment_level_f16.hip", "segment_level_bf16.hip",
+           "segment_backward.hip", "autoregressive.hip", "capi.hip")
 ARCH = "gfx950"
 
 

@@ -311,6 +311,9 @@ static ramnet::SegmentJob make_segment_job(const void *x, int dtype, const float
     job.Kr = static_cast<int>(r_top_k);
     job.mass_aware = mass_aware ? 1 : 0;
     job.eps = eps;
+    job.x_stride[0] = job.y_stride[0] = H * T * C;
+    job.x_stride[1] = job.y_stride[1] = T * C;
+    job.x_stride[2] = job.y_stride[2] = C;
     return job;
 }
 

@@ -153,6 +153,9 @@ struct SegmentJob {
     // pre-pass for the paired scan (segment_scan_pair.hpp); null otherwise.
     int *flags;
     SavedRows save;           // rows for the segment backward (save.w null: none)
+    // elements between batch rows, heads and tokens of x and y (channels are
+    // adjacent): (B, H, T, C) in memory order unless the caller says otherwise
+    int64_t x_stride[3], y_stride[3];
     int dtype;
     int B, H, T, A, C, Kw, Kr;
     int mass_aware;

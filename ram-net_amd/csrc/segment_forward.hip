@@ -30,6 +30,7 @@
 #include "ramnet_kernels.hpp"
 #include "segment_scan.hpp"
 #include "segment_scan_pair.hpp"
+#include "segment_level.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -81,8 +82,15 @@ struct Plan {
     size_t lds;
     bool pre;     // mass pre-pass + precomputed-gain scan
     int nr = 1;   // slot ranges, scanned one launch each (precomputed-gain form)
-    int tp = 1;   // tokens per wave step: 2 = the paired scan (precomputed-gain form, one range)
+    int tp = 1;   // tokens per wave step: 2 = the paired scan (precomputed-gain form, one range);
+                  // kLevelPlan = the level-scheduled scan (vec channels per lane)
+    int km = 0;   // level-scheduled scan: padded events per token
+    double us = 0;  // and its estimated time
 };
+constexpr int kLevelPlan = 3;
+// Calls of at most this many tokens are never left to the one-token scan: its
+// launch costs more than their levels can.
+constexpr int kLevelAlone = 2 * kScanPad;
 
 // Cost model of one layout, in cycles per token of one round of resident
 // workgroups: a wave's token loop is bound by its dependency chain (LDS
@@ -146,14 +154,14 @@ static bool save_layout_ok(const SavedRows *sv, int vec, int epp, int np, int cs
 // forms: mass wave allowed (mass_ok), precomputed gains allowed (pre_ok);
 // sv: the layout saves rows in those slices.
 static bool plan_layout(int B, int H, int AL, int A_full, int C, int kmax, int elem, int n_cu, int T, bool mass_ok,
-                        bool pre_ok, Plan *out, int64_t *best_cost, const SavedRows *sv = nullptr) {
+                        bool pre_ok, Plan *out, int64_t *best_cost, const SavedRows *sv = nullptr, bool pair_ok = true) {
     const int64_t tt = std::max(1, T);
     const int epp0 = std::min(kWave, std::max(4, pow2_ceil(kmax)));
     bool found = false;
     int64_t best = 0;
     // paired scan: the precomputed-gain form over the whole slot space, one
     // pass of events
-    if (!sv && pre_ok && AL == A_full && AL <= kMaxPairSlots && pair_records_fit(kmax, T)) {
+    if (!sv && pair_ok && pre_ok && AL == A_full && AL <= kMaxPairSlots && pair_records_fit(kmax, T)) {
         for (int epp = 2; epp <= kWave / 2; epp <<= 1) {
             if (epp < kmax)
                 continue;
@@ -236,12 +244,77 @@ static bool plan_layout(int B, int H, int AL, int A_full, int C, int kmax, int e
     return found;
 }
 
+// Padded events per token of the level-scheduled scan (0: top-K too wide).
+int level_events(int kmax) { return kmax <= 4 ? 4 : kmax <= 8 ? 8 : kmax <= 16 ? 16 : 0; }
+
+// A level-scheduled layout, if it is compiled and fits in LDS.
+bool level_layout(int A, int T, int vec, int nw, int kmax, bool mass_aware, Plan *out) {
+    const int km = level_events(kmax);
+    if (km == 0 || !level_layout_compiled(km, vec) || (nw != 1 && nw != 2 && nw != 4) || A > 0xffff ||
+        static_cast<int64_t>(scan_t_pad(std::max(T, 0))) * kmax * 16 > INT_MAX)
+        return false;
+    const size_t lds = level_lds_bytes(A, vec, nw, km, mass_aware);
+    if (static_cast<int64_t>(lds) > kLdsPerCu || static_cast<int64_t>(schedule_lds_bytes(A)) > kLdsPerCu)
+        return false;
+    *out = {vec, kWave / kTile, 1, nw, nw * vec * (kWave / kTile), lds, true};
+    out->tp = kLevelPlan;
+    out->km = km;
+    return true;
+}
+
+// The level-scheduled layout with the least estimated time. A chunk (32
+// tokens) takes a state wave at least `chain` (its LDS round trips and the
+// issue of one wave), or what the waves of a SIMD issue together; times the
+// rounds of resident workgroups. Constants in microseconds and instructions,
+// from MI355X measurements of one call (schedule and scan, bf16, C = 128):
+// 8 heads, T = 2048, A = 1024, K = 8, one workgroup of one wave per CU: 88,
+// 87 and 107 us with 1, 2 and 4 channels per lane; 128 heads, T = 4096: 471
+// us with (4 channels, 4 waves), 609 with (2, 4); 32 heads, T = 8192, A =
+// 4096, K = 16: 936 us with (2, 2), 959 with (1, 4), 1733 with (2, 1), and
+// 3.8 ms with (4, 1), whose 16 events spill registers.
+bool plan_level(int B, int H, int A, int C, int kmax, int n_cu, int T, bool mass_aware, Plan *out) {
+    bool found = false;
+    double best = 0;
+    for (int vec = 4; vec >= 1; vec >>= 1) {
+        for (int nw = kLevelMaxWaves; nw >= 1; nw >>= 1) {
+            Plan p{};
+            if (!level_layout(A, T, vec, nw, kmax, mass_aware, &p))
+                continue;
+            const int64_t units = static_cast<int64_t>(B) * H * ((C + p.cs - 1) / p.cs);
+            const int64_t gran = (static_cast<int64_t>(p.lds) + kLdsGranule - 1) / kLdsGranule * kLdsGranule;
+            const int64_t per_cu = std::min<int64_t>(kLdsPerCu / gran, std::max(1, (p.km > 8 ? 8 : 12) / (nw + 1)));
+            const int64_t rounds = (units + per_cu * n_cu - 1) / (per_cu * n_cu);
+            const int64_t resident = std::min<int64_t>(per_cu, (units + n_cu - 1) / n_cu);
+            const double chain = 0.75 + 0.05 * p.km + 0.012 * p.km * vec;
+            const double wave = 100 + p.km * (14 + 8.5 * vec), mass = 100 + 10 * p.km;  // instructions per chunk
+            const double issue = resident * (nw * wave + mass) / 4 * 6.5 / 2400;  // 6.5 cycles each, as measured
+            double cost = static_cast<double>((T + kTile - 1) / kTile) * rounds * std::max(chain, issue);
+            if (C % p.cs != 0)
+                cost *= 1.2;  // partial slices take the guarded path
+            if (!found || cost < best) {
+                *out = p;
+                out->us = best = cost;
+                found = true;
+            }
+        }
+    }
+    return found;
+}
+
 bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, int T, Plan *out,
-               const SavedRows *sv = nullptr) {
+               const SavedRows *sv = nullptr, bool mass_aware = true) {
     const int kmax = std::max(Kw, Kr);
     if (kmax > 2 * kWave || A < 1)
         return false;
     int64_t cost = 0;
+    // Where a chunk's writes are many for the slots, levels pile up even for
+    // evenly spread addresses. Against the one-token forms: K = 8, T = 1500,
+    // 1.07x at A = 144, 0.77x at A = 64; K = 16, 0.78x at A = 256 (T = 1500)
+    // and 0.6x at 512 (T = 84), 1.5x at A = 1728 (K = 12).
+    const int64_t writes = static_cast<int64_t>(kTile) * kmax;
+    if (!sv && B > 0 && T > 1 && (kmax <= 8 ? 2 * writes <= 3 * static_cast<int64_t>(A) : 5 * writes <= 3 * static_cast<int64_t>(A)) &&
+        plan_level(B, H, A, C, kmax, n_cu, T, mass_aware, out))
+        return true;
     if (sv)  // saving rows: the precomputed-gain form over the whole slot space
         return A <= kMaxPrePassSlots && save_fits(*sv, T) &&
                plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, false, true, out, &cost, sv);
@@ -561,7 +634,7 @@ __device__ __forceinline__ void mass_fetch(const MassLanes<MP, HALF> &ln, const 
 // past the last (b, h) repeating it); LDS holds (a, b) per slot and unit.
 template<int MP, int NU = 1>
 __global__ __launch_bounds__(kWave) void mass_chunk_map_kernel(const SegmentJob job, float2 *maps, int t_pad,
-                                                              int chunk_len) {
+                                                              int chunk_len, int crowded) {
     static_assert(NU == 1 || MP == 1, "several units per wave: one pass of events");
     constexpr int HALF = kWave / NU / 2;
     using L = MassLanes<MP, HALF>;
@@ -573,6 +646,8 @@ __global__ __launch_bounds__(kWave) void mass_chunk_map_kernel(const SegmentJob 
     const int ck = blockIdx.y, nck = gridDim.y;
     const int lane = static_cast<int>(threadIdx.x);
     const int bh = min(static_cast<int>(blockIdx.x) * NU + lane / (2 * HALF), n_bh - 1);
+    if (crowded && !level_crowded(job.flags, n_bh, t_pad, job.T))
+        return;
     const bool wlane = (lane / HALF) % 2 == 0;
     const int A = job.A, Kw = job.Kw, Kr = job.Kr;
     // unit v's maps at cm + v * (A + 2) + 2; [-2]: the no-op slot of padding records
@@ -652,10 +727,13 @@ __global__ __launch_bounds__(kWave) void mass_chunk_map_kernel(const SegmentJob 
 
 // Step 2: one thread per (b, h, slot); the map of chunk c is replaced by
 // (m_start of chunk c, unused).
-__global__ __launch_bounds__(256) void mass_chunk_scan_kernel(const SegmentJob job, float2 *maps, int nck) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void mass_chunk_scan_kernel(const SegmentJob job, float2 *maps, int nck, int crowded) {
     const int A = job.A;
-    if (i >= static_cast<int64_t>(job.B) * job.H * A)
+    const int64_t n = static_cast<int64_t>(job.B) * job.H * A;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (crowded && !level_crowded(job.flags, job.B * job.H, scan_t_pad(job.T), job.T))  // (by whole waves)
+        return;
+    if (i >= n)
         return;
     const int64_t bh = i / A;
     const int a = static_cast<int>(i - bh * A);
@@ -695,7 +773,7 @@ __global__ __launch_bounds__(256) void mass_chunk_scan_kernel(const SegmentJob j
 // (whose predecessor another chunk replays) is flagged.
 template<bool MA, int MP, int AUX = 0, int NU = 1, bool FL = false>
 __global__ __launch_bounds__(kWave) void segment_mass_kernel(const SegmentJob job, int t_pad, int chunk_len,
-                                                            const float2 *starts, const MassAux aux) {
+                                                            const float2 *starts, const MassAux aux, int crowded = 0) {
     static_assert(NU == 1 || (MP == 1 && !AUX), "several units per wave: one pass of events, no AUX");
     static_assert(!(FL && AUX), "flags: the forward pre-pass only");
     constexpr int HALF = kWave / NU / 2;
@@ -708,6 +786,8 @@ __global__ __launch_bounds__(kWave) void segment_mass_kernel(const SegmentJob jo
     const int lane = static_cast<int>(threadIdx.x);
     const int unit = lane / (2 * HALF);
     const int bh = min(static_cast<int>(blockIdx.x) * NU + unit, n_bh - 1);
+    if (AUX == 0 && crowded && !level_crowded(job.flags, n_bh, t_pad, job.T))
+        return;
     const int hl = lane % HALF;
     const bool wlane = (lane / HALF) % 2 == 0;
     const int A = job.A, Kw = job.Kw, Kr = job.Kr;
@@ -1005,9 +1085,9 @@ size_t mass_lds_bytes(int A, bool aux, int nu = 1, bool fl = false) {
 // groups of NU.
 template<bool MA, int MP, int AUX, int NU>
 void launch_replay_units(const SegmentJob &job, int t_pad, int len, int nck, const float2 *starts, const MassAux &aux,
-                         hipStream_t stream) {
+                         int crowded, hipStream_t stream) {
     const unsigned groups = static_cast<unsigned>((job.B * job.H + NU - 1) / NU);
-    const bool fl = !AUX && job.flags;
+    const bool fl = !AUX && job.flags && !crowded;
     const dim3 grid(groups, static_cast<unsigned>(nck));
     if constexpr (!AUX) {
         if (fl) {
@@ -1017,7 +1097,7 @@ void launch_replay_units(const SegmentJob &job, int t_pad, int len, int nck, con
         }
     }
     hipLaunchKernelGGL((segment_mass_kernel<MA, MP, AUX, NU>), grid, dim3(kWave), mass_lds_bytes(job.A, AUX != 0, NU),
-                       stream, job, t_pad, len, starts, aux);
+                       stream, job, t_pad, len, starts, aux, crowded);
 }
 
 // Units per replay wave: four when a token has at most 8 events and the
@@ -1028,37 +1108,38 @@ void launch_replay_units(const SegmentJob &job, int t_pad, int len, int nck, con
 // slower with the time chunks halved to keep the wave count.
 template<bool MA, int MP, int AUX>
 void launch_mass_replay_nu(const SegmentJob &job, int t_pad, int len, int nck, const float2 *starts,
-                           const MassAux &aux, hipStream_t stream) {
+                           const MassAux &aux, int crowded, hipStream_t stream) {
     if constexpr (MP == 1 && !AUX) {
         if (std::max(job.Kw, job.Kr) <= 8 && mass_lds_bytes(job.A, false, 4, job.flags != nullptr) <= 64 * 1024)
-            return launch_replay_units<MA, MP, AUX, 4>(job, t_pad, len, nck, starts, aux, stream);
+            return launch_replay_units<MA, MP, AUX, 4>(job, t_pad, len, nck, starts, aux, crowded, stream);
     }
-    launch_replay_units<MA, MP, AUX, 1>(job, t_pad, len, nck, starts, aux, stream);
+    launch_replay_units<MA, MP, AUX, 1>(job, t_pad, len, nck, starts, aux, crowded, stream);
 }
 
 // `maps` is scratch for the chunk maps (maps_bytes of it); the final masses
-// go to job.mass_out.
+// go to job.mass_out. crowded: only for a call that the level-scheduled scan
+// leaves to the one-token scan.
 template<bool MA, int MP, int AUX>
 hipError_t launch_mass_pass_mp(const SegmentJob &job, int t_pad, int n_cu, void *maps_buf, size_t maps_bytes,
-                               const MassAux &aux, hipStream_t stream) {
+                               const MassAux &aux, hipStream_t stream, int crowded = 0) {
     int len = 0;
     const int nck = mass_chunks(job, maps_bytes, n_cu, &len);
     const unsigned bh = static_cast<unsigned>(job.B * job.H);
     if (nck <= 1) {
-        launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, job.T, 1, nullptr, aux, stream);
+        launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, job.T, 1, nullptr, aux, crowded, stream);
         return hipGetLastError();
     }
     auto *maps = static_cast<float2 *>(maps_buf);
     if (MP == 1 && std::max(job.Kw, job.Kr) <= 8 && static_cast<size_t>(job.A + 2) * 8 * 4 <= 64 * 1024)
         hipLaunchKernelGGL((mass_chunk_map_kernel<1, 4>), dim3((bh + 3) / 4, nck), dim3(kWave),
-                           static_cast<size_t>(job.A + 2) * 8 * 4, stream, job, maps, t_pad, len);
+                           static_cast<size_t>(job.A + 2) * 8 * 4, stream, job, maps, t_pad, len, crowded);
     else
         hipLaunchKernelGGL((mass_chunk_map_kernel<MP>), dim3(bh, nck), dim3(kWave),
-                           static_cast<size_t>(job.A + 2) * 8, stream, job, maps, t_pad, len);
+                           static_cast<size_t>(job.A + 2) * 8, stream, job, maps, t_pad, len, crowded);
     const int64_t n = static_cast<int64_t>(bh) * job.A;
     hipLaunchKernelGGL(mass_chunk_scan_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, job,
-                       maps, nck);
-    launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, len, nck, maps, aux, stream);
+                       maps, nck, crowded);
+    launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, len, nck, maps, aux, crowded, stream);
     return hipGetLastError();
 }
 
@@ -1355,6 +1436,9 @@ static int layout_override(const SegmentJob &job, Plan *p, const char **why) {
         return 0;
     int vec = 0, epp = 0, np = 0, nw = 0, pre = 0, tp = 1;
     const int n = std::sscanf(env, "%d,%d,%d,%d,%d,%d", &vec, &epp, &np, &nw, &pre, &tp);
+    if (n == 6 && tp == kLevelPlan && pre == 1 && np == 1 && epp == kWave / kTile &&
+        level_layout(job.A, job.T, vec, nw, std::max(job.Kw, job.Kr), job.mass_aware != 0, p))
+        return 1;
     const bool pair = n == 6 && tp == 2;
     const bool named = pair ? pre == 1 && np == 1 && scan_pair_layout_compiled(vec, epp, nw)
                             : (n >= 4 && n <= 6) && (pre == 0 || pre == 1) && tp == 1 &&
@@ -1396,7 +1480,8 @@ static bool pick_plan(const SegmentJob &job, Plan *p, const char **why) {
     const int forced = layout_override(job, p, why);
     if (forced < 0)
         return false;
-    if (!forced && !make_plan(job.B, job.H, job.A, job.C, job.Kw, job.Kr, dtype_bytes(job.dtype), cu_count(), job.T, p)) {
+    if (!forced && !make_plan(job.B, job.H, job.A, job.C, job.Kw, job.Kr, dtype_bytes(job.dtype), cu_count(), job.T, p, nullptr,
+                              job.mass_aware != 0)) {
         *why = "segment forward: shape outside the LDS-resident scan (top_k <= 128; slot spaces wider than one "
                "resident slice are scanned in at most 4096 slot ranges)";
         return false;
@@ -1435,6 +1520,100 @@ bool segment_forward_can_save(int B, int H, int T, int A, int C, int Kw, int Kr,
     return make_plan(B, H, A, C, Kw, Kr, dtype_bytes(dtype), cu_count(), T, &p, &geo);
 }
 
+static hipError_t launch_scan_layout(const SegmentJob &job, const ScanGeom &geo, const Plan &p, hipStream_t stream) {
+    switch (job.dtype) {
+        case kF32: return launch_scan_f32(job, geo, p.vec, p.epp, p.np, p.nw, p.pre, stream);
+        case kF16: return launch_scan_f16(job, geo, p.vec, p.epp, p.np, p.nw, p.pre, stream);
+        default: return launch_scan_bf16(job, geo, p.vec, p.epp, p.np, p.nw, p.pre, stream);
+    }
+}
+
+// A call that the level-scheduled scan leaves as too crowded: the one-token
+// scan, whose waves return at once otherwise. It runs before the
+// level-scheduled scan: a pre-pass that is not needed leaves y and the final
+// masses alone, and one that is has read what it needs of the schedule
+// before the gain records replace it. Each launch that returns at once takes
+// about 4 us, so the pre-pass form is for calls of kCrowdedPreUs and more.
+constexpr double kCrowdedPreUs = 200;
+static hipError_t launch_crowded(const SegmentJob &job, double us, hipStream_t stream, const char **why) {
+    Plan p{};
+    int64_t cost = 0;
+    const int t_pad = scan_t_pad(job.T), n_cu = cu_count();
+    const SavedRows *none = nullptr;
+    if (!plan_layout(job.B, job.H, job.A, job.A, job.C, std::max(job.Kw, job.Kr), dtype_bytes(job.dtype), n_cu, job.T,
+                     true, us >= kCrowdedPreUs, &p, &cost, none, false)) {
+        *why = "segment forward: no one-token layout for a crowded call";
+        return hipErrorInvalidValue;
+    }
+    ScanGeom geo{};
+    geo.n_slices = (job.C + p.cs - 1) / p.cs;
+    geo.n_units = job.B * job.H * geo.n_slices;
+    geo.n_chunks = (job.T + kChunk - 1) / kChunk;
+    geo.t_pad = t_pad;
+    geo.n_local = job.A;
+    geo.last = 1;
+    geo.crowded = 1;
+    if (p.pre) {
+        const size_t y_bytes = static_cast<size_t>(job.B) * job.H * job.T * job.C * dtype_bytes(job.dtype);
+        const MassAux none_aux{};
+        const hipError_t err = job.mass_aware
+                                   ? launch_mass_pass_mp<true, 1, 0>(job, t_pad, n_cu, job.y, y_bytes, none_aux, stream, 1)
+                                   : launch_mass_pass_mp<false, 1, 0>(job, t_pad, n_cu, job.y, y_bytes, none_aux, stream, 1);
+        if (err != hipSuccess)
+            return err;
+    }
+    return launch_scan_layout(job, geo, p, stream);
+}
+
+// Event schedule, then the scan.
+static hipError_t launch_level_scan(const SegmentJob &job, const Plan &p, hipStream_t stream, const char **why) {
+    if (!job.gain || !job.flags) {
+        *why = "segment forward: the level-scheduled scan needs the schedule part of the scan workspace";
+        return hipErrorInvalidValue;
+    }
+    if (job.dtype != kF32 && job.dtype != kF16 && job.dtype != kBF16) {
+        *why = "segment forward: unsupported dtype";
+        return hipErrorInvalidValue;
+    }
+    const int t_pad = scan_t_pad(job.T);
+    const dim3 grid(static_cast<unsigned>((t_pad + kWave - 1) / kWave) * static_cast<unsigned>(job.B * job.H));
+    const size_t lds = schedule_lds_bytes(job.A);
+    if (p.km == 4)
+        hipLaunchKernelGGL((segment_schedule_kernel<4>), grid, dim3(kWave), lds, stream, job, t_pad);
+    else if (p.km == 8)
+        hipLaunchKernelGGL((segment_schedule_kernel<8>), grid, dim3(kWave), lds, stream, job, t_pad);
+    else
+        hipLaunchKernelGGL((segment_schedule_kernel<16>), grid, dim3(kWave), lds, stream, job, t_pad);
+    if (const hipError_t err = hipGetLastError(); err != hipSuccess)
+        return err;
+    LevelGeom geo{};
+    geo.n_slices = (job.C + p.cs - 1) / p.cs;
+    geo.n_units = job.B * job.H * geo.n_slices;
+    geo.t_pad = t_pad;
+    geo.nw = p.nw;
+    geo.leave_crowded = job.T > kLevelAlone;
+    if (geo.leave_crowded) {
+        if (const hipError_t err = launch_crowded(job, p.us, stream, why); err != hipSuccess)
+            return err;
+    }
+    // whole slices, and x and y aligned for VEC elements at a time
+    const int es = dtype_bytes(job.dtype);
+    auto aligned = [&](const void *q, const int64_t (&st)[3]) {
+        uint64_t bits = reinterpret_cast<uintptr_t>(q);
+        for (int64_t v : st)
+            bits |= static_cast<uint64_t>(v * es);
+        return bits % static_cast<unsigned>(p.vec * es) == 0;
+    };
+    auto spans = [&](const int64_t (&st)[3]) { return ((job.T + kTile) * st[2] + job.C) * es <= INT_MAX; };
+    const bool full = job.C % p.cs == 0 && aligned(job.x, job.x_stride) && aligned(job.y, job.y_stride) &&
+                      spans(job.x_stride) && spans(job.y_stride);
+    switch (job.dtype) {
+        case kF32: return launch_level_f32(job, geo, p.vec, p.km, full, stream);
+        case kF16: return launch_level_f16(job, geo, p.vec, p.km, full, stream);
+        default: return launch_level_bf16(job, geo, p.vec, p.km, full, stream);
+    }
+}
+
 hipError_t launch_segment_forward(const SegmentJob &job, hipStream_t stream, const char **why) {
     if (static_cast<int64_t>(job.B) * job.H == 0)
         return hipSuccess;
@@ -1460,6 +1639,8 @@ hipError_t launch_segment_forward(const SegmentJob &job, hipStream_t stream, con
         *why = "segment forward: the paired layout needs the flags of the scan workspace";
         return hipErrorInvalidValue;
     }
+    if (p.tp == kLevelPlan)
+        return launch_level_scan(job, p, stream, why);
     // the pre-pass writes the paired scan's flags only when it runs
     SegmentJob pj = job;
     if (p.tp != 2)
@@ -1515,11 +1696,7 @@ hipError_t launch_segment_forward(const SegmentJob &job, hipStream_t stream, con
         geo.n_local = std::min(al, job.A - geo.r0);
         geo.last = r == p.nr - 1 ? 1 : 0;
         hipError_t err;
-        switch (job.dtype) {
-            case kF32: err = launch_scan_f32(job, geo, p.vec, p.epp, p.np, p.nw, p.pre, stream); break;
-            case kF16: err = launch_scan_f16(job, geo, p.vec, p.epp, p.np, p.nw, p.pre, stream); break;
-            default: err = launch_scan_bf16(job, geo, p.vec, p.epp, p.np, p.nw, p.pre, stream); break;
-        }
+        err = launch_scan_layout(job, geo, p, stream);
         if (err != hipSuccess)
             return err;
     }

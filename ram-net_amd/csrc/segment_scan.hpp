@@ -40,7 +40,46 @@ struct ScanGeom {
     int r0;
     int n_local;
     int last;
+    // 1: only a call that the level-scheduled scan leaves to this one
+    int crowded = 0;
 };
+
+// Whether a call's addresses are too concentrated for the level-scheduled
+// scan (segment_level.hpp): each of its levels costs it about a third of a
+// chunk's level-0 pass however few events it holds, and its slowest heads
+// decide, so beyond kCrowdedMean late levels per 32-token chunk on average,
+// or with more than one chunk in kCrowdedPart past kCrowdedLevels, the
+// one-token scan takes the call. Both are launched and decide alike from the
+// schedule's counts (in the flags of the workspace: word 0 of each chunk,
+// bits 0..7) of at most 256 chunks spread over the call. At config 2 sizes
+// with a mean of m late levels: 280 + 82 m us against 725 us (m = 2.3 on the
+// benchmark data). Called by whole waves.
+constexpr int kCrowdedMean = 5;
+constexpr int kCrowdedLevels = 14;
+constexpr int kCrowdedPart = 16;
+__device__ __forceinline__ bool level_crowded(const int *flags, int n_heads, int t_pad, int T) {
+    const int lane = static_cast<int>(threadIdx.x % kWave), nc = (T + kScanPad - 1) / kScanPad;
+    const int64_t total = static_cast<int64_t>(n_heads) * nc;
+    const int n = static_cast<int>(min(total, static_cast<int64_t>(4 * kWave)));
+    int levels[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int64_t c = min(i * kWave + lane, n - 1) * total / n;
+        const int64_t bh = c / nc;
+        levels[i] = flags[bh * t_pad + (c - bh * nc) * kScanPad] & 0xff;
+    }
+    int sum = 0, many = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool in = i * kWave + lane < n;
+        sum += in ? levels[i] : 0;
+        many += __popcll(__ballot(in && levels[i] > kCrowdedLevels));
+    }
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1)
+        sum += __shfl_xor(sum, d);
+    return __builtin_amdgcn_readfirstlane(sum) > kCrowdedMean * n || many * kCrowdedPart > n;
+}
 
 // 1/d refined by one Newton step; gain = w / (m + eps) to ~1 ulp.
 __device__ __forceinline__ float scan_gain(float w, float d) {
@@ -426,6 +465,8 @@ __device__ __forceinline__ void segment_scan_body(const SegmentJob &job, const S
     const int bh = unit / geo.n_slices;
     const int c0 = (unit - bh * geo.n_slices) * CS;
     const int T = job.T, A = job.A, C = job.C, Kw = job.Kw, Kr = job.Kr, Tp = geo.t_pad;
+    if (geo.crowded && !level_crowded(job.flags, job.B * job.H, Tp, T))
+        return;
     const float eps = job.eps;
     // resident slot range: [r0, r0 + AL) (the whole space but in the
     // split launches of a wide one)
