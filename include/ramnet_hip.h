@@ -281,6 +281,34 @@ int ramnet_ram_attn_forward(const void *w_addr, const void *r_addr, const void *
                             float eps, void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
+ * ramnet_ram_attn_forward and ramnet_topk_addr_forward on tensors that need
+ * not be in memory order, so that activations laid out (B, T, H, ...) are
+ * taken where they are. `strides` (host memory, elements, >= 0; every tensor
+ * within int32 elements of its start):
+ *   ram_attn_forward   w_addr [b, h, u, p, t], r_addr [b, h, u, p, t],
+ *                      x [b, h, t], y [b, h, t], gamma [b, h, t],
+ *                      position_ids [b, t]   (21 values)
+ *   topk_addr_forward  w_addr [b, h, u, p, t], r_addr [b, h, u, p, t],
+ *                      position_ids [b, t]   (12 values)
+ * Digits follow each other at P times the logits' stride; channels of x and
+ * y are adjacent; y's rows fill B * H * T * C elements (they may be in any
+ * order of b, h and t). Outputs other than y, the state and the mask are in
+ * memory order.
+ */
+int ramnet_ram_attn_forward_strided(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
+                                    int dtype, const uint8_t *mask, int64_t embed_num, const int32_t *position_ids,
+                                    const float *init_slot, const float *init_mass, float *slot_out, float *mass_out,
+                                    void *y, int64_t B, int64_t H, int64_t U, int64_t P, int64_t T, int64_t A,
+                                    int64_t C, int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
+                                    int mass_aware, float eps, const int64_t *strides, void *workspace,
+                                    int64_t workspace_bytes, void *stream);
+int ramnet_topk_addr_forward_strided(const void *w_addr, const void *r_addr, int dtype, int64_t B, int64_t H,
+                                     int64_t U, int64_t P, int64_t T, int64_t embed_num, int64_t A,
+                                     const int32_t *position_ids, int64_t w_top_k, int64_t r_top_k, float w_re_norm,
+                                     float r_re_norm, int encode_batch_idx, const int64_t *strides, int32_t *idx_out,
+                                     float *val_out, void *stream);
+
+/*
  * One fused decode step on a persistent state, updated in place.
  * Replaces ramnet_ops::topk_autoregressive_ (ram_attn_bind.cpp:92-101,
  * ram_attn_ops.cpp:349-394).

@@ -6,6 +6,7 @@
 #include "ramnet_kernels.hpp"
 #include "ramnet_search.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <stdio.h>
@@ -67,6 +68,68 @@ int check_addr_shape(int64_t B, int64_t H, int64_t U, int64_t P, int64_t T, int6
     return RAMNET_OK;
 }
 
+// Strides, in elements, of a call's tensors.
+struct Layout {
+    int64_t w[5], r[5];  // logits: b, h, u, p, t
+    int64_t x[3], y[3];  // b, h, t; channels adjacent
+    int64_t gamma[3];    // b, h, t
+    int64_t pos[2];      // b, t
+};
+
+Layout memory_order(int64_t B, int64_t H, int64_t U, int64_t P, int64_t T, int64_t C) {
+    (void)B;
+    return {{H * U * P * T, U * P * T, P * T, T, 1},
+            {H * U * P * T, U * P * T, P * T, T, 1},
+            {H * T * C, T * C, C},
+            {H * T * C, T * C, C},
+            {H * T, T, 1},
+            {T, 1}};
+}
+
+// Whether every element lies within int32 reach of the tensor's start.
+bool stride_ok(const int64_t *stride, std::initializer_list<int64_t> sizes) {
+    int64_t far = 0;
+    int i = 0;
+    for (int64_t n : sizes) {
+        const int64_t s = stride[i++];
+        if (s < 0 || (n > 1 && s > kIntMax / (n - 1)))
+            return false;
+        far += n > 1 ? s * (n - 1) : 0;
+    }
+    return far < kIntMax;
+}
+
+// Whether rows of C elements at these strides fill B * H * T * C elements.
+bool stride_dense(const int64_t *stride, int64_t B, int64_t H, int64_t T, int64_t C) {
+    int64_t n[3] = {B, H, T}, next = C;
+    for (int done = 0; done < 3; ++done) {
+        int at = -1;
+        for (int d = 0; d < 3; ++d)
+            if (n[d] == 1 || (n[d] > 0 && stride[d] == next))
+                at = at < 0 || n[d] == 1 ? d : at;
+        if (at < 0)
+            return false;
+        next *= n[at];
+        n[at] = 0;  // taken
+    }
+    return true;
+}
+
+void set_source(ramnet::AddrSource &src, const int64_t (&s)[5]) {
+    src.stride[0] = s[0];
+    src.stride[1] = s[1];
+    src.stride[2] = s[4];
+    src.step = static_cast<int>(s[3]);
+}
+
+// The logits' strides: one step from each logit of an address to the next.
+int check_logits(const int64_t (&s)[5], int64_t B, int64_t H, int64_t U, int64_t P, int64_t T) {
+    RAMNET_REQUIRE(stride_ok(s, {B, H, U, P, T}), "address strides must be >= 0 and within int32");
+    RAMNET_REQUIRE((U == 1 || s[2] == P * s[3]) && U * P * s[3] < kIntMax,
+                   "address strides: digits must follow each other at P times the logits' stride");
+    return RAMNET_OK;
+}
+
 
 // One decoder source of a backward call (the k rows k_off .. k_off + top_k).
 int addr_backward(const int32_t *idx, const float *val, const void *addr, const float *grad_val, int dtype,
@@ -124,6 +187,10 @@ int ramnet_topk_addr_single_forward(const void *addr, int dtype, int64_t B, int6
     ramnet::AddrJob job{};
     job.src[0] = {addr, static_cast<int>(top_k), top_k_re_norm, addr_val_neg ? -1.f : 1.f, 0};
     job.n_src = 1;
+    const Layout lay = memory_order(B, H, U, P, T, 1);
+    set_source(job.src[0], lay.w);
+    job.pos_stride[0] = lay.pos[0];
+    job.pos_stride[1] = lay.pos[1];
     job.dtype = dtype;
     job.B = static_cast<int>(B);
     job.H = static_cast<int>(H);
@@ -184,10 +251,11 @@ int ramnet_topk_addr_backward(const int32_t *idx, const float *val, const void *
                          r_top_k, r_re_norm, -1.f, grad_r_addr, stream);
 }
 
-int ramnet_topk_addr_forward(const void *w_addr, const void *r_addr, int dtype, int64_t B, int64_t H, int64_t U,
+static int topk_addr_forward(const void *w_addr, const void *r_addr, int dtype, int64_t B, int64_t H, int64_t U,
                              int64_t P, int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
                              int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
-                             int encode_batch_idx, int32_t *idx_out, float *val_out, void *stream) {
+                             int encode_batch_idx, const Layout &lay, int32_t *idx_out, float *val_out,
+                             void *stream) {
     if (int rc = check_addr_shape(B, H, U, P, T, embed_num, A))
         return rc;
     RAMNET_REQUIRE(valid_dtype(dtype), "addr dtype must be float32, float16 or bfloat16");
@@ -199,10 +267,19 @@ int ramnet_topk_addr_forward(const void *w_addr, const void *r_addr, int dtype, 
     if (B * T == 0)
         return RAMNET_OK;
     RAMNET_REQUIRE(w_addr && r_addr && position_ids && idx_out && val_out, "null tensor pointer");
+    if (int rc = check_logits(lay.w, B, H, U, P, T))
+        return rc;
+    if (int rc = check_logits(lay.r, B, H, U, P, T))
+        return rc;
+    RAMNET_REQUIRE(stride_ok(lay.pos, {B, T}), "position strides must be >= 0 and within int32");
     ramnet::AddrJob job{};
     job.src[0] = {w_addr, static_cast<int>(w_top_k), w_re_norm, 1.f, 0};
     job.src[1] = {r_addr, static_cast<int>(r_top_k), r_re_norm, -1.f, static_cast<int>(w_top_k)};
     job.n_src = 2;
+    set_source(job.src[0], lay.w);
+    set_source(job.src[1], lay.r);
+    job.pos_stride[0] = lay.pos[0];
+    job.pos_stride[1] = lay.pos[1];
     job.dtype = dtype;
     job.B = static_cast<int>(B);
     job.H = static_cast<int>(H);
@@ -219,6 +296,29 @@ int ramnet_topk_addr_forward(const void *w_addr, const void *r_addr, int dtype, 
     const char *why = nullptr;
     const hipError_t err = ramnet::launch_topk_addr(job, static_cast<hipStream_t>(stream), &why);
     return finish(err, why, "topk_addr_forward launch");
+}
+
+int ramnet_topk_addr_forward(const void *w_addr, const void *r_addr, int dtype, int64_t B, int64_t H, int64_t U,
+                             int64_t P, int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
+                             int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
+                             int encode_batch_idx, int32_t *idx_out, float *val_out, void *stream) {
+    return topk_addr_forward(w_addr, r_addr, dtype, B, H, U, P, T, embed_num, A, position_ids, w_top_k, r_top_k,
+                             w_re_norm, r_re_norm, encode_batch_idx, memory_order(B, H, U, P, T, 1), idx_out, val_out,
+                             stream);
+}
+
+int ramnet_topk_addr_forward_strided(const void *w_addr, const void *r_addr, int dtype, int64_t B, int64_t H,
+                                     int64_t U, int64_t P, int64_t T, int64_t embed_num, int64_t A,
+                                     const int32_t *position_ids, int64_t w_top_k, int64_t r_top_k, float w_re_norm,
+                                     float r_re_norm, int encode_batch_idx, const int64_t *strides, int32_t *idx_out,
+                                     float *val_out, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    Layout lay{};
+    std::copy_n(strides, 5, lay.w);
+    std::copy_n(strides + 5, 5, lay.r);
+    std::copy_n(strides + 10, 2, lay.pos);
+    return topk_addr_forward(w_addr, r_addr, dtype, B, H, U, P, T, embed_num, A, position_ids, w_top_k, r_top_k,
+                             w_re_norm, r_re_norm, encode_batch_idx, lay, idx_out, val_out, stream);
 }
 
 // Decoder records, then the gain records of the precomputed-gain scan and
@@ -410,7 +510,7 @@ int ramnet_topk_segment_forward_(const int32_t *addr_idx, const float *addr_val,
 static int addr_records(const void *w_addr, const void *r_addr, const void *gamma, int dtype, const uint8_t *mask,
                         int64_t embed_num, const int32_t *position_ids, int64_t B, int64_t H, int64_t U, int64_t P,
                         int64_t T, int64_t A, int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
-                        void *workspace, int64_t workspace_bytes, int64_t need, void *stream) {
+                        const Layout &at, void *workspace, int64_t workspace_bytes, int64_t need, void *stream) {
     if (int rc = check_addr_shape(B, H, U, P, T, embed_num, A))
         return rc;
     RAMNET_REQUIRE(valid_dtype(dtype), "addr dtype must be float32, float16 or bfloat16");
@@ -425,12 +525,22 @@ static int addr_records(const void *w_addr, const void *r_addr, const void *gamm
     if (B * T == 0)
         return RAMNET_OK;
     RAMNET_REQUIRE(w_addr && r_addr && gamma && position_ids, "null tensor pointer");
+    if (int rc = check_logits(at.w, B, H, U, P, T))
+        return rc;
+    if (int rc = check_logits(at.r, B, H, U, P, T))
+        return rc;
+    RAMNET_REQUIRE(stride_ok(at.pos, {B, T}) && stride_ok(at.gamma, {B, H, T}),
+                   "position and gamma strides must be >= 0 and within int32");
     ramnet::SegmentJob lay = make_segment_job(nullptr, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, T,
                                               A, 1, w_top_k, r_top_k, 0, 1.f, workspace);
     ramnet::AddrJob dec{};
     dec.src[0] = {w_addr, static_cast<int>(w_top_k), w_re_norm, 1.f, 0};
     dec.src[1] = {r_addr, static_cast<int>(r_top_k), r_re_norm, 1.f, 0};
     dec.n_src = 2;
+    set_source(dec.src[0], at.w);
+    set_source(dec.src[1], at.r);
+    std::copy_n(at.pos, 2, dec.pos_stride);
+    std::copy_n(at.gamma, 3, dec.gamma_stride);
     dec.dtype = dtype;
     dec.B = static_cast<int>(B);
     dec.H = static_cast<int>(H);
@@ -453,8 +563,8 @@ static int addr_records(const void *w_addr, const void *r_addr, const void *gamm
 
 static int segment_scan(const void *x, int dtype, const float *init_slot, const float *init_mass, float *slot_out,
                         float *mass_out, void *y, int64_t B, int64_t H, int64_t T, int64_t A, int64_t C,
-                        int64_t w_top_k, int64_t r_top_k, int mass_aware, float eps, void *workspace,
-                        int64_t workspace_bytes, int64_t need, void *stream) {
+                        int64_t w_top_k, int64_t r_top_k, int mass_aware, float eps, const Layout &at,
+                        void *workspace, int64_t workspace_bytes, int64_t need, void *stream) {
     if (int rc = segment_checks(x, x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C, w_top_k,
                                 r_top_k, eps, workspace, workspace_bytes, need))
         return rc;
@@ -462,6 +572,10 @@ static int segment_scan(const void *x, int dtype, const float *init_slot, const 
         return RAMNET_OK;
     ramnet::SegmentJob job = make_segment_job(x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C,
                                               w_top_k, r_top_k, mass_aware, eps, workspace);
+    RAMNET_REQUIRE(T == 0 || (stride_ok(at.x, {B, H, T}) && stride_dense(at.y, B, H, T, C)),
+                   "x strides must be >= 0 and within int32, y's rows must fill B * H * T * C elements");
+    std::copy_n(at.x, 3, job.x_stride);
+    std::copy_n(at.y, 3, job.y_stride);
     const char *why = nullptr;
     const hipError_t err = ramnet::launch_segment_forward(job, static_cast<hipStream_t>(stream), &why);
     return finish(err, why, "segment_scan launch");
@@ -472,17 +586,18 @@ static int ram_attn_forward(const void *w_addr, const void *r_addr, const void *
                             const float *init_slot, const float *init_mass, float *slot_out, float *mass_out, void *y,
                             int64_t B, int64_t H, int64_t U, int64_t P, int64_t T, int64_t A, int64_t C,
                             int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm, int mass_aware,
-                            float eps, void *workspace, int64_t workspace_bytes, int64_t need, void *stream) {
+                            float eps, const Layout &at, void *workspace, int64_t workspace_bytes, int64_t need,
+                            void *stream) {
     if (int rc = segment_checks(x, gamma, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C, w_top_k,
                                 r_top_k, eps, workspace, workspace_bytes, need))
         return rc;
     if (B > 0 && T > 0) {
         if (int rc = addr_records(w_addr, r_addr, gamma, dtype, mask, embed_num, position_ids, B, H, U, P, T, A,
-                                  w_top_k, r_top_k, w_re_norm, r_re_norm, workspace, workspace_bytes, need, stream))
+                                  w_top_k, r_top_k, w_re_norm, r_re_norm, at, workspace, workspace_bytes, need, stream))
             return rc;
     }
     return segment_scan(x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C, w_top_k, r_top_k,
-                        mass_aware, eps, workspace, workspace_bytes, need, stream);
+                        mass_aware, eps, at, workspace, workspace_bytes, need, stream);
 }
 
 int ramnet_topk_addr_records(const void *w_addr, const void *r_addr, const void *gamma, int dtype,
@@ -491,7 +606,8 @@ int ramnet_topk_addr_records(const void *w_addr, const void *r_addr, const void 
                              float w_re_norm, float r_re_norm, void *workspace, int64_t workspace_bytes,
                              void *stream) {
     return addr_records(w_addr, r_addr, gamma, dtype, mask, embed_num, position_ids, B, H, U, P, T, A, w_top_k,
-                        r_top_k, w_re_norm, r_re_norm, workspace, workspace_bytes, -1, stream);
+                        r_top_k, w_re_norm, r_re_norm, memory_order(B, H, U, P, T, 1), workspace, workspace_bytes,
+                        -1, stream);
 }
 
 int ramnet_segment_scan(const void *x, int dtype, const float *init_slot, const float *init_mass, float *slot_out,
@@ -499,7 +615,7 @@ int ramnet_segment_scan(const void *x, int dtype, const float *init_slot, const 
                         int64_t w_top_k, int64_t r_top_k, int mass_aware, float eps, void *workspace,
                         int64_t workspace_bytes, void *stream) {
     return segment_scan(x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C, w_top_k, r_top_k,
-                        mass_aware, eps, workspace, workspace_bytes, -1, stream);
+                        mass_aware, eps, memory_order(B, H, 1, 1, T, C), workspace, workspace_bytes, -1, stream);
 }
 
 int ramnet_ram_attn_forward(const void *w_addr, const void *r_addr, const void *x, const void *gamma, int dtype,
@@ -510,7 +626,27 @@ int ramnet_ram_attn_forward(const void *w_addr, const void *r_addr, const void *
                             float eps, void *workspace, int64_t workspace_bytes, void *stream) {
     return ram_attn_forward(w_addr, r_addr, x, gamma, dtype, mask, embed_num, position_ids, init_slot, init_mass,
                             slot_out, mass_out, y, B, H, U, P, T, A, C, w_top_k, r_top_k, w_re_norm, r_re_norm,
-                            mass_aware, eps, workspace, workspace_bytes, -1, stream);
+                            mass_aware, eps, memory_order(B, H, U, P, T, C), workspace, workspace_bytes, -1, stream);
+}
+
+int ramnet_ram_attn_forward_strided(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
+                                    int dtype, const uint8_t *mask, int64_t embed_num, const int32_t *position_ids,
+                                    const float *init_slot, const float *init_mass, float *slot_out, float *mass_out,
+                                    void *y, int64_t B, int64_t H, int64_t U, int64_t P, int64_t T, int64_t A,
+                                    int64_t C, int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
+                                    int mass_aware, float eps, const int64_t *strides, void *workspace,
+                                    int64_t workspace_bytes, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    Layout at{};
+    std::copy_n(strides, 5, at.w);
+    std::copy_n(strides + 5, 5, at.r);
+    std::copy_n(strides + 10, 3, at.x);
+    std::copy_n(strides + 13, 3, at.y);
+    std::copy_n(strides + 16, 3, at.gamma);
+    std::copy_n(strides + 19, 2, at.pos);
+    return ram_attn_forward(w_addr, r_addr, x, gamma, dtype, mask, embed_num, position_ids, init_slot, init_mass,
+                            slot_out, mass_out, y, B, H, U, P, T, A, C, w_top_k, r_top_k, w_re_norm, r_re_norm,
+                            mass_aware, eps, at, workspace, workspace_bytes, -1, stream);
 }
 
 static int64_t backward_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t Kw,
@@ -886,7 +1022,8 @@ int ramnet_ram_attn_forward_noalloc(const void *w_addr, const void *r_addr, cons
     }
     return ram_attn_forward(w_addr, r_addr, x, gamma, dtype, mask, embed_num, position_ids, init_slot, init_mass,
                             slot_out, mass_out, y, B, H, U, P, T, A, C, w_top_k, r_top_k, w_re_norm, r_re_norm,
-                            mass_aware, eps, ws, RAMNET_NOALLOC_SCRATCH_BYTES, need, stream);
+                            mass_aware, eps, memory_order(B, H, U, P, T, C), ws, RAMNET_NOALLOC_SCRATCH_BYTES, need,
+                            stream);
 }
 
 }  // extern "C"

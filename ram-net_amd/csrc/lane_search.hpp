@@ -241,10 +241,14 @@ __device__ __forceinline__ uint64_t prefix_key(float s, int c) {
 // reads through one buffer resource based at the wave's first lane with
 // 32-bit per-lane offsets, which keeps the per-load addresses out of scalar
 // registers (the host picks it when every offset fits in 31 bits).
+// RowLogits reads an address whose U * P logits are adjacent, 16 bytes (a
+// whole digit, if it is shorter) at a time: PIECE bytes divide a digit, and
+// every address starts on a multiple of them.
 template<typename Scalar>
 struct GlobalLogits {
+    static constexpr bool kRows = false;
     const Scalar *base;  // logit 0 of digit 0 for this lane
-    int stride;          // elements between consecutive logits (T); U * P * T fits an int
+    int stride;          // elements between consecutive logits; U * P * stride fits an int
     int P;
     __device__ __forceinline__ uint32_t operator()(int u, int p) const {
         return raw_bits<Scalar>(base + (u * P + p) * stride);
@@ -252,6 +256,7 @@ struct GlobalLogits {
 };
 template<typename Scalar>
 struct BufferLogits {
+    static constexpr bool kRows = false;
     __amdgpu_buffer_rsrc_t rsrc;
     int lane_off;  // bytes from the resource base to this lane's logit 0 of digit 0
     int step;      // bytes between consecutive logits (T * sizeof(Scalar))
@@ -262,6 +267,35 @@ struct BufferLogits {
             return __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0);
         else
             return __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0);
+    }
+};
+template<typename Scalar, int NP>
+constexpr int row_piece_bytes() {
+    const int digit = NP * static_cast<int>(sizeof(Scalar));
+    return digit < 16 ? digit : 16;
+}
+// FULL: P == NP; otherwise the pieces past the digit repeat its last one.
+template<typename Scalar, int NP, bool FULL>
+struct RowLogits {
+    static constexpr bool kRows = true;
+    const Scalar *base;  // logit 0 of digit 0 for this lane
+    int P;
+    __device__ __forceinline__ void digit(int u, uint32_t (&bits)[NP]) const {
+        constexpr int ES = static_cast<int>(sizeof(Scalar));
+        constexpr int PIECE = row_piece_bytes<Scalar, NP>(), N = NP * ES / PIECE, E = PIECE / ES;
+        typedef uint32_t Words __attribute__((ext_vector_type(PIECE / 4)));
+        const char *row = reinterpret_cast<const char *>(base + u * P);
+        const int last = P * ES / PIECE - 1;
+        Words w[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            w[i] = *reinterpret_cast<const Words *>(row + (FULL || i < last ? i : last) * PIECE);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                bits[i * E + e] = ES == 4 ? w[i][e] : (w[i][e / 2] >> (e % 2 * 16)) & 0xFFFFu;
+        }
     }
 };
 
@@ -279,9 +313,13 @@ __device__ __forceinline__ bool digit_top(const Load &load, int u, int P_, float
     // logit. A guarded load or a branch on P would wait for each load's data
     // before issuing the next.
     uint32_t bits[NP];
+    if constexpr (Load::kRows) {
+        load.digit(u, bits);
+    } else {
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-        bits[p] = load(u, p < P ? p : P - 1);
+        for (int p = 0; p < NP; ++p)
+            bits[p] = load(u, p < P ? p : P - 1);
+    }
     // padding keys are masked to 0 arithmetically (no branch)
 #pragma unroll
     for (int p = 0; p < NP; ++p) {

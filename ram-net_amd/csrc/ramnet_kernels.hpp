@@ -17,6 +17,11 @@ struct AddrSource {
     float re_norm;  // top_k_re_norm exponent r in [0, 1]
     float sign;     // +1, or -1 when the weights are returned negated
     int k_off;      // first row of this address in the (B, H, k_total, T) outputs
+    // elements between batch rows, heads and tokens, and between the U * P
+    // consecutive logits of one address (a digit's P logits, then the next
+    // digit's). (B, H, U, P, T) in memory order: {H U P T, U P T, 1}, T.
+    int64_t stride[3];
+    int step;
 };
 
 // Per-event records consumed by the segment scan, laid out
@@ -83,7 +88,9 @@ struct AddrJob {
     int embed_num;           // CAPE applies to heads h < embed_num
     int encode_batch_idx;    // idx = (b*H + h)*A + a, else h*A + a
     int k_total;
-    const int32_t *position_ids;  // (B, T)
+    // position of token t of batch row b: position_ids[b * pos_stride[0] + t * pos_stride[1]]
+    const int32_t *position_ids;
+    int64_t pos_stride[2];
     int32_t *idx_out;             // (B, H, k_total, T)
     float *val_out;               // (B, H, k_total, T)
     // Record mode (both set): instead of idx/val, write scan records for
@@ -91,6 +98,7 @@ struct AddrJob {
     WriteRec *wrec;               // (B*H, Kw, T_pad)
     ReadRec *rrec;                // (B*H, Kr, T_pad)
     const void *gamma;            // (B, H, T) in dtype, for alpha
+    int64_t gamma_stride[3];      // elements between its batch rows, heads and tokens
     const uint8_t *mask;          // (B, T) or null
 };
 
@@ -133,6 +141,12 @@ struct SavedRows {
     MassAux aux;
 };
 
+// Offset of head bh's first token under strides {batch row, head, token}.
+__host__ __device__ inline int64_t row_offset(const int64_t *stride, int H, int bh) {
+    const int b = bh / H;
+    return b * stride[0] + (bh - b * H) * stride[1];
+}
+
 // Time-sequential gated sparse update + top-K read over a whole sequence.
 struct SegmentJob {
     const WriteRec *wrec;     // (B*H, Kw, T_pad) scan records
@@ -144,8 +158,8 @@ struct SegmentJob {
     float *slot_out;          // (B, H, A, C); may alias init_slot
     float *mass_out;          // (B, H, A); may alias init_mass
     void *y;                  // (B, H, T, C) in dtype
-    // (B, H, T, C) fp32 read sums carried from one slot range to the next
-    // when the scan is split into slot ranges: y itself for fp32 y, else a
+    // fp32 read sums carried from one slot range to the next when the scan
+    // is split into slot ranges, in y's layout: y itself for fp32 y, else a
     // workspace buffer (so y is rounded once, from the full sum)
     float *yacc;
     // (B*H, T_pad) per token: 1 if one of its write slots is a read slot of
@@ -154,7 +168,9 @@ struct SegmentJob {
     int *flags;
     SavedRows save;           // rows for the segment backward (save.w null: none)
     // elements between batch rows, heads and tokens of x and y (channels are
-    // adjacent): (B, H, T, C) in memory order unless the caller says otherwise
+    // adjacent): (B, H, T, C) in memory order unless the caller says
+    // otherwise. y's rows fill B * H * T * C elements in some order of b, h
+    // and t. Forward scans only; the backward takes contiguous tensors.
     int64_t x_stride[3], y_stride[3];
     int dtype;
     int B, H, T, A, C, Kw, Kr;

@@ -696,8 +696,10 @@ __device__ __forceinline__ void segment_scan_body(const SegmentJob &job, const S
             svo[p] = (((c >> lg) * Tp * sv.kp + p * EPP + ev) * sv.csw + (c & (sv.csw - 1))) * 4;
         sv_tok = sv.kp * sv.csw * 4;
     }
-    const Scalar *gx = static_cast<const Scalar *>(job.x) + static_cast<int64_t>(bh) * T * C;
-    Scalar *gy = static_cast<Scalar *>(job.y) + static_cast<int64_t>(bh) * T * C;
+    const int64_t xt = job.x_stride[2], yt = job.y_stride[2];  // elements between tokens
+    const Scalar *gx = static_cast<const Scalar *>(job.x) + row_offset(job.x_stride, job.H, bh);
+    const int64_t y_head = row_offset(job.y_stride, job.H, bh);
+    Scalar *gy = static_cast<Scalar *>(job.y) + y_head;
     // Items past the end are clamped to the last item, so the threads that
     // hold them load and store identical data (no branch).
     auto x_fetch = [&](int t0, Bits (&xb)[XI]) {
@@ -707,7 +709,7 @@ __device__ __forceinline__ void segment_scan_body(const SegmentJob &job, const S
             const int j = it / CS, c = it % CS;
             const int t = t0 + j < T ? t0 + j : T - 1;
             const int ch = c0 + c < C ? c0 + c : C - 1;
-            xb[k] = *reinterpret_cast<const Bits *>(gx + static_cast<int64_t>(t) * C + ch);
+            xb[k] = *reinterpret_cast<const Bits *>(gx + t * xt + ch);
         }
     };
     auto x_deposit = [&](int buf, const Bits (&xb)[XI]) {
@@ -765,7 +767,7 @@ __device__ __forceinline__ void segment_scan_body(const SegmentJob &job, const S
             const int j = it / CSW, c = wave * CSW + it % CSW;
             const int t = t0 + j < T ? t0 + j : T - 1;
             const int ch = c0 + c < C ? c0 + c : C - 1;
-            f.x[k] = *reinterpret_cast<const Bits *>(gx + static_cast<int64_t>(t) * C + ch);
+            f.x[k] = *reinterpret_cast<const Bits *>(gx + t * xt + ch);
         }
         // write event 0's record carries the token's overlap flag (a load
         // without a branch: a conditional one would be waited for at once)
@@ -989,12 +991,12 @@ __device__ __forceinline__ void segment_scan_body(const SegmentJob &job, const S
         for (int q = 0; q < NSL; ++q) {
             const int j = EPP <= CH ? q * EPP + ev : ev % CH;
             const int t = t0 + j;
-            Scalar *yp = gy + static_cast<int64_t>(t) * C + c0 + cl;
+            Scalar *yp = gy + t * yt + c0 + cl;
             if constexpr (RANGE) {
                 // slot ranges: the read sums of the ranges so far stay fp32
                 // in yacc; the last range adds its own and stores y
                 if (t < T) {
-                    float *ap = job.yacc + (static_cast<int64_t>(bh) * T + t) * C + c0 + cl;
+                    float *ap = job.yacc + y_head + t * yt + c0 + cl;
 #pragma unroll
                     for (int v = 0; v < VEC; ++v) {
                         if (FAST || c0 + cl + v < C) {

@@ -129,8 +129,9 @@ __global__ __launch_bounds__(kWave * NW) void segment_scan_pair_kernel(const Seg
     const GainRec *gp = job.gain + static_cast<int64_t>(bh) * EK * Tp;
     const WriteRec *gw = job.wrec + static_cast<int64_t>(bh) * job.Kw * Tp;
     const int *gf = job.flags + static_cast<int64_t>(bh) * Tp;
-    const Scalar *gx = static_cast<const Scalar *>(job.x) + static_cast<int64_t>(bh) * T * C;
-    Scalar *gy = static_cast<Scalar *>(job.y) + static_cast<int64_t>(bh) * T * C;
+    const int64_t xt = job.x_stride[2], yt = job.y_stride[2];  // elements between tokens
+    const Scalar *gx = static_cast<const Scalar *>(job.x) + row_offset(job.x_stride, job.H, bh);
+    Scalar *gy = static_cast<Scalar *>(job.y) + row_offset(job.y_stride, job.H, bh);
     // this wave's x stage: row (channel c of the wave, parity q) at (2 c + q) * XRB
     char *px = stage0 + wave * (CSW * 2 * XRB);
 
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(kWave * NW) void segment_scan_pair_kernel(const Seg
             const int j = it / CSW, c = wave * CSW + it % CSW;
             const int t = t0 + j < T ? t0 + j : T - 1;
             const int ch = c0 + c < C ? c0 + c : C - 1;
-            f.x[k] = *reinterpret_cast<const Bits *>(gx + static_cast<int64_t>(t) * C + ch);
+            f.x[k] = *reinterpret_cast<const Bits *>(gx + t * xt + ch);
         }
         // (loads without a branch: a conditional one would be waited for at once)
         const int tf = t0 + min(lane, CH - 1);
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(kWave * NW) void segment_scan_pair_kernel(const Seg
         // lane (tp, ev, cg) holds pair ev >> SH: token t0 + 2 (ev >> SH) + tp
         const int t = t0 + 2 * (ev >> SH) + tp;
         if ((ev & ((1 << SH) - 1)) == 0 && (!TAIL || t < T)) {
-            Scalar *yp = gy + static_cast<int64_t>(t) * C + c0 + cl;
+            Scalar *yp = gy + t * yt + c0 + cl;
             if constexpr (FAST) {
                 store_act_vec<Scalar, VEC>(yp, y);
             } else {

@@ -32,14 +32,18 @@ namespace {
 
 constexpr float kNegInf = -__builtin_huge_valf();
 
+__device__ __forceinline__ const int32_t *position_of(const AddrJob &job, int b, int t) {
+    return job.position_ids + b * job.pos_stride[0] + t * job.pos_stride[1];
+}
+
 // Whether token tl of batch row b is unmasked. Without a mask the load reads
-// a byte of this row's position ids instead (always in bounds) and is
+// a byte of this token's position instead (always in bounds) and is
 // ignored: a load that is always made needs no branch.
 __device__ __forceinline__ bool addr_unmasked(const AddrJob &job, int b, int tl) {
     const bool has = job.mask != nullptr;
-    const uint8_t *row = has ? job.mask + static_cast<int64_t>(b) * job.T
-                             : reinterpret_cast<const uint8_t *>(job.position_ids + static_cast<int64_t>(b) * job.T);
-    return !has | (row[tl] != 0);
+    const uint8_t *at = has ? job.mask + static_cast<int64_t>(b) * job.T + tl
+                            : reinterpret_cast<const uint8_t *>(position_of(job, b, tl));
+    return !has | (*at != 0);
 }
 
 // Record mode output of one address (source 0 = writes, 1 = reads). `get(k,
@@ -56,7 +60,10 @@ __device__ __forceinline__ void write_records(const AddrJob &job, int which, int
     // (conditions are bitwise: a short-circuit test of a lane value becomes
     // an exec-mask region, scalar instructions and a scheduling boundary)
     const bool live = (t < T) & addr_unmasked(job, b, tl) & !inactive;
-    const float g = which == 0 ? load_f32(static_cast<const Scalar *>(job.gamma) + bh * T + tl) : 0.f;
+    const float g = which == 0 ? load_f32(static_cast<const Scalar *>(job.gamma) + b * job.gamma_stride[0] +
+                                          (bh - static_cast<int64_t>(b) * job.H) * job.gamma_stride[1] +
+                                          tl * job.gamma_stride[2])
+                               : 0.f;
     // this lane's record of event 0; event k is k * Tp records further (a
     // uniform 32-bit step, not a 64-bit index product per event)
     WriteRec *wr0 = job.wrec + bh * K * Tp + t;
@@ -90,10 +97,17 @@ __device__ __forceinline__ void write_records(const AddrJob &job, int which, int
     }
 }
 
-// FAST: P == NP and the logits are read through a buffer resource with
-// 32-bit lane offsets (the host checks that every offset fits); otherwise
-// any P <= NP, through 64-bit pointers.
-template<typename Scalar, int NP, int KM, bool FAST>
+// How the lane kernel reads its logits. kLaneBuffer: (B, H, U, P, T) in
+// memory order and P == NP, through a buffer resource with 32-bit lane
+// offsets (the host checks that every offset fits). kLaneRow / kLaneRowPart:
+// each address's U * P logits adjacent and aligned, P == NP / P < NP, in
+// 16-byte loads. kLaneAny: any strides, P <= NP, through 64-bit pointers.
+// The search, not the loads, bounds all of them: B 8, H 16, T 4096, P 32,
+// top-K 8 in bf16 takes 81 us from (B, H, U, P, T) and 80 us from (B, T, H,
+// U, P) rows, where each lane's row is its own cache line; bringing two such
+// tensors into memory order first took 87 us each.
+enum : int { kLaneAny = 0, kLaneBuffer = 1, kLaneRow = 2, kLaneRowPart = 3 };
+template<typename Scalar, int NP, int KM, int LAY>
 // Occupancy: the per-lane search holds its digit in registers (about 210
 // VGPRs unconstrained, two waves per SIMD). Capping it at 168 (three waves)
 // hides more of the sort chains' latency at the cost of a few spills at
@@ -115,13 +129,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     const int64_t bh = gid / Tg;
     const int h = static_cast<int>(bh % H);
     const int b = static_cast<int>(bh / H);
-    const Scalar *base = static_cast<const Scalar *>(src.addr) + bh * static_cast<int64_t>(U * P) * T + tl;
+    const Scalar *base = static_cast<const Scalar *>(src.addr) + b * src.stride[0] + h * src.stride[1] +
+                         tl * src.stride[2];
 
     float mv[KM];  // sorted top-KM scores
     int mi[KM];    // their content indices
     uint32_t ok[KM];
     bool found;
-    if constexpr (FAST) {
+    if constexpr (LAY == kLaneRow || LAY == kLaneRowPart) {
+        constexpr bool full = LAY == kLaneRow;
+        const RowLogits<Scalar, NP, full> load{base, P};
+        found = lane_search<Scalar, NP, KM, full>(load, U, P, mv, mi, ok);
+    } else if constexpr (LAY == kLaneBuffer) {
         // resource based at the first active lane's logits: later lanes sit at
         // equal or higher addresses (same or later (b, h, t)), within
         // 2 * U * P * T elements of it
@@ -141,7 +160,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
             static_cast<int>(mine - first), T * static_cast<int>(sizeof(Scalar)), P};
         found = lane_search<Scalar, NP, KM, true>(load, U, P, mv, mi, ok);
     } else {
-        const GlobalLogits<Scalar> load{base, T, P};
+        const GlobalLogits<Scalar> load{base, src.step, P};
         found = lane_search<Scalar, NP, KM, false>(load, U, P, mv, mi, ok);
     }
     const bool inactive = !found;
@@ -159,7 +178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
             sum += __builtin_amdgcn_exp2f((mv[k] - mv[0]) * kLog2e);
     const bool norm = (src.re_norm != 0.f) & !inactive & (mv[0] > kNegInf);
     const float lse = norm ? mv[0] + log_sum(sum) : 0.f;
-    const int shift = h < job.embed_num ? pos_mod(job.position_ids[static_cast<int64_t>(b) * T + tl], A) : 0;
+    const int shift = h < job.embed_num ? pos_mod(*position_of(job, b, tl), A) : 0;
     if (rec_mode) {
         // Overlap flags of the write address, bit d - 1 for d = 1, 2, 3:
         // whether a written slot of this token is also written by token
@@ -236,7 +255,8 @@ __global__ __launch_bounds__(256) void topk_addr_bruteforce_kernel(const AddrJob
     const int64_t bh = gid / Tg;
     const int h = static_cast<int>(bh % H);
     const int b = static_cast<int>(bh / H);
-    const Scalar *base = static_cast<const Scalar *>(src.addr) + bh * static_cast<int64_t>(U * P) * T + tl;
+    const Scalar *base = static_cast<const Scalar *>(src.addr) + b * src.stride[0] + h * src.stride[1] +
+                         tl * src.stride[2];
 
     const int K = src.top_k;
     float *lg = smem;
@@ -251,15 +271,15 @@ __global__ __launch_bounds__(256) void topk_addr_bruteforce_kernel(const AddrJob
     __shared__ float s_lse;
     bool inactive;
     if constexpr (STAIR)
-        inactive = block_search_stair(base, static_cast<int64_t>(T), U, P, K, NPD, NA, lg, ex, di, sv, si, pv, pi, off,
+        inactive = block_search_stair(base, static_cast<int64_t>(src.step), U, P, K, NPD, NA, lg, ex, di, sv, si, pv, pi, off,
                                       &s_flag);
     else
-        inactive = block_search_exact(base, static_cast<int64_t>(T), U, P, A, NA, NPD, lg, ex, sv, si, &s_flag);
+        inactive = block_search_exact(base, static_cast<int64_t>(src.step), U, P, A, NA, NPD, lg, ex, sv, si, &s_flag);
     const int tid = threadIdx.x;
     if (tid == 0)
         s_lse = (src.re_norm != 0.f && !inactive) ? topk_lse_serial(sv, K) : 0.f;
     __syncthreads();
-    const int shift = h < job.embed_num ? pos_mod(job.position_ids[static_cast<int64_t>(b) * T + tl], A) : 0;
+    const int shift = h < job.embed_num ? pos_mod(*position_of(job, b, tl), A) : 0;
     if (rec_mode) {
         if (tid == 0)
             write_records<Scalar, 0>(job, blockIdx.y, bh, b, t, tl, inactive, [&](int k, int &c, float &v) {
@@ -301,17 +321,46 @@ int stair_buffer(int P, int K, int NPD) {
 
 namespace {
 
+// The lane kernel's read path. Rows need every address of every source on a
+// multiple of the piece it is read in, and a digit of whole pieces.
+template<typename T, int NP>
+int lane_layout(const AddrJob &job) {
+    constexpr int64_t ES = sizeof(T), piece = row_piece_bytes<T, NP>();
+    bool buffer = job.P == NP, rows = job.P * ES % piece == 0;
+    const int64_t up = static_cast<int64_t>(job.U) * job.P;
+    for (int s = 0; s < job.n_src; ++s) {
+        const AddrSource &a = job.src[s];
+        buffer = buffer && a.step == job.T && a.stride[2] == 1 && (job.H == 1 || a.stride[1] == up * job.T) &&
+                 (job.B == 1 || a.stride[0] == job.H * up * job.T);
+        rows = rows && a.step == 1 && reinterpret_cast<uintptr_t>(a.addr) % piece == 0;
+        const int n[3] = {job.B, job.H, job.T};
+        for (int d = 0; d < 3; ++d)
+            rows = rows && (n[d] == 1 || a.stride[d] * ES % piece == 0);
+    }
+    if (rows)
+        return job.P == NP ? kLaneRow : kLaneRowPart;
+    // a wave spans at most two (b, h) rows: lane offsets stay below
+    // 2 * U * P * T elements from the wave's first lane
+    return buffer && 2 * up * job.T * ES + 256 <= 0x7fffffff ? kLaneBuffer : kLaneAny;
+}
+
 template<typename T, int NP, int KM>
 hipError_t launch_lane(const AddrJob &job, hipStream_t stream) {
     const int64_t n = static_cast<int64_t>(job.B) * job.H * grid_t(job);
     const dim3 grid(static_cast<unsigned>((n + 255) / 256), job.n_src);
-    // a wave spans at most two (b, h) rows: lane offsets stay below
-    // 2 * U * P * T elements from the wave's first lane
-    const int64_t span = 2 * static_cast<int64_t>(job.U) * job.P * job.T * static_cast<int64_t>(sizeof(T)) + 256;
-    if (span <= 0x7fffffff && job.P == NP)
-        hipLaunchKernelGGL((topk_addr_lane_kernel<T, NP, KM, true>), grid, dim3(256), 0, stream, job);
-    else
-        hipLaunchKernelGGL((topk_addr_lane_kernel<T, NP, KM, false>), grid, dim3(256), 0, stream, job);
+    switch (lane_layout<T, NP>(job)) {
+        case kLaneBuffer:
+            hipLaunchKernelGGL((topk_addr_lane_kernel<T, NP, KM, kLaneBuffer>), grid, dim3(256), 0, stream, job);
+            break;
+        case kLaneRow:
+            hipLaunchKernelGGL((topk_addr_lane_kernel<T, NP, KM, kLaneRow>), grid, dim3(256), 0, stream, job);
+            break;
+        case kLaneRowPart:
+            hipLaunchKernelGGL((topk_addr_lane_kernel<T, NP, KM, kLaneRowPart>), grid, dim3(256), 0, stream, job);
+            break;
+        default:
+            hipLaunchKernelGGL((topk_addr_lane_kernel<T, NP, KM, kLaneAny>), grid, dim3(256), 0, stream, job);
+    }
     return hipGetLastError();
 }
 

@@ -31,6 +31,7 @@ _c_i64 = ctypes.c_int64
 _c_int = ctypes.c_int
 _c_float = ctypes.c_float
 _c_ptr = ctypes.c_void_p
+_c_i64s = ctypes.POINTER(_c_i64)
 
 # name -> argtypes, in header order
 SIGNATURES: dict[str, tuple[type, list]] = {
@@ -72,6 +73,13 @@ SIGNATURES: dict[str, tuple[type, list]] = {
         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_float, _c_float, _c_int,
         _c_float, _c_ptr]),
+    "ramnet_ram_attn_forward_strided": (_c_int, [
+        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_float, _c_float, _c_int,
+        _c_float, _c_i64s, _c_ptr, _c_i64, _c_ptr]),
+    "ramnet_topk_addr_forward_strided": (_c_int, [
+        _c_ptr, _c_ptr, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr,
+        _c_i64, _c_i64, _c_float, _c_float, _c_int, _c_i64s, _c_ptr, _c_ptr, _c_ptr]),
     "ramnet_topk_autoregressive_": (_c_int, [
         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_float, _c_float,
@@ -178,6 +186,11 @@ def segment_backward_saved_workspace_bytes(B: int, H: int, T: int, A: int, C: in
                                            r_top_k: int) -> int:
     """Device workspace (bytes) of the segment backward that takes saved rows."""
     return int(lib().ramnet_segment_backward_saved_workspace_bytes(B, H, T, A, C, w_top_k, r_top_k))
+
+
+def strides(*values: int) -> ctypes.Array:
+    """Host array of strides for the ``_strided`` entry points."""
+    return (_c_i64 * len(values))(*values)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

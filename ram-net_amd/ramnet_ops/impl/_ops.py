@@ -83,6 +83,46 @@ def _require_given(name: str, **tensors: Tensor) -> None:
 
 
 # --------------------------------------------------------------------------
+# layouts the kernels read where they are (the _strided entry points); any
+# other is copied into memory order first
+
+_REACH = 2 ** 31 - 1  # elements from a tensor's start that the kernels index
+
+
+def _reach(t: Tensor) -> int:
+    return sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+
+
+def _logits(t: Tensor) -> Tensor:
+    """Logits (B, H, U, P, T) whose U * P logits lie one fixed step apart."""
+    _, _, U, P, _ = t.shape
+    u, p = t.stride()[2:4]
+    if (U == 1 or u == P * p) and U * P * p < _REACH and _reach(t) < _REACH:
+        return t
+    return t.contiguous()
+
+
+def _rows(x: Tensor) -> Tensor:
+    """Values (B, H, T, C) with adjacent channels."""
+    return x if (x.shape[-1] == 1 or x.stride(-1) == 1) and _reach(x) < _REACH else x.contiguous()
+
+
+def _rows_like(x: Tensor) -> Tensor:
+    """An uninitialised y for values x: x's order of dimensions, channels adjacent."""
+    y = torch.empty_like(x)
+    return y if y.stride(-1) == 1 else x.new_empty(x.shape)
+
+
+def _position_words(t: Tensor) -> tuple[Tensor, tuple[int, int]]:
+    """Positions (B, T) and their strides in int32 words: an int64 position
+    is read through its low word, which is what a cast to int32 keeps."""
+    if t.dtype not in (torch.int32, torch.int64) or 2 * _reach(t) >= _REACH:
+        t = t.to(torch.int32).contiguous()
+    words = t.element_size() // 4
+    return t, (t.stride(0) * words, t.stride(1) * words)
+
+
+# --------------------------------------------------------------------------
 # address decoder
 
 @torch.library.custom_op(f"{_NS}::topk_addr_single_forward", mutates_args=(), device_types="cuda")
@@ -123,15 +163,16 @@ def topk_addr_forward(w_addr: Tensor, r_addr: Tensor, embed_num: int, A: int, po
     _check_shapes(op, r_addr=(r_addr, (B, H, U, P, T)), position_ids=(position_ids, (B, T)))
     if r_addr.dtype != w_addr.dtype:
         raise RuntimeError("topk_addr_forward: w_addr and r_addr must share shape and dtype")
-    w_addr, r_addr = w_addr.contiguous(), r_addr.contiguous()
-    pos = position_ids.to(device=w_addr.device, dtype=torch.int32).contiguous()
+    w_addr, r_addr = _logits(w_addr), _logits(r_addr)
+    pos, pos_s = _position_words(position_ids.to(device=w_addr.device))
     K = w_top_k + r_top_k
     idx = torch.empty((B, H, K, T), dtype=torch.int32, device=w_addr.device)
     val = torch.empty((B, H, K, T), dtype=torch.float32, device=w_addr.device)
     with torch.cuda.device(w_addr.device):
-        nat.call("ramnet_topk_addr_forward", w_addr.data_ptr(), r_addr.data_ptr(), _code(w_addr), B, H, U, P, T,
+        nat.call("ramnet_topk_addr_forward_strided", w_addr.data_ptr(), r_addr.data_ptr(), _code(w_addr), B, H, U, P, T,
                  embed_num, A, pos.data_ptr(), w_top_k, r_top_k, float(w_re_norm), float(r_re_norm),
-                 int(encode_batch_idx), idx.data_ptr(), val.data_ptr(), nat.stream_of(w_addr))
+                 int(encode_batch_idx), nat.strides(*w_addr.stride(), *r_addr.stride(), *pos_s), idx.data_ptr(),
+                 val.data_ptr(), nat.stream_of(w_addr))
     return idx, val
 
 
@@ -592,16 +633,20 @@ def _ram_attn_call(w_addr, r_addr, x, gamma, mask, embed_num, position_ids, init
     A = P ** U
     if r_addr.dtype != w_addr.dtype or x.dtype != w_addr.dtype:
         raise RuntimeError("ram_attn_forward: w_addr, r_addr and x must share dtype and address shape")
-    w_addr, r_addr = w_addr.contiguous(), r_addr.contiguous()
-    x, gamma, mask = _segment_args(x, gamma, mask)
-    pos = position_ids.to(device=x.device, dtype=torch.int32).contiguous()
-    y = torch.empty_like(x)
+    y = _rows_like(x)
+    w_addr, r_addr, x, gamma = _logits(w_addr), _logits(r_addr), _rows(x), gamma.to(dtype=x.dtype)
+    if _reach(gamma) >= _REACH:
+        gamma = gamma.contiguous()
+    if mask is not None:
+        mask = mask.to(device=x.device, dtype=torch.bool).contiguous()
+    pos, pos_s = _position_words(position_ids.to(device=x.device))
     ws = _workspace(x, B, H, T, A, C, w_top_k, r_top_k)
+    at = nat.strides(*w_addr.stride(), *r_addr.stride(), *x.stride()[:3], *y.stride()[:3], *gamma.stride(), *pos_s)
     with torch.cuda.device(x.device):
-        nat.call("ramnet_ram_attn_forward", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(), gamma.data_ptr(),
+        nat.call("ramnet_ram_attn_forward_strided", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(), gamma.data_ptr(),
                  _code(x), nat.ptr(mask), embed_num, pos.data_ptr(), init_slot.data_ptr(), init_mass.data_ptr(),
                  slot.data_ptr(), mass.data_ptr(), y.data_ptr(), B, H, U, P, T, A, C, w_top_k, r_top_k,
-                 float(w_re_norm), float(r_re_norm), int(mass_aware), float(eps), ws.data_ptr(), ws.numel(),
+                 float(w_re_norm), float(r_re_norm), int(mass_aware), float(eps), at, ws.data_ptr(), ws.numel(),
                  nat.stream_of(x))
     return y
 
@@ -626,7 +671,7 @@ def ram_attn_forward(w_addr: Tensor, r_addr: Tensor, x: Tensor, gamma: Tensor, i
 @ram_attn_forward.register_fake
 def _(w_addr, r_addr, x, gamma, init_slot, init_mass, mask, embed_num, position_ids, w_top_k, r_top_k, w_re_norm,
       r_re_norm, mass_aware, eps):
-    return (x.new_empty(x.shape), init_slot.new_empty(init_slot.shape, dtype=torch.float32),
+    return (_rows_like(x), init_slot.new_empty(init_slot.shape, dtype=torch.float32),
             init_mass.new_empty(init_mass.shape, dtype=torch.float32))
 
 
@@ -646,7 +691,7 @@ def ram_attn_forward_(w_addr: Tensor, r_addr: Tensor, x: Tensor, gamma: Tensor, 
 @ram_attn_forward_.register_fake
 def _(w_addr, r_addr, x, gamma, slot, mass, mask, embed_num, position_ids, w_top_k, r_top_k, w_re_norm, r_re_norm,
       mass_aware, eps):
-    return x.new_empty(x.shape)
+    return _rows_like(x)
 
 
 # --------------------------------------------------------------------------

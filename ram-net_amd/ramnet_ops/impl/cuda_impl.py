@@ -93,7 +93,9 @@ def _cuda_ram_attn(
 
     requires_grad = torch.is_grad_enabled() and any(
         t.requires_grad for t in (w_addr, r_addr, xs, gamma, init_slot, init_mass))
-    position_ids = position_ids.to(device=xs.device, dtype=torch.int32)
+    # the decoders read int64 positions where they are
+    position_ids = position_ids.to(device=xs.device,
+                                   dtype=None if position_ids.dtype in (torch.int32, torch.int64) else torch.int32)
     if mask is not None:
         mask = mask.to(device=xs.device, dtype=torch.bool)
 
