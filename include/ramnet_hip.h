@@ -281,15 +281,20 @@ int ramnet_ram_attn_forward(const void *w_addr, const void *r_addr, const void *
                             float eps, void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
- * ramnet_ram_attn_forward and ramnet_topk_addr_forward on tensors that need
- * not be in memory order, so that activations laid out (B, T, H, ...) are
- * taken where they are. `strides` (host memory, elements, >= 0; every tensor
+ * The same calls on tensors that need not be in memory order, so that
+ * activations laid out (B, T, H, ...) are taken where they are; int64
+ * positions are given as int32 words (their low words are read) with
+ * doubled strides. `strides` (host memory, elements, >= 0; every tensor
  * within int32 elements of its start):
  *   ram_attn_forward   w_addr [b, h, u, p, t], r_addr [b, h, u, p, t],
  *                      x [b, h, t], y [b, h, t], gamma [b, h, t],
  *                      position_ids [b, t]   (21 values)
  *   topk_addr_forward  w_addr [b, h, u, p, t], r_addr [b, h, u, p, t],
  *                      position_ids [b, t]   (12 values)
+ *   topk_addr_single_forward  addr [b, h, u, p, t], position_ids [b, t]
+ *                      (7 values)
+ *   topk_autoregressive_ (below)        position_ids [b]     (1 value)
+ *   topk_autoregressive_steps_ (below)  position_ids [s, b]  (2 values)
  * Digits follow each other at P times the logits' stride; channels of x and
  * y are adjacent; y's rows fill B * H * T * C elements (they may be in any
  * order of b, h and t). Outputs other than y, the state and the mask are in
@@ -307,6 +312,23 @@ int ramnet_topk_addr_forward_strided(const void *w_addr, const void *r_addr, int
                                      const int32_t *position_ids, int64_t w_top_k, int64_t r_top_k, float w_re_norm,
                                      float r_re_norm, int encode_batch_idx, const int64_t *strides, int32_t *idx_out,
                                      float *val_out, void *stream);
+int ramnet_topk_addr_single_forward_strided(const void *addr, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
+                                            int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
+                                            int64_t top_k, float top_k_re_norm, int addr_val_neg,
+                                            int encode_batch_idx, const int64_t *strides, int32_t *idx_out,
+                                            float *val_out, void *stream);
+int ramnet_topk_autoregressive_strided_(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
+                                        int dtype, float *slot, float *mass, const uint8_t *mask, int64_t embed_num,
+                                        const int32_t *position_ids, int64_t B, int64_t H, int64_t U, int64_t P,
+                                        int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k, float w_re_norm,
+                                        float r_re_norm, int mass_aware, float eps, const int64_t *strides, void *y,
+                                        void *stream);
+int ramnet_topk_autoregressive_steps_strided_(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
+                                              int dtype, float *slot, float *mass, const uint8_t *mask,
+                                              int64_t embed_num, const int32_t *position_ids, int64_t S, int64_t B,
+                                              int64_t H, int64_t U, int64_t P, int64_t A, int64_t C, int64_t w_top_k,
+                                              int64_t r_top_k, float w_re_norm, float r_re_norm, int mass_aware,
+                                              float eps, const int64_t *strides, void *y, void *stream);
 
 /*
  * One fused decode step on a persistent state, updated in place.

@@ -471,7 +471,7 @@ __global__ __launch_bounds__(64) void autoregressive_fast_kernel(const DecodeJob
     XRaw<T, kCpl, FULLC> xr;
     xr.load(static_cast<const T *>(job.x) + static_cast<int64_t>(bh) * C, coff, lane);
     const float gamma = load_f32(static_cast<const T *>(job.gamma) + bh);
-    const int pos = job.position_ids[b];
+    const int pos = job.position_ids[b * job.pos_stride[1]];
     const uint8_t valid = job.mask ? job.mask[b] : 1;
     if (!valid) {
         for (int c = lane; c < C; c += kWave)
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(2 * kWave) void autoregressive_steps_kernel(const D
     // see is uniform), so it stays a vector value: a scalar load would share
     // its completion counter with the LDS accesses, and a uniform vector load
     // would be moved to a scalar register right after it issues.
-    const int32_t *pp = job.position_ids + b + static_cast<int>(opaque(0u));
+    const int32_t *pp = job.position_ids + b * job.pos_stride[1] + static_cast<int>(opaque(0u));
     const bool cape = h < job.embed_num;
     GroupLogits<T> lg;
     int pos = 0;
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(2 * kWave) void autoregressive_steps_kernel(const D
         decode_events<T, GW, KE, kCpl>(job, lg, lg, cape ? pos_mod(pos, A) : 0, lane, s_ws, s_rs, s_wv, ev);
         const int64_t n = next < last ? next : last;
         lg.load(ap + n * step_addr, U, P, lane & 31);
-        pos = pp[n * B];
+        pos = pp[n * job.pos_stride[0]];
         forward_map<KE, kCpl>(job, lane, s_ws, s_rs, s_wv, ev);
         ring.ev[slot][lane] = make_int2(ev.ow, __float_as_int(ev.vw));
         if (lane == 0) {
@@ -670,7 +670,7 @@ __global__ __launch_bounds__(64) void autoregressive_general_kernel(const Decode
     int *off = pi + (STAIR ? KM : 0);
     int *ev_slot = off + (STAIR ? KM + 1 : 0);  // Kw + Kr
     float *ev_val = reinterpret_cast<float *>(ev_slot + Kw + Kr);  // Kw + Kr
-    const int shift = h < job.embed_num ? pos_mod(job.position_ids[b], A) : 0;
+    const int shift = h < job.embed_num ? pos_mod(job.position_ids[b * job.pos_stride[1]], A) : 0;
 
     for (int which = 0; which < 2; ++which) {
         const T *ptr = static_cast<const T *>(which ? job.r_addr : job.w_addr) + static_cast<int64_t>(bh) * U * P;
@@ -862,7 +862,7 @@ hipError_t launch_typed_steps(const DecodeJob &job, int S, hipStream_t stream, c
         one.x = static_cast<const T *>(job.x) + s * BH * job.C;
         one.gamma = static_cast<const T *>(job.gamma) + s * BH;
         one.y = static_cast<T *>(job.y) + s * BH * job.C;
-        one.position_ids = job.position_ids + static_cast<int64_t>(s) * job.B;
+        one.position_ids = job.position_ids + s * job.pos_stride[0];
         one.mask = job.mask ? job.mask + static_cast<int64_t>(s) * job.B : nullptr;
         const hipError_t err = launch_typed<T>(one, stream, why);
         if (err != hipSuccess)

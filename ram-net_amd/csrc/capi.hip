@@ -171,10 +171,10 @@ int ramnet_int_bits(void) { return 32; }
 
 const char *ramnet_last_error(void) { return g_last_error.c_str(); }
 
-int ramnet_topk_addr_single_forward(const void *addr, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
+static int topk_addr_single_forward(const void *addr, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
                                     int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
                                     int64_t top_k, float top_k_re_norm, int addr_val_neg, int encode_batch_idx,
-                                    int32_t *idx_out, float *val_out, void *stream) {
+                                    const Layout &lay, int32_t *idx_out, float *val_out, void *stream) {
     if (int rc = check_addr_shape(B, H, U, P, T, embed_num, A))
         return rc;
     RAMNET_REQUIRE(valid_dtype(dtype), "addr dtype must be float32, float16 or bfloat16");
@@ -184,10 +184,12 @@ int ramnet_topk_addr_single_forward(const void *addr, int dtype, int64_t B, int6
     if (B * T == 0)
         return RAMNET_OK;
     RAMNET_REQUIRE(addr && position_ids && idx_out && val_out, "null tensor pointer");
+    if (int rc = check_logits(lay.w, B, H, U, P, T))
+        return rc;
+    RAMNET_REQUIRE(stride_ok(lay.pos, {B, T}), "position strides must be >= 0 and within int32");
     ramnet::AddrJob job{};
     job.src[0] = {addr, static_cast<int>(top_k), top_k_re_norm, addr_val_neg ? -1.f : 1.f, 0};
     job.n_src = 1;
-    const Layout lay = memory_order(B, H, U, P, T, 1);
     set_source(job.src[0], lay.w);
     job.pos_stride[0] = lay.pos[0];
     job.pos_stride[1] = lay.pos[1];
@@ -207,6 +209,28 @@ int ramnet_topk_addr_single_forward(const void *addr, int dtype, int64_t B, int6
     const char *why = nullptr;
     const hipError_t err = ramnet::launch_topk_addr(job, static_cast<hipStream_t>(stream), &why);
     return finish(err, why, "topk_addr_single_forward launch");
+}
+
+int ramnet_topk_addr_single_forward(const void *addr, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
+                                    int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
+                                    int64_t top_k, float top_k_re_norm, int addr_val_neg, int encode_batch_idx,
+                                    int32_t *idx_out, float *val_out, void *stream) {
+    return topk_addr_single_forward(addr, dtype, B, H, U, P, T, embed_num, A, position_ids, top_k, top_k_re_norm,
+                                    addr_val_neg, encode_batch_idx, memory_order(B, H, U, P, T, 1), idx_out, val_out,
+                                    stream);
+}
+
+int ramnet_topk_addr_single_forward_strided(const void *addr, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
+                                            int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
+                                            int64_t top_k, float top_k_re_norm, int addr_val_neg,
+                                            int encode_batch_idx, const int64_t *strides, int32_t *idx_out,
+                                            float *val_out, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    Layout lay{};
+    std::copy_n(strides, 5, lay.w);
+    std::copy_n(strides + 5, 2, lay.pos);
+    return topk_addr_single_forward(addr, dtype, B, H, U, P, T, embed_num, A, position_ids, top_k, top_k_re_norm,
+                                    addr_val_neg, encode_batch_idx, lay, idx_out, val_out, stream);
 }
 
 int ramnet_topk_addr_single_backward(const int32_t *idx, const float *val, const void *addr, const float *grad_val,
@@ -897,21 +921,47 @@ static int decode_job(const void *w_addr, const void *r_addr, const void *x, con
     return RAMNET_OK;
 }
 
+static int autoregressive(const void *w_addr, const void *r_addr, const void *x, const void *gamma, int dtype,
+                          float *slot, float *mass, const uint8_t *mask, int64_t embed_num,
+                          const int32_t *position_ids, int64_t S, int64_t B, int64_t H, int64_t U, int64_t P,
+                          int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
+                          int mass_aware, float eps, const int64_t (&pos)[2], bool steps, void *y, void *stream) {
+    ramnet::DecodeJob job;
+    if (int rc = decode_job(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, S, B, H, U, P,
+                            A, C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, y, job))
+        return rc;
+    if (B == 0 || S == 0)
+        return RAMNET_OK;
+    RAMNET_REQUIRE(w_addr && r_addr && x && gamma && slot && mass && position_ids && y, "null tensor pointer");
+    RAMNET_REQUIRE(stride_ok(pos, {S, B}), "position strides must be >= 0 and within int32");
+    std::copy_n(pos, 2, job.pos_stride);
+    const char *why = nullptr;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    const hipError_t err = steps ? ramnet::launch_autoregressive_steps(job, static_cast<int>(S), st, &why)
+                                 : ramnet::launch_autoregressive(job, st, &why);
+    return finish(err, why, steps ? "topk_autoregressive_steps_ launch" : "topk_autoregressive_ launch");
+}
+
 int ramnet_topk_autoregressive_(const void *w_addr, const void *r_addr, const void *x, const void *gamma, int dtype,
                                 float *slot, float *mass, const uint8_t *mask, int64_t embed_num,
                                 const int32_t *position_ids, int64_t B, int64_t H, int64_t U, int64_t P, int64_t A,
                                 int64_t C, int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
                                 int mass_aware, float eps, void *y, void *stream) {
-    ramnet::DecodeJob job;
-    if (int rc = decode_job(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, 1, B, H, U, P,
-                            A, C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, y, job))
-        return rc;
-    if (B == 0)
-        return RAMNET_OK;
-    RAMNET_REQUIRE(w_addr && r_addr && x && gamma && slot && mass && position_ids && y, "null tensor pointer");
-    const char *why = nullptr;
-    const hipError_t err = ramnet::launch_autoregressive(job, static_cast<hipStream_t>(stream), &why);
-    return finish(err, why, "topk_autoregressive_ launch");
+    const int64_t pos[2] = {B, 1};
+    return autoregressive(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, 1, B, H, U, P, A,
+                          C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, pos, false, y, stream);
+}
+
+int ramnet_topk_autoregressive_strided_(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
+                                        int dtype, float *slot, float *mass, const uint8_t *mask, int64_t embed_num,
+                                        const int32_t *position_ids, int64_t B, int64_t H, int64_t U, int64_t P,
+                                        int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k, float w_re_norm,
+                                        float r_re_norm, int mass_aware, float eps, const int64_t *strides, void *y,
+                                        void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    const int64_t pos[2] = {0, strides[0]};
+    return autoregressive(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, 1, B, H, U, P, A,
+                          C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, pos, false, y, stream);
 }
 
 int ramnet_topk_autoregressive_steps_(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
@@ -920,17 +970,21 @@ int ramnet_topk_autoregressive_steps_(const void *w_addr, const void *r_addr, co
                                       int64_t P, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
                                       float w_re_norm, float r_re_norm, int mass_aware, float eps, void *y,
                                       void *stream) {
-    ramnet::DecodeJob job;
-    if (int rc = decode_job(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, S, B, H, U, P,
-                            A, C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, y, job))
-        return rc;
-    if (B == 0 || S == 0)
-        return RAMNET_OK;
-    RAMNET_REQUIRE(w_addr && r_addr && x && gamma && slot && mass && position_ids && y, "null tensor pointer");
-    const char *why = nullptr;
-    const hipError_t err =
-        ramnet::launch_autoregressive_steps(job, static_cast<int>(S), static_cast<hipStream_t>(stream), &why);
-    return finish(err, why, "topk_autoregressive_steps_ launch");
+    const int64_t pos[2] = {B, 1};
+    return autoregressive(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, S, B, H, U, P, A,
+                          C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, pos, true, y, stream);
+}
+
+int ramnet_topk_autoregressive_steps_strided_(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
+                                              int dtype, float *slot, float *mass, const uint8_t *mask,
+                                              int64_t embed_num, const int32_t *position_ids, int64_t S, int64_t B,
+                                              int64_t H, int64_t U, int64_t P, int64_t A, int64_t C, int64_t w_top_k,
+                                              int64_t r_top_k, float w_re_norm, float r_re_norm, int mass_aware,
+                                              float eps, const int64_t *strides, void *y, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    const int64_t pos[2] = {strides[0], strides[1]};
+    return autoregressive(w_addr, r_addr, x, gamma, dtype, slot, mass, mask, embed_num, position_ids, S, B, H, U, P, A,
+                          C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, pos, true, y, stream);
 }
 
 // The query has no token count: it answers for a call of kPlanQueryTokens

@@ -212,7 +212,9 @@ struct DecodeJob {
     const void *x;            // (B, H, C)
     const void *gamma;        // (B, H)
     const uint8_t *mask;      // (B) or null
-    const int32_t *position_ids;  // (B)
+    // position of row b at step s: position_ids[s * pos_stride[0] + b * pos_stride[1]]
+    const int32_t *position_ids;
+    int64_t pos_stride[2];
     float *slot;              // (B, H, A, C), updated in place
     float *mass;              // (B, H, A), updated in place
     void *y;                  // (B, H, C)

@@ -113,13 +113,13 @@ def _rows_like(x: Tensor) -> Tensor:
     return y if y.stride(-1) == 1 else x.new_empty(x.shape)
 
 
-def _position_words(t: Tensor) -> tuple[Tensor, tuple[int, int]]:
-    """Positions (B, T) and their strides in int32 words: an int64 position
-    is read through its low word, which is what a cast to int32 keeps."""
+def _position_words(t: Tensor) -> tuple[Tensor, tuple[int, ...]]:
+    """Positions and their strides in int32 words: an int64 position is read
+    through its low word, which is what a cast to int32 keeps."""
     if t.dtype not in (torch.int32, torch.int64) or 2 * _reach(t) >= _REACH:
         t = t.to(torch.int32).contiguous()
     words = t.element_size() // 4
-    return t, (t.stride(0) * words, t.stride(1) * words)
+    return t, tuple(s * words for s in t.stride())
 
 
 # --------------------------------------------------------------------------
@@ -134,14 +134,14 @@ def topk_addr_single_forward(addr: Tensor, embed_num: int, A: int, position_ids:
     B, H, U, P, T = _dims(op, "addr", addr, 5)
     _check_slots(op, U, P, A)
     _check_shapes(op, position_ids=(position_ids, (B, T)))
-    addr = addr.contiguous()
-    pos = position_ids.to(device=addr.device, dtype=torch.int32).contiguous()
+    addr = _logits(addr)
+    pos, pos_s = _position_words(position_ids.to(device=addr.device))
     idx = torch.empty((B, H, top_k, T), dtype=torch.int32, device=addr.device)
     val = torch.empty((B, H, top_k, T), dtype=torch.float32, device=addr.device)
     with torch.cuda.device(addr.device):
-        nat.call("ramnet_topk_addr_single_forward", addr.data_ptr(), _code(addr), B, H, U, P, T, embed_num, A,
+        nat.call("ramnet_topk_addr_single_forward_strided", addr.data_ptr(), _code(addr), B, H, U, P, T, embed_num, A,
                  pos.data_ptr(), top_k, float(top_k_re_norm), int(addr_val_neg), int(encode_batch_idx),
-                 idx.data_ptr(), val.data_ptr(), nat.stream_of(addr))
+                 nat.strides(*addr.stride(), *pos_s), idx.data_ptr(), val.data_ptr(), nat.stream_of(addr))
     return idx, val
 
 
@@ -714,14 +714,14 @@ def topk_autoregressive_(w_addr: Tensor, r_addr: Tensor, x: Tensor, gamma: Tenso
     _check_decode_dtypes(op, w_addr, r_addr, x)
     w_addr, r_addr, x = w_addr.contiguous(), r_addr.contiguous(), x.contiguous()
     gamma = gamma.to(dtype=x.dtype).contiguous()
-    pos = position_ids.to(device=x.device, dtype=torch.int32).contiguous()
+    pos, pos_s = _position_words(position_ids.to(device=x.device))
     m = None if mask is None or mask.numel() == 0 else mask.to(device=x.device, dtype=torch.bool).contiguous()
     y = torch.empty_like(x)
     with torch.cuda.device(x.device):
-        nat.call("ramnet_topk_autoregressive_", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(), gamma.data_ptr(),
+        nat.call("ramnet_topk_autoregressive_strided_", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(), gamma.data_ptr(),
                  _code(x), slot.data_ptr(), mass.data_ptr(), nat.ptr(m), embed_num, pos.data_ptr(), B, H, U, P, A, C,
-                 w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), int(mass_aware), float(eps), y.data_ptr(),
-                 nat.stream_of(x))
+                 w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), int(mass_aware), float(eps),
+                 nat.strides(*pos_s), y.data_ptr(), nat.stream_of(x))
     return y
 
 
@@ -754,14 +754,14 @@ def topk_autoregressive_steps_(w_addr: Tensor, r_addr: Tensor, x: Tensor, gamma:
     _check_decode_dtypes(op, w_addr, r_addr, x)
     w_addr, r_addr, x = w_addr.contiguous(), r_addr.contiguous(), x.contiguous()
     gamma = gamma.to(dtype=x.dtype).contiguous()
-    pos = position_ids.to(device=x.device, dtype=torch.int32).contiguous()
+    pos, pos_s = _position_words(position_ids.to(device=x.device))
     m = None if mask is None or mask.numel() == 0 else mask.to(device=x.device, dtype=torch.bool).contiguous()
     y = torch.empty_like(x)
     with torch.cuda.device(x.device):
-        nat.call("ramnet_topk_autoregressive_steps_", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(),
+        nat.call("ramnet_topk_autoregressive_steps_strided_", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), slot.data_ptr(), mass.data_ptr(), nat.ptr(m), embed_num, pos.data_ptr(),
                  S, B, H, U, P, A, C, w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), int(mass_aware),
-                 float(eps), y.data_ptr(), nat.stream_of(x))
+                 float(eps), nat.strides(*pos_s), y.data_ptr(), nat.stream_of(x))
     return y
 
 

@@ -50,7 +50,7 @@ def _cuda_topk_autoregressive_(
     mask = empty if mask is None else mask.to(device=x.device, dtype=torch.bool).contiguous()
     return torch.ops.ramnet_ops.topk_autoregressive_(
         w_addr.contiguous(), r_addr.contiguous(), x.contiguous(), gamma.contiguous(), slot_, mass_,
-        mask, embed_num, position_ids.contiguous(), w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps)
+        mask, embed_num, position_ids, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps)
 
 
 def _cuda_ram_attn(
@@ -192,6 +192,6 @@ def _cuda_topk_addr(
     assert isinstance(encode_batch_idx, bool), f"Expected boolean encode_batch_idx, got {encode_batch_idx!r}."
     assert tuple(position_ids.shape) == (B, T), f"Expected position_ids.shape={(B, T)}, got {tuple(position_ids.shape)}."
     check_int_capacity(B, H, U, P, A, T, embed_num, top_k, B * H * U * P * T, B * H * A, B * H * top_k * T)
-    position_ids = position_ids.to(device=addr.device, dtype=torch.int32)
+    position_ids = position_ids.to(device=addr.device)
     return torch.ops.ramnet_ops.topk_addr_single_forward(
         addr, embed_num, A, position_ids, top_k, float(top_k_re_norm), addr_val_neg, encode_batch_idx)

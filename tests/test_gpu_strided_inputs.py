@@ -114,6 +114,34 @@ def test_strided_scan_layouts(monkeypatch, layout):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("P,Kw", [(16, 4), (48, 12), (5, 20)], ids=["half", "wave", "general"])
+def test_decode_positions(P, Kw):
+    """int64 and strided positions in the decode step, the multi-step call
+    (one launch, or one a step) and the single decoder."""
+    B, H, U, C, S = 3, 2, 2, 16, 3
+    d = _inputs(B, H, U, P, S, C, torch.bfloat16)
+    w, r = (d[n].permute(2, 0, 1, 3, 4).contiguous() for n in ("w", "r"))
+    x, gamma = d["x"].permute(2, 0, 1, 3).contiguous(), d["gamma"].permute(2, 0, 1).contiguous()
+    pos = torch.arange(S, device=DEV).view(S, 1) * 5 + torch.arange(B, device=DEV).view(1, B) * 11 - 7
+    none = torch.empty(0, dtype=torch.bool, device=DEV)
+    ops = torch.ops.ramnet_ops
+    outs = []
+    # the positions as int32, as int64, as a column-major view and every other word of a wider row
+    wide = torch.zeros(S, 2 * B, dtype=torch.int64, device=DEV)
+    wide[:, ::2] = pos
+    for p in (pos.to(torch.int32), pos, pos.t().contiguous().t(), wide[:, ::2]):
+        slot, mass = d["slot"].clone(), d["mass"].clone()
+        y = ops.topk_autoregressive_steps_(w, r, x, gamma, slot, mass, none, 1, p, Kw, 3, 0.0, 0.0, True, 1e-6)
+        slot1, mass1 = d["slot"].clone(), d["mass"].clone()
+        y1 = torch.stack([ops.topk_autoregressive_(w[s], r[s], x[s], gamma[s], slot1, mass1, none, 1, p[s], Kw, 3,
+                                                   0.0, 0.0, True, 1e-6) for s in range(S)])
+        idx, val = ops.topk_addr_single_forward(w.permute(1, 2, 3, 4, 0), 1, P ** U, p.t(), Kw, 0.5)
+        outs.append((y, slot, mass, y1, slot1, mass1, idx, val))
+    for other in outs[1:]:
+        for a, b in zip(other, outs[0]):
+            assert torch.equal(a, b)
+
+
 def test_refused_strides():
     """Steps the kernels cannot follow are refused by the native entry."""
     z = torch.zeros(64, device=DEV)
