@@ -138,7 +138,7 @@ def topk_addr_single_forward(addr: Tensor, embed_num: int, A: int, position_ids:
     pos, pos_s = _position_words(position_ids.to(device=addr.device))
     idx = torch.empty((B, H, top_k, T), dtype=torch.int32, device=addr.device)
     val = torch.empty((B, H, top_k, T), dtype=torch.float32, device=addr.device)
-    with torch.cuda.device(addr.device):
+    with nat.on_device(addr):
         nat.call("ramnet_topk_addr_single_forward_strided", addr.data_ptr(), _code(addr), B, H, U, P, T, embed_num, A,
                  pos.data_ptr(), top_k, float(top_k_re_norm), int(addr_val_neg), int(encode_batch_idx),
                  nat.strides(*addr.stride(), *pos_s), idx.data_ptr(), val.data_ptr(), nat.stream_of(addr))
@@ -168,7 +168,7 @@ def topk_addr_forward(w_addr: Tensor, r_addr: Tensor, embed_num: int, A: int, po
     K = w_top_k + r_top_k
     idx = torch.empty((B, H, K, T), dtype=torch.int32, device=w_addr.device)
     val = torch.empty((B, H, K, T), dtype=torch.float32, device=w_addr.device)
-    with torch.cuda.device(w_addr.device):
+    with nat.on_device(w_addr):
         nat.call("ramnet_topk_addr_forward_strided", w_addr.data_ptr(), r_addr.data_ptr(), _code(w_addr), B, H, U, P, T,
                  embed_num, A, pos.data_ptr(), w_top_k, r_top_k, float(w_re_norm), float(r_re_norm),
                  int(encode_batch_idx), nat.strides(*w_addr.stride(), *r_addr.stride(), *pos_s), idx.data_ptr(),
@@ -202,7 +202,7 @@ def topk_addr_single_backward(idx: Tensor, val: Tensor, addr: Tensor, D_val: Ten
     addr = addr.to(dtype).contiguous()
     pos = position_ids.to(device=addr.device, dtype=torch.int32).contiguous()
     grad = torch.empty((B, H, U, P, T), dtype=dtype, device=addr.device)
-    with torch.cuda.device(addr.device):
+    with nat.on_device(addr):
         nat.call("ramnet_topk_addr_single_backward", idx.to(torch.int32).contiguous().data_ptr(),
                  val.to(torch.float32).contiguous().data_ptr(), addr.data_ptr(),
                  D_val.to(torch.float32).contiguous().data_ptr(), _code(addr), B, H, U, P, T, embed_num, A,
@@ -234,7 +234,7 @@ def topk_addr_backward(idx: Tensor, val: Tensor, w_addr: Tensor, r_addr: Tensor,
     pos = position_ids.to(device=w_addr.device, dtype=torch.int32).contiguous()
     gw = torch.empty((B, H, U, P, T), dtype=dtype, device=w_addr.device)
     gr = torch.empty_like(gw)
-    with torch.cuda.device(w_addr.device):
+    with nat.on_device(w_addr):
         nat.call("ramnet_topk_addr_backward", idx.to(torch.int32).contiguous().data_ptr(),
                  val.to(torch.float32).contiguous().data_ptr(), w_addr.data_ptr(), r_addr.data_ptr(),
                  D_val.to(torch.float32).contiguous().data_ptr(), _code(w_addr), B, H, U, P, T, embed_num, A,
@@ -342,7 +342,7 @@ def topk_segment_forward(addr_idx: Tensor, addr_val: Tensor, x: Tensor, gamma: T
     mass = torch.empty_like(init_mass)
     y = torch.empty_like(x)
     ws = _workspace(x, B, H, T, A, C, w_top_k, r_top_k)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_segment_forward", addr_idx.data_ptr(), addr_val.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), nat.ptr(mask), init_slot.data_ptr(), init_mass.data_ptr(),
                  slot.data_ptr(), mass.data_ptr(), y.data_ptr(), B, H, T, A, C, w_top_k, r_top_k, int(mass_aware),
@@ -395,7 +395,7 @@ def topk_segment_backward(addr_idx: Tensor, addr_val: Tensor, x: Tensor, gamma: 
     if nbytes < 0:
         raise RuntimeError(f"topk_segment_backward: shape not supported (A={A}, C={C}, top_k=({w_top_k}, {r_top_k}))")
     ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_segment_backward", addr_idx.data_ptr(), addr_val.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), nat.ptr(mask), init_slot.data_ptr(), init_mass.data_ptr(),
                  D_y.data_ptr(), nat.ptr(D_post_slot), nat.ptr(D_post_mass), D_addr.data_ptr(), D_x.data_ptr(),
@@ -481,7 +481,7 @@ def topk_segment_forward_saved(addr_idx: Tensor, addr_val: Tensor, x: Tensor, ga
     y = torch.empty_like(x)
     ws = _workspace(x, B, H, T, A, C, w_top_k, r_top_k)
     saved = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_segment_forward_save", addr_idx.data_ptr(), addr_val.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), nat.ptr(mask), init_slot.data_ptr(), init_mass.data_ptr(),
                  slot.data_ptr(), mass.data_ptr(), y.data_ptr(), B, H, T, A, C, w_top_k, r_top_k, int(mass_aware),
@@ -535,7 +535,7 @@ def topk_segment_backward_saved(addr_val: Tensor, x: Tensor, gamma: Tensor, init
     D_mass = torch.empty_like(init_mass)
     ws = torch.empty(max(1, nat.segment_backward_saved_workspace_bytes(B, H, T, A, C, w_top_k, r_top_k)),
                      dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_segment_backward_saved", addr_val.data_ptr(), x.data_ptr(), gamma.data_ptr(), _code(x),
                  init_slot.data_ptr(), init_mass.data_ptr(), D_y.data_ptr(), nat.ptr(D_post_slot),
                  nat.ptr(D_post_mass), D_addr.data_ptr(), D_x.data_ptr(), D_gamma.data_ptr(), D_slot.data_ptr(),
@@ -598,7 +598,7 @@ def topk_segment_forward_(addr_idx: Tensor, addr_val: Tensor, x: Tensor, gamma: 
     mass_in = mass.clone()
     y = torch.empty_like(x)
     ws = _workspace(x, B, H, T, A, C, w_top_k, r_top_k)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_segment_forward_", addr_idx.data_ptr(), addr_val.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), nat.ptr(mask), slot.data_ptr(), mass.data_ptr(), mass_in.data_ptr(),
                  y.data_ptr(), B, H, T, A, C, w_top_k, r_top_k, int(mass_aware), float(eps), ws.data_ptr(),
@@ -642,7 +642,7 @@ def _ram_attn_call(w_addr, r_addr, x, gamma, mask, embed_num, position_ids, init
     pos, pos_s = _position_words(position_ids.to(device=x.device))
     ws = _workspace(x, B, H, T, A, C, w_top_k, r_top_k)
     at = nat.strides(*w_addr.stride(), *r_addr.stride(), *x.stride()[:3], *y.stride()[:3], *gamma.stride(), *pos_s)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_ram_attn_forward_strided", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(), gamma.data_ptr(),
                  _code(x), nat.ptr(mask), embed_num, pos.data_ptr(), init_slot.data_ptr(), init_mass.data_ptr(),
                  slot.data_ptr(), mass.data_ptr(), y.data_ptr(), B, H, U, P, T, A, C, w_top_k, r_top_k,
@@ -717,7 +717,7 @@ def topk_autoregressive_(w_addr: Tensor, r_addr: Tensor, x: Tensor, gamma: Tenso
     pos, pos_s = _position_words(position_ids.to(device=x.device))
     m = None if mask is None or mask.numel() == 0 else mask.to(device=x.device, dtype=torch.bool).contiguous()
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_autoregressive_strided_", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(), gamma.data_ptr(),
                  _code(x), slot.data_ptr(), mass.data_ptr(), nat.ptr(m), embed_num, pos.data_ptr(), B, H, U, P, A, C,
                  w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), int(mass_aware), float(eps),
@@ -757,7 +757,7 @@ def topk_autoregressive_steps_(w_addr: Tensor, r_addr: Tensor, x: Tensor, gamma:
     pos, pos_s = _position_words(position_ids.to(device=x.device))
     m = None if mask is None or mask.numel() == 0 else mask.to(device=x.device, dtype=torch.bool).contiguous()
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with nat.on_device(x):
         nat.call("ramnet_topk_autoregressive_steps_strided_", w_addr.data_ptr(), r_addr.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), slot.data_ptr(), mass.data_ptr(), nat.ptr(m), embed_num, pos.data_ptr(),
                  S, B, H, U, P, A, C, w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), int(mass_aware),

@@ -47,9 +47,9 @@ def _cuda_topk_autoregressive_(
     assert slot_.is_contiguous() and mass_.is_contiguous(), \
         f"Expected contiguous state, got slot={slot_.is_contiguous()}, mass={mass_.is_contiguous()}."
     empty = torch.empty(0, dtype=torch.bool, device=x.device)
-    mask = empty if mask is None else mask.to(device=x.device, dtype=torch.bool).contiguous()
+    mask = empty if mask is None else mask.to(device=x.device, dtype=torch.bool)
     return torch.ops.ramnet_ops.topk_autoregressive_(
-        w_addr.contiguous(), r_addr.contiguous(), x.contiguous(), gamma.contiguous(), slot_, mass_,
+        w_addr, r_addr, x, gamma, slot_, mass_,
         mask, embed_num, position_ids, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps)
 
 
@@ -83,26 +83,13 @@ def _cuda_ram_attn(
     B, H, T, C = xs.shape
     U, P = w_addr.shape[2], w_addr.shape[3]
     A = P ** U
-    w_top_k, r_top_k = top_k
-    w_re, r_re = (float(v) for v in top_k_re_norm)
     assert all(k <= A for k in top_k), f"Expected top_k <= A={A}, got {top_k}."
     assert isinstance(embed_num, int) and 0 <= embed_num <= H, f"Expected embed_num in [0, {H}], got {embed_num!r}."
-    assert A < ADDRESS_LIMIT, f"Address space overflow: A={A}, limit={ADDRESS_LIMIT}."
-    check_int_capacity(B, H, U, P, A, C, T, embed_num, w_top_k, r_top_k,
-                       B * H * U * P * T, B * H * A * C, B * H * T * C, B * H * T * (w_top_k + r_top_k))
-
-    requires_grad = torch.is_grad_enabled() and any(
-        t.requires_grad for t in (w_addr, r_addr, xs, gamma, init_slot, init_mass))
-    # the decoders read int64 positions where they are
-    position_ids = position_ids.to(device=xs.device,
-                                   dtype=None if position_ids.dtype in (torch.int32, torch.int64) else torch.int32)
-    if mask is not None:
-        mask = mask.to(device=xs.device, dtype=torch.bool)
 
     assert w_addr.dtype == r_addr.dtype == xs.dtype == gamma.dtype, \
         f"Expected matching dtypes, got w={w_addr.dtype}, r={r_addr.dtype}, x={xs.dtype}, gamma={gamma.dtype}."
     assert w_addr.device == r_addr.device == xs.device == gamma.device == init_slot.device == init_mass.device \
-        == position_ids.device, "Expected all inputs on one device."
+        == xs.device, "Expected all inputs on one device."
     expected_shapes = (
         ("w_addr", w_addr, (B, H, U, P, T)),
         ("r_addr", r_addr, (B, H, U, P, T)),
@@ -115,6 +102,30 @@ def _cuda_ram_attn(
     for name, tensor, shape in expected_shapes:
         assert tuple(tensor.shape) == shape, f"Expected {name}.shape == {shape}, but got {tuple(tensor.shape)}."
     assert mask is None or tuple(mask.shape) == (B, T), f"Expected mask.shape={(B, T)}, got {tuple(mask.shape)}."
+
+    return _cuda_ram_attn_run(w_addr, r_addr, xs, gamma, init_slot, init_mass, mask, embed_num, position_ids, top_k,
+                              tuple(float(v) for v in top_k_re_norm), mass_aware, eps, inplace)
+
+
+def _cuda_ram_attn_run(w_addr, r_addr, xs, gamma, init_slot, init_mass, mask, embed_num, position_ids, top_k,
+                       top_k_re_norm, mass_aware, eps, inplace):
+    """``_cuda_ram_attn`` on arguments of the shapes, dtypes and devices it checks."""
+    B, H, T, C = xs.shape
+    U, P = w_addr.shape[2], w_addr.shape[3]
+    A = P ** U
+    w_top_k, r_top_k = top_k
+    w_re, r_re = top_k_re_norm
+    assert A < ADDRESS_LIMIT, f"Address space overflow: A={A}, limit={ADDRESS_LIMIT}."
+    check_int_capacity(B, H, U, P, A, C, T, embed_num, w_top_k, r_top_k,
+                       B * H * U * P * T, B * H * A * C, B * H * T * C, B * H * T * (w_top_k + r_top_k))
+
+    requires_grad = torch.is_grad_enabled() and any(
+        t.requires_grad for t in (w_addr, r_addr, xs, gamma, init_slot, init_mass))
+    # the decoders read int64 positions where they are
+    position_ids = position_ids.to(device=xs.device,
+                                   dtype=None if position_ids.dtype in (torch.int32, torch.int64) else torch.int32)
+    if mask is not None:
+        mask = mask.to(device=xs.device, dtype=torch.bool)
 
     acc_type = torch.float32 if xs.dtype in (torch.float16, torch.bfloat16) else xs.dtype
     if acc_type != torch.float32:
