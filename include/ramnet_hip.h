@@ -293,6 +293,13 @@ int ramnet_ram_attn_forward(const void *w_addr, const void *r_addr, const void *
  *                      position_ids [b, t]   (12 values)
  *   topk_addr_single_forward  addr [b, h, u, p, t], position_ids [b, t]
  *                      (7 values)
+ *   topk_addr_backward w_addr, r_addr, grad_w_addr, grad_r_addr
+ *                      [b, h, u, p, t] each, position_ids [b, t]
+ *                      (22 values)
+ *   topk_segment_forward_save   x [b, h, t], y [b, h, t]   (6 values)
+ *   topk_segment_backward_saved grad_y [b, h, t], grad_x [b, h, t]
+ *                      (6 values); grad_x is in `dtype` where grad_x_typed
+ *                      is nonzero, else fp32
  *   topk_autoregressive_ (below)        position_ids [b]     (1 value)
  *   topk_autoregressive_steps_ (below)  position_ids [s, b]  (2 values)
  * Digits follow each other at P times the logits' stride; channels of x and
@@ -317,6 +324,24 @@ int ramnet_topk_addr_single_forward_strided(const void *addr, int dtype, int64_t
                                             int64_t top_k, float top_k_re_norm, int addr_val_neg,
                                             int encode_batch_idx, const int64_t *strides, int32_t *idx_out,
                                             float *val_out, void *stream);
+int ramnet_topk_addr_backward_strided(const int32_t *idx, const float *val, const void *w_addr, const void *r_addr,
+                                      const float *grad_val, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
+                                      int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
+                                      int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
+                                      const int64_t *strides, void *grad_w_addr, void *grad_r_addr, void *stream);
+int ramnet_topk_segment_forward_save_strided(const int32_t *addr_idx, const float *addr_val, const void *x,
+                                     const void *gamma, int dtype, const uint8_t *mask, const float *init_slot,
+                                     const float *init_mass, float *slot_out, float *mass_out, void *y, int64_t B,
+                                     int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
+                                     int mass_aware, float eps, void *workspace, int64_t workspace_bytes, void *saved,
+                                     int64_t saved_bytes, const int64_t *strides, void *stream);
+int ramnet_topk_segment_backward_saved_strided(const float *addr_val, const void *x, const void *gamma, int dtype,
+                                       const float *init_slot, const float *init_mass, const void *grad_y,
+                                       const float *grad_slot, const float *grad_mass, float *grad_addr_val,
+                                       void *grad_x, float *grad_gamma, float *grad_init_slot, float *grad_init_mass,
+                                       int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k,
+                                       int64_t r_top_k, int mass_aware, float eps, const void *saved,
+                                       int64_t saved_bytes, const int64_t *strides, int grad_x_typed, void *workspace, int64_t workspace_bytes, void *stream);
 int ramnet_topk_autoregressive_strided_(const void *w_addr, const void *r_addr, const void *x, const void *gamma,
                                         int dtype, float *slot, float *mass, const uint8_t *mask, int64_t embed_num,
                                         const int32_t *position_ids, int64_t B, int64_t H, int64_t U, int64_t P,

@@ -135,8 +135,22 @@ int check_logits(const int64_t (&s)[5], int64_t B, int64_t H, int64_t U, int64_t
 int addr_backward(const int32_t *idx, const float *val, const void *addr, const float *grad_val, int dtype,
                   int64_t B, int64_t H, int64_t U, int64_t P, int64_t T, int64_t embed_num, int64_t A,
                   const int32_t *position_ids, int64_t k_total, int64_t k_off, int64_t top_k, float re_norm,
-                  float sign, void *grad_addr, void *stream) {
+                  float sign, const int64_t (&at)[5], const int64_t (&grad_at)[5], const int64_t (&pos)[2],
+                  void *grad_addr, void *stream) {
+    if (int rc = check_logits(at, B, H, U, P, T))
+        return rc;
+    if (int rc = check_logits(grad_at, B, H, U, P, T))
+        return rc;
+    RAMNET_REQUIRE(stride_ok(pos, {B, T}), "position strides must be >= 0 and within int32");
     ramnet::AddrBwdJob job{};
+    const int dims[3] = {0, 1, 4};
+    for (int d = 0; d < 3; ++d) {
+        job.stride[d] = at[dims[d]];
+        job.grad_stride[d] = grad_at[dims[d]];
+    }
+    job.step = static_cast<int>(at[3]);
+    job.grad_step = static_cast<int>(grad_at[3]);
+    std::copy_n(pos, 2, job.pos_stride);
     job.addr = addr;
     job.idx = idx;
     job.val = val;
@@ -246,15 +260,16 @@ int ramnet_topk_addr_single_backward(const int32_t *idx, const float *val, const
     if (B * H * T == 0)
         return RAMNET_OK;
     RAMNET_REQUIRE(idx && val && addr && grad_val && position_ids && grad_addr, "null tensor pointer");
+    const Layout lay = memory_order(B, H, U, P, T, 1);
     return addr_backward(idx, val, addr, grad_val, dtype, B, H, U, P, T, embed_num, A, position_ids, top_k, 0, top_k,
-                         top_k_re_norm, addr_val_neg ? -1.f : 1.f, grad_addr, stream);
+                         top_k_re_norm, addr_val_neg ? -1.f : 1.f, lay.w, lay.w, lay.pos, grad_addr, stream);
 }
 
-int ramnet_topk_addr_backward(const int32_t *idx, const float *val, const void *w_addr, const void *r_addr,
+static int topk_addr_backward(const int32_t *idx, const float *val, const void *w_addr, const void *r_addr,
                               const float *grad_val, int dtype, int64_t B, int64_t H, int64_t U, int64_t P, int64_t T,
                               int64_t embed_num, int64_t A, const int32_t *position_ids, int64_t w_top_k,
-                              int64_t r_top_k, float w_re_norm, float r_re_norm, void *grad_w_addr,
-                              void *grad_r_addr, void *stream) {
+                              int64_t r_top_k, float w_re_norm, float r_re_norm, const Layout &lay,
+                              const Layout &grad, void *grad_w_addr, void *grad_r_addr, void *stream) {
     if (int rc = check_addr_shape(B, H, U, P, T, embed_num, A))
         return rc;
     RAMNET_REQUIRE(valid_dtype(dtype), "addr dtype must be float32, float16 or bfloat16");
@@ -269,10 +284,36 @@ int ramnet_topk_addr_backward(const int32_t *idx, const float *val, const void *
                    "null tensor pointer");
     const int64_t kt = w_top_k + r_top_k;
     if (int rc = addr_backward(idx, val, w_addr, grad_val, dtype, B, H, U, P, T, embed_num, A, position_ids, kt, 0,
-                               w_top_k, w_re_norm, 1.f, grad_w_addr, stream))
+                               w_top_k, w_re_norm, 1.f, lay.w, grad.w, lay.pos, grad_w_addr, stream))
         return rc;
     return addr_backward(idx, val, r_addr, grad_val, dtype, B, H, U, P, T, embed_num, A, position_ids, kt, w_top_k,
-                         r_top_k, r_re_norm, -1.f, grad_r_addr, stream);
+                         r_top_k, r_re_norm, -1.f, lay.r, grad.r, lay.pos, grad_r_addr, stream);
+}
+
+int ramnet_topk_addr_backward(const int32_t *idx, const float *val, const void *w_addr, const void *r_addr,
+                              const float *grad_val, int dtype, int64_t B, int64_t H, int64_t U, int64_t P, int64_t T,
+                              int64_t embed_num, int64_t A, const int32_t *position_ids, int64_t w_top_k,
+                              int64_t r_top_k, float w_re_norm, float r_re_norm, void *grad_w_addr,
+                              void *grad_r_addr, void *stream) {
+    const Layout lay = memory_order(B, H, U, P, T, 1);
+    return topk_addr_backward(idx, val, w_addr, r_addr, grad_val, dtype, B, H, U, P, T, embed_num, A, position_ids,
+                              w_top_k, r_top_k, w_re_norm, r_re_norm, lay, lay, grad_w_addr, grad_r_addr, stream);
+}
+
+int ramnet_topk_addr_backward_strided(const int32_t *idx, const float *val, const void *w_addr, const void *r_addr,
+                                      const float *grad_val, int dtype, int64_t B, int64_t H, int64_t U, int64_t P,
+                                      int64_t T, int64_t embed_num, int64_t A, const int32_t *position_ids,
+                                      int64_t w_top_k, int64_t r_top_k, float w_re_norm, float r_re_norm,
+                                      const int64_t *strides, void *grad_w_addr, void *grad_r_addr, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    Layout lay{}, grad{};
+    std::copy_n(strides, 5, lay.w);
+    std::copy_n(strides + 5, 5, lay.r);
+    std::copy_n(strides + 10, 5, grad.w);
+    std::copy_n(strides + 15, 5, grad.r);
+    std::copy_n(strides + 20, 2, lay.pos);
+    return topk_addr_backward(idx, val, w_addr, r_addr, grad_val, dtype, B, H, U, P, T, embed_num, A, position_ids,
+                              w_top_k, r_top_k, w_re_norm, r_re_norm, lay, grad, grad_w_addr, grad_r_addr, stream);
 }
 
 static int topk_addr_forward(const void *w_addr, const void *r_addr, int dtype, int64_t B, int64_t H, int64_t U,
@@ -720,6 +761,9 @@ int ramnet_topk_segment_backward(const int32_t *addr_idx, const float *addr_val,
             return finish(err, why, "topk_segment_backward launch");
     }
     ramnet::SegmentBwdJob job{};
+    const Layout lay = memory_order(B, H, 1, 1, T, C);
+    std::copy_n(lay.y, 3, job.dy_stride);
+    std::copy_n(lay.x, 3, job.gx_stride);
     job.fwd = fj;
     job.addr_val = addr_val;
     job.gamma = gamma;
@@ -786,12 +830,12 @@ int64_t ramnet_segment_saved_bytes(int64_t B, int64_t H, int64_t T, int64_t A, i
     return saved_layout(B, H, T, A, C, w_top_k, r_top_k, dtype, &geo, &parts) ? parts.total() : -1;
 }
 
-int ramnet_topk_segment_forward_save(const int32_t *addr_idx, const float *addr_val, const void *x,
+static int segment_forward_save(const int32_t *addr_idx, const float *addr_val, const void *x,
                                      const void *gamma, int dtype, const uint8_t *mask, const float *init_slot,
                                      const float *init_mass, float *slot_out, float *mass_out, void *y, int64_t B,
                                      int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
                                      int mass_aware, float eps, void *workspace, int64_t workspace_bytes, void *saved,
-                                     int64_t saved_bytes, void *stream) {
+                                     int64_t saved_bytes, const Layout &at, void *stream) {
     if (int rc = segment_checks(x, gamma, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C, w_top_k,
                                 r_top_k, eps, workspace, workspace_bytes))
         return rc;
@@ -803,6 +847,10 @@ int ramnet_topk_segment_forward_save(const int32_t *addr_idx, const float *addr_
     RAMNET_REQUIRE(addr_idx && addr_val, "null tensor pointer");
     ramnet::SegmentJob job = make_segment_job(x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C,
                                               w_top_k, r_top_k, mass_aware, eps, workspace);
+    RAMNET_REQUIRE(T == 0 || (stride_ok(at.x, {B, H, T}) && stride_dense(at.y, B, H, T, C)),
+                   "x strides must be >= 0 and within int32, y's rows must fill B * H * T * C elements");
+    std::copy_n(at.x, 3, job.x_stride);
+    std::copy_n(at.y, 3, job.y_stride);
     char *sv = static_cast<char *>(saved);
     job.wrec = reinterpret_cast<const ramnet::WriteRec *>(sv);
     job.rrec = reinterpret_cast<const ramnet::ReadRec *>(sv + B * H * ramnet::scan_t_pad64(T) * w_top_k *
@@ -817,6 +865,32 @@ int ramnet_topk_segment_forward_save(const int32_t *addr_idx, const float *addr_
     return finish(err, why, "topk_segment_forward_save launch");
 }
 
+int ramnet_topk_segment_forward_save(const int32_t *addr_idx, const float *addr_val, const void *x,
+                                     const void *gamma, int dtype, const uint8_t *mask, const float *init_slot,
+                                     const float *init_mass, float *slot_out, float *mass_out, void *y, int64_t B,
+                                     int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
+                                     int mass_aware, float eps, void *workspace, int64_t workspace_bytes, void *saved,
+                                     int64_t saved_bytes, void *stream) {
+    return segment_forward_save(addr_idx, addr_val, x, gamma, dtype, mask, init_slot, init_mass, slot_out, mass_out, y,
+                                B, H, T, A, C, w_top_k, r_top_k, mass_aware, eps, workspace, workspace_bytes, saved,
+                                saved_bytes, memory_order(B, H, 1, 1, T, C), stream);
+}
+
+int ramnet_topk_segment_forward_save_strided(const int32_t *addr_idx, const float *addr_val, const void *x,
+                                     const void *gamma, int dtype, const uint8_t *mask, const float *init_slot,
+                                     const float *init_mass, float *slot_out, float *mass_out, void *y, int64_t B,
+                                     int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
+                                     int mass_aware, float eps, void *workspace, int64_t workspace_bytes, void *saved,
+                                     int64_t saved_bytes, const int64_t *strides, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    Layout at{};
+    std::copy_n(strides, 3, at.x);
+    std::copy_n(strides + 3, 3, at.y);
+    return segment_forward_save(addr_idx, addr_val, x, gamma, dtype, mask, init_slot, init_mass, slot_out, mass_out, y,
+                                B, H, T, A, C, w_top_k, r_top_k, mass_aware, eps, workspace, workspace_bytes, saved,
+                                saved_bytes, at, stream);
+}
+
 int64_t ramnet_segment_backward_saved_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t A, int64_t C,
                                                       int64_t w_top_k, int64_t r_top_k) {
     if (backward_workspace_bytes(B, H, T, A, C, w_top_k, r_top_k) < 0)
@@ -826,13 +900,14 @@ int64_t ramnet_segment_backward_saved_workspace_bytes(int64_t B, int64_t H, int6
                                            static_cast<int>(r_top_k), nullptr, nullptr, true);
 }
 
-int ramnet_topk_segment_backward_saved(const float *addr_val, const void *x, const void *gamma, int dtype,
+static int segment_backward_saved(const float *addr_val, const void *x, const void *gamma, int dtype,
                                        const float *init_slot, const float *init_mass, const void *grad_y,
                                        const float *grad_slot, const float *grad_mass, float *grad_addr_val,
-                                       float *grad_x, float *grad_gamma, float *grad_init_slot, float *grad_init_mass,
+                                       void *grad_x, float *grad_gamma, float *grad_init_slot, float *grad_init_mass,
                                        int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k,
                                        int64_t r_top_k, int mass_aware, float eps, const void *saved,
-                                       int64_t saved_bytes, void *workspace, int64_t workspace_bytes, void *stream) {
+                                       int64_t saved_bytes, const Layout &at, int grad_x_typed, void *workspace,
+                                  int64_t workspace_bytes, void *stream) {
     const int64_t need = ramnet_segment_backward_saved_workspace_bytes(B, H, T, A, C, w_top_k, r_top_k);
     if (int rc = segment_checks(x, gamma, dtype, init_slot, init_mass, grad_init_slot, grad_init_mass, grad_x, B, H,
                                 T, A, C, w_top_k, r_top_k, eps, workspace, workspace_bytes, need < 0 ? 0 : need))
@@ -845,6 +920,8 @@ int ramnet_topk_segment_backward_saved(const float *addr_val, const void *x, con
     RAMNET_REQUIRE(workspace_bytes >= need && workspace,
                    "workspace too small: see ramnet_segment_backward_saved_workspace_bytes");
     RAMNET_REQUIRE(addr_val && grad_y && grad_addr_val && grad_gamma, "null tensor pointer");
+    RAMNET_REQUIRE(T == 0 || (stride_ok(at.y, {B, H, T}) && stride_ok(at.x, {B, H, T})),
+                   "grad_y and grad_x strides must be >= 0 and within int32");
     // the records were packed into the saved buffer by the forward
     ramnet::SegmentJob fj = make_segment_job(x, dtype, init_slot, init_mass, nullptr, nullptr, nullptr, B, H, T, A, C,
                                              w_top_k, r_top_k, mass_aware, eps, const_cast<void *>(saved));
@@ -855,6 +932,9 @@ int ramnet_topk_segment_backward_saved(const float *addr_val, const void *x, con
     job.addr_val = addr_val;
     job.gamma = gamma;
     job.grad_y = grad_y;
+    job.grad_x_typed = grad_x_typed;
+    std::copy_n(at.y, 3, job.dy_stride);
+    std::copy_n(at.x, 3, job.gx_stride);
     job.grad_slot = grad_slot;
     job.grad_mass = grad_mass;
     job.grad_val = grad_addr_val;
@@ -875,6 +955,36 @@ int ramnet_topk_segment_backward_saved(const float *addr_val, const void *x, con
     const char *why = nullptr;
     const hipError_t err = ramnet::launch_segment_backward(job, static_cast<hipStream_t>(stream), &why);
     return finish(err, why, "topk_segment_backward_saved launch");
+}
+
+int ramnet_topk_segment_backward_saved(const float *addr_val, const void *x, const void *gamma, int dtype,
+                                       const float *init_slot, const float *init_mass, const void *grad_y,
+                                       const float *grad_slot, const float *grad_mass, float *grad_addr_val,
+                                       float *grad_x, float *grad_gamma, float *grad_init_slot, float *grad_init_mass,
+                                       int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k,
+                                       int64_t r_top_k, int mass_aware, float eps, const void *saved,
+                                       int64_t saved_bytes, void *workspace, int64_t workspace_bytes, void *stream) {
+    return segment_backward_saved(addr_val, x, gamma, dtype, init_slot, init_mass, grad_y, grad_slot, grad_mass,
+                                  grad_addr_val, grad_x, grad_gamma, grad_init_slot, grad_init_mass, B, H, T, A, C,
+                                  w_top_k, r_top_k, mass_aware, eps, saved, saved_bytes, memory_order(B, H, 1, 1, T, C),
+                                  0, workspace, workspace_bytes, stream);
+}
+
+int ramnet_topk_segment_backward_saved_strided(const float *addr_val, const void *x, const void *gamma, int dtype,
+                                       const float *init_slot, const float *init_mass, const void *grad_y,
+                                       const float *grad_slot, const float *grad_mass, float *grad_addr_val,
+                                       void *grad_x, float *grad_gamma, float *grad_init_slot, float *grad_init_mass,
+                                       int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k,
+                                       int64_t r_top_k, int mass_aware, float eps, const void *saved,
+                                       int64_t saved_bytes, const int64_t *strides, int grad_x_typed, void *workspace, int64_t workspace_bytes, void *stream) {
+    RAMNET_REQUIRE(strides, "null strides");
+    Layout at{};
+    std::copy_n(strides, 3, at.y);      // grad_y
+    std::copy_n(strides + 3, 3, at.x);  // grad_x
+    return segment_backward_saved(addr_val, x, gamma, dtype, init_slot, init_mass, grad_y, grad_slot, grad_mass,
+                                  grad_addr_val, grad_x, grad_gamma, grad_init_slot, grad_init_mass, B, H, T, A, C,
+                                  w_top_k, r_top_k, mass_aware, eps, saved, saved_bytes, at, grad_x_typed ? 1 : 0,
+                                  workspace, workspace_bytes, stream);
 }
 
 // Checks and job of one decode step (S = 1) or S steps of one shape.

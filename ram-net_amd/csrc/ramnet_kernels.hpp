@@ -106,11 +106,15 @@ struct AddrJob {
 // (positive-weight convention) -> gradient of the logits.
 struct AddrBwdJob {
     const void *addr;             // (B, H, U, P, T) logits in dtype
+    // strides as in AddrSource: of the logits, and of their gradients
+    int64_t stride[3], grad_stride[3];
+    int step, grad_step;
     const int32_t *idx;           // (B, H, k_total, T), this source at k_off .. k_off + K
     const float *val;             // (B, H, k_total, T), stored weights (negated when sign < 0)
     const float *grad_val;        // (B, H, k_total, T), gradient of the positive weights
     void *grad_addr;              // (B, H, U, P, T) in dtype
-    const int32_t *position_ids;  // (B, T)
+    const int32_t *position_ids;  // by strides, as in AddrJob
+    int64_t pos_stride[2];
     int dtype;
     int B, H, U, P, T, A;
     int embed_num;
@@ -170,7 +174,7 @@ struct SegmentJob {
     // elements between batch rows, heads and tokens of x and y (channels are
     // adjacent): (B, H, T, C) in memory order unless the caller says
     // otherwise. y's rows fill B * H * T * C elements in some order of b, h
-    // and t. Forward scans only; the backward takes contiguous tensors.
+    // and t.
     int64_t x_stride[3], y_stride[3];
     int dtype;
     int B, H, T, A, C, Kw, Kr;
@@ -189,7 +193,9 @@ struct SegmentBwdJob {
     const float *grad_slot;   // (B, H, A, C) or null (zero)
     const float *grad_mass;   // (B, H, A) or null (zero)
     float *grad_val;          // (B, H, Kw + Kr, T): positive-weight gradients
-    float *grad_x;            // (B, H, T, C)
+    void *grad_x;             // (B, H, T, C): fp32, or dtype where grad_x_typed
+    int grad_x_typed;
+    int64_t dy_stride[3], gx_stride[3];  // of grad_y and grad_x, as x_stride
     float *grad_gamma;        // (B, H, T)
     float *grad_init_slot;    // (B, H, A, C)
     float *grad_init_mass;    // (B, H, A)

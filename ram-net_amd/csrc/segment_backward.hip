@@ -224,13 +224,14 @@ __global__ __launch_bounds__(kWave) void segment_bwd_scan_kernel(const SegmentBw
         const int t = decltype(fwd_tag)::value ? ci * CH + j : T - 1 - ci * CH - j;
         return min(max(t, 0), T - 1);
     };
-    // Offsets within the head are 32-bit (T * K and T * C fit an int: the
-    // host checks B * H * T * C and B * H * T_pad * (Kw + Kr)), from bases
+    // Offsets within the head are 32-bit (the host checks that T * K and the
+    // tensors' reach by their strides fit an int), from bases
     // per head, so a load costs no 64-bit index arithmetic.
     const int4 *wev_h = job.aux.wev + static_cast<int64_t>(bh) * T * Kw;
     const int2 *rev_h = rev2 + 2 * static_cast<int64_t>(bh) * T * Kr;
-    const Scalar *dy_h = dys + static_cast<int64_t>(bh) * T * C;
-    const Scalar *x_h = xs + static_cast<int64_t>(bh) * T * C;
+    const Scalar *dy_h = dys + row_offset(job.dy_stride, fj.H, bh);
+    const Scalar *x_h = xs + row_offset(fj.x_stride, fj.H, bh);
+    const int dyt = static_cast<int>(job.dy_stride[2]), xt = static_cast<int>(fj.x_stride[2]);
     auto prefetch = [&](int ci, Pre &pf, auto fwd_tag) {
 #pragma unroll
         for (int i = 0; i < RPL; ++i) {
@@ -244,10 +245,10 @@ __global__ __launch_bounds__(kWave) void segment_bwd_scan_kernel(const SegmentBw
         for (int i = 0; i < XPL; ++i) {
             const int idx = min(lane + kWave * i, NXE - 1);
             const int c = min(sub * CSW + idx % CSW, C - 1);
-            const uint32_t o = static_cast<uint32_t>(token(ci, idx / CSW, fwd_tag) * C + c);
-            pf.dy[i] = raw_load(dy_h + o);
+            const int t = token(ci, idx / CSW, fwd_tag);
+            pf.dy[i] = raw_load(dy_h + static_cast<uint32_t>(t * dyt + c));
             if constexpr (decltype(fwd_tag)::value)
-                pf.x[i] = raw_load(x_h + o);
+                pf.x[i] = raw_load(x_h + static_cast<uint32_t>(t * xt + c));
         }
     };
     auto stage = [&](const Pre &pf, auto fwd_tag) {
@@ -510,7 +511,9 @@ __global__ __launch_bounds__(kWave) void segment_bwd_scan_kernel(const SegmentBw
             float dr[SAVED ? NG : 1][NP];  // SAVED: d_j of token (group start - q)
         };
         Out out;
-        float *gx = job.grad_x + static_cast<int64_t>(bh) * T * C;
+        const int64_t gx_head = row_offset(job.gx_stride, fj.H, bh), gxt = job.gx_stride[2];
+        float *gx = static_cast<float *>(job.grad_x) + gx_head;
+        Scalar *gx_typed = static_cast<Scalar *>(job.grad_x) + gx_head;
         auto flush = [&](int ci) {
             const int n = min(CH, T - ci * CH);
             const int t0 = T - 1 - ci * CH;  // the chunk's first token; group g's in this lane: t0 - g * LPE - q (Dg), t0 - g * GX - e (Dx)
@@ -534,8 +537,12 @@ __global__ __launch_bounds__(kWave) void segment_bwd_scan_kernel(const SegmentBw
                             const int64_t tg = t0 - g * GX - e;
 #pragma unroll
                             for (int v = 0; v < VEC; ++v)
-                                if (c0 + v < C)
-                                    gx[tg * C + c0 + v] = out.gx[g][v];
+                                if (c0 + v < C) {
+                                    if (job.grad_x_typed)
+                                        store_f32(gx_typed + tg * gxt + c0 + v, out.gx[g][v]);
+                                    else
+                                        gx[tg * gxt + c0 + v] = out.gx[g][v];
+                                }
                         }
                 }
             };

@@ -419,6 +419,15 @@ hipError_t launch_typed(const AddrJob &job, hipStream_t stream, const char **why
     return hipGetLastError();
 }
 
+// The 16 bits of v in a 16-bit type, rounded as store_f32 rounds.
+template<typename Scalar>
+__device__ __forceinline__ uint32_t half_bits(float v) {
+    if constexpr (__is_same(Scalar, bf16_t))
+        return f32_to_bf16_bits(v);
+    else
+        return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
+}
+
 // ---- backward (reference: csrc/ram_attn_topk_addr.cu:119-226)
 //
 // With v_k the selected weights, D_k = dL/dv_k * v_k is the gradient of the
@@ -431,13 +440,16 @@ hipError_t launch_typed(const AddrJob &job, hipStream_t stream, const char **why
 // logits of a digit are read coalesced across the lanes' consecutive t,
 // once into registers when P <= PR, else in three passes (max, sum,
 // gradient). KM > 0 keeps the K terms in registers; KM = 0 streams them for
-// any K. BUF (P == PR, and every lane's offsets from the wave's first lane
-// fit in 31 bits): the logits and their gradients go through buffer
-// resources based at the wave's first lane, with 32-bit lane offsets, so the
-// 2 * U * P per-lane addresses are not kept in (spilled) scalar registers.
-template<typename Scalar, int KM, int PR, bool BUF = false>
+// any K. LAY as in the forward: kLaneBuffer (memory order, P == PR, and every
+// lane's offsets from the wave's first lane fit in 31 bits): the logits and
+// their gradients go through buffer resources based at the wave's first
+// lane, with 32-bit lane offsets, so the 2 * U * P per-lane addresses are not
+// kept in (spilled) scalar registers. kLaneRow, kLaneRowPart: rows of
+// adjacent logits read, and rows of gradients written, 16 bytes at a time.
+template<typename Scalar, int KM, int PR, int LAY = kLaneAny>
 __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJob job) {
-    static_assert(!BUF || PR > 0, "buffer resources: the logits held in registers");
+    constexpr bool BUF = LAY == kLaneBuffer, ROW = LAY == kLaneRow || LAY == kLaneRowPart;
+    static_assert(LAY == kLaneAny || PR > 0, "the logits held in registers");
     const int T = job.T, H = job.H, A = job.A, P = job.P, U = job.U, K = job.K;
     const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (gid >= static_cast<int64_t>(job.B) * H * T)
@@ -447,7 +459,8 @@ __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJo
     const int b = static_cast<int>(bh / H), h = static_cast<int>(bh % H);
     const int64_t row0 = (bh * job.k_total + job.k_off) * T + t;  // event k at row0 + k * T
     const float re = job.re_norm;
-    const int shift = h < job.embed_num ? pos_mod(job.position_ids[static_cast<int64_t>(b) * T + t], A) : 0;
+    const int shift = h < job.embed_num ? pos_mod(job.position_ids[b * job.pos_stride[0] + t * job.pos_stride[1]], A)
+                                        : 0;
     auto weight = [&](int k) { return job.sign * job.val[row0 + static_cast<int64_t>(k) * T]; };
     auto dscore = [&](int k) { return job.grad_val[row0 + static_cast<int64_t>(k) * T] * weight(k); };
     auto content = [&](int k) {
@@ -499,8 +512,10 @@ __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJo
         }
     }
     const float dsoft = (1.f - re) * dsum;
-    const Scalar *xp = static_cast<const Scalar *>(job.addr) + bh * U * P * static_cast<int64_t>(T) + t;
-    Scalar *gp = static_cast<Scalar *>(job.grad_addr) + bh * U * P * static_cast<int64_t>(T) + t;
+    const Scalar *xp = static_cast<const Scalar *>(job.addr) + b * job.stride[0] + h * job.stride[1] + t * job.stride[2];
+    Scalar *gp = static_cast<Scalar *>(job.grad_addr) + b * job.grad_stride[0] + h * job.grad_stride[1] +
+                 t * job.grad_stride[2];
+    const int64_t xs = job.step, gs = job.grad_step;
     // BUF: resources based at the first active lane's logit and gradient
     // (later lanes are at equal or higher addresses, within 2 * U * P * T
     // elements: a wave spans at most two (b, h) rows). readfirstlane returns
@@ -520,8 +535,8 @@ __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJo
     [[maybe_unused]] const int step = T * static_cast<int>(sizeof(Scalar));
     int stride = 1;
     for (int u = 0; u < U; ++u, stride *= P) {
-        const Scalar *xu = xp + static_cast<int64_t>(u) * P * T;
-        Scalar *gu = gp + static_cast<int64_t>(u) * P * T;
+        const Scalar *xu = xp + u * P * xs;
+        Scalar *gu = gp + u * P * gs;
         float xr[PR > 0 ? PR : 1];  // the digit's logits, then their exponentials
         float mx = -__builtin_huge_valf();
         if constexpr (BUF) {
@@ -536,15 +551,23 @@ __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJo
                 xr[q] = bits_f32<Scalar>(bits);
                 mx = fmaxf(mx, xr[q]);
             }
+        } else if constexpr (ROW) {
+            uint32_t bits[PR];
+            RowLogits<Scalar, PR, LAY == kLaneRow>{xp, P}.digit(u, bits);
+#pragma unroll
+            for (int q = 0; q < PR; ++q) {
+                xr[q] = bits_value<Scalar>(bits[q]);
+                mx = LAY == kLaneRow || q < P ? fmaxf(mx, xr[q]) : mx;
+            }
         } else if constexpr (PR > 0) {
 #pragma unroll
             for (int q = 0; q < PR; ++q) {
-                xr[q] = load_f32(xu + static_cast<int64_t>(q < P ? q : P - 1) * T);
+                xr[q] = load_f32(xu + (q < P ? q : P - 1) * xs);
                 mx = q < P ? fmaxf(mx, xr[q]) : mx;
             }
         } else {
             for (int q = 0; q < P; ++q)
-                mx = fmaxf(mx, load_f32(xu + static_cast<int64_t>(q) * T));
+                mx = fmaxf(mx, load_f32(xu + q * xs));
         }
         const bool live = mx > -__builtin_huge_valf();
         float se = 0.f;
@@ -559,7 +582,7 @@ __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJo
             }
         } else {
             for (int q = 0; q < P; ++q)
-                se += live ? expf(load_f32(xu + static_cast<int64_t>(q) * T) - mx) : 0.f;
+                se += live ? expf(load_f32(xu + q * xs) - mx) : 0.f;
         }
         const float scale = live ? dsoft / se : 0.f;
         int du[KM > 0 ? KM : 1];
@@ -596,27 +619,47 @@ __global__ __launch_bounds__(256) void topk_addr_backward_kernel(const AddrBwdJo
                 const float v = grad_of(q) - xr[q] * scale;
                 if constexpr (sizeof(Scalar) == 4)
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), grs, o, 0, 0);
-                else if constexpr (__is_same(Scalar, bf16_t))
-                    __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16_bits(v), grs, o, 0, 0);
                 else
-                    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, static_cast<_Float16>(v)), grs, o,
-                                                          0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(half_bits<Scalar>(v)), grs, o, 0, 0);
+            }
+        } else if constexpr (ROW) {
+            constexpr int ES = static_cast<int>(sizeof(Scalar));
+            constexpr int PIECE = row_piece_bytes<Scalar, PR>(), N = PR * ES / PIECE, E = PIECE / ES;
+            typedef uint32_t Words __attribute__((ext_vector_type(PIECE / 4)));
+            char *row = reinterpret_cast<char *>(gu);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                if (LAY == kLaneRow || i * E < P) {  // uniform
+                    Words w;
+#pragma unroll
+                    for (int e = 0; e < E; e += 4 / ES) {
+                        const int q = i * E + e;
+                        const float v = grad_of(q) - xr[q] * scale;
+                        if constexpr (ES == 4) {
+                            w[e] = __float_as_uint(v);
+                        } else {
+                            const float v2 = grad_of(q + 1) - xr[q + 1] * scale;
+                            w[e / 2] = half_bits<Scalar>(v) | half_bits<Scalar>(v2) << 16;
+                        }
+                    }
+                    *reinterpret_cast<Words *>(row + i * PIECE) = w;
+                }
             }
         } else if constexpr (PR > 0) {
             if (P == PR) {  // the common case: stores without a branch each
 #pragma unroll
                 for (int q = 0; q < PR; ++q)
-                    store_f32(gu + static_cast<int64_t>(q) * T, grad_of(q) - xr[q] * scale);
+                    store_f32(gu + q * gs, grad_of(q) - xr[q] * scale);
             } else {
 #pragma unroll
                 for (int q = 0; q < PR; ++q)
                     if (q < P)
-                        store_f32(gu + static_cast<int64_t>(q) * T, grad_of(q) - xr[q] * scale);
+                        store_f32(gu + q * gs, grad_of(q) - xr[q] * scale);
             }
         } else {
             for (int q = 0; q < P; ++q) {
-                const float sm = live ? expf(load_f32(xu + static_cast<int64_t>(q) * T) - mx) : 0.f;
-                store_f32(gu + static_cast<int64_t>(q) * T, grad_of(q) - sm * scale);
+                const float sm = live ? expf(load_f32(xu + q * xs) - mx) : 0.f;
+                store_f32(gu + q * gs, grad_of(q) - sm * scale);
             }
         }
     }
@@ -627,22 +670,45 @@ hipError_t launch_backward_typed(const AddrBwdJob &job, hipStream_t stream) {
     const int64_t n = static_cast<int64_t>(job.B) * job.H * job.T;
     const dim3 grid(static_cast<unsigned>((n + 255) / 256)), blk(256);
     // a digit's logits fit in registers up to P = 32; P = 16 has its own
-    // instance, whose stores need no per-logit branch
+    // instances, whose stores need no per-logit branch
+    const int64_t up = static_cast<int64_t>(job.U) * job.P, piece = row_piece_bytes<T, 16>();
+    const int n_of[3] = {job.B, job.H, job.T};
+    const int64_t order[3] = {job.H * up * job.T, up * job.T, 1};
+    bool buf = job.step == job.T && job.grad_step == job.T;
+    bool row = job.step == 1 && job.grad_step == 1 && job.P * static_cast<int64_t>(sizeof(T)) % piece == 0 &&
+               reinterpret_cast<uintptr_t>(job.addr) % piece == 0 &&
+               reinterpret_cast<uintptr_t>(job.grad_addr) % piece == 0;
+    for (int d = 0; d < 3; ++d) {
+        if (n_of[d] == 1)
+            continue;
+        buf = buf && job.stride[d] == order[d] && job.grad_stride[d] == order[d];
+        row = row && job.stride[d] * static_cast<int64_t>(sizeof(T)) % piece == 0 &&
+              job.grad_stride[d] * static_cast<int64_t>(sizeof(T)) % piece == 0;
+    }
     // offsets from a wave's first lane stay below 2 * U * P * T elements
-    const bool buf = 2 * static_cast<int64_t>(job.U) * job.P * job.T * static_cast<int64_t>(sizeof(T)) + 256 <=
-                     0x7fffffff;
-#define RAMNET_ADDR_BWD(KM)                                                                          \
-    do {                                                                                             \
-        if (job.P == 16 && buf)                                                                      \
-            hipLaunchKernelGGL((topk_addr_backward_kernel<T, KM, 16, true>), grid, blk, 0, stream, job); \
-        else if (job.P == 32 && buf)                                                                 \
-            hipLaunchKernelGGL((topk_addr_backward_kernel<T, KM, 32, true>), grid, blk, 0, stream, job); \
-        else if (job.P == 16)                                                                        \
-            hipLaunchKernelGGL((topk_addr_backward_kernel<T, KM, 16>), grid, blk, 0, stream, job);   \
-        else if (job.P <= 32)                                                                        \
-            hipLaunchKernelGGL((topk_addr_backward_kernel<T, KM, 32>), grid, blk, 0, stream, job);   \
-        else                                                                                         \
-            hipLaunchKernelGGL((topk_addr_backward_kernel<T, KM, 0>), grid, blk, 0, stream, job);    \
+    buf = buf && 2 * up * job.T * static_cast<int64_t>(sizeof(T)) + 256 <= 0x7fffffff;
+#define RAMNET_ADDR_BWD_AT(KM, PR, LAY) \
+    hipLaunchKernelGGL((topk_addr_backward_kernel<T, KM, PR, LAY>), grid, blk, 0, stream, job)
+#define RAMNET_ADDR_BWD(KM)                             \
+    do {                                                \
+        if (row && job.P == 16)                         \
+            RAMNET_ADDR_BWD_AT(KM, 16, kLaneRow);       \
+        else if (row && job.P == 32)                    \
+            RAMNET_ADDR_BWD_AT(KM, 32, kLaneRow);       \
+        else if (row && job.P < 16)                     \
+            RAMNET_ADDR_BWD_AT(KM, 16, kLaneRowPart);   \
+        else if (row && job.P < 32)                     \
+            RAMNET_ADDR_BWD_AT(KM, 32, kLaneRowPart);   \
+        else if (job.P == 16 && buf)                    \
+            RAMNET_ADDR_BWD_AT(KM, 16, kLaneBuffer);    \
+        else if (job.P == 32 && buf)                    \
+            RAMNET_ADDR_BWD_AT(KM, 32, kLaneBuffer);    \
+        else if (job.P == 16)                           \
+            RAMNET_ADDR_BWD_AT(KM, 16, kLaneAny);       \
+        else if (job.P <= 32)                           \
+            RAMNET_ADDR_BWD_AT(KM, 32, kLaneAny);       \
+        else                                            \
+            RAMNET_ADDR_BWD_AT(KM, 0, kLaneAny);        \
     } while (0)
     if (job.K <= 8)
         RAMNET_ADDR_BWD(8);
@@ -653,6 +719,7 @@ hipError_t launch_backward_typed(const AddrBwdJob &job, hipStream_t stream) {
     else
         RAMNET_ADDR_BWD(0);
 #undef RAMNET_ADDR_BWD
+#undef RAMNET_ADDR_BWD_AT
     return hipGetLastError();
 }
 

@@ -84,6 +84,17 @@ SIGNATURES: dict[str, tuple[type, list]] = {
     "ramnet_topk_addr_single_forward_strided": (_c_int, [
         _c_ptr, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr,
         _c_i64, _c_float, _c_int, _c_int, _c_i64s, _c_ptr, _c_ptr, _c_ptr]),
+    "ramnet_topk_addr_backward_strided": (_c_int, [
+        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+        _c_ptr, _c_i64, _c_i64, _c_float, _c_float, _c_i64s, _c_ptr, _c_ptr, _c_ptr]),
+    "ramnet_topk_segment_forward_save_strided": (_c_int, [
+        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_float, _c_ptr, _c_i64, _c_ptr, _c_i64,
+        _c_i64s, _c_ptr]),
+    "ramnet_topk_segment_backward_saved_strided": (_c_int, [
+        _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+        _c_int, _c_float, _c_ptr, _c_i64, _c_i64s, _c_int, _c_ptr, _c_i64, _c_ptr]),
     "ramnet_topk_autoregressive_strided_": (_c_int, [
         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_float, _c_float,

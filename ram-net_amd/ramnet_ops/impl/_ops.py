@@ -113,6 +113,13 @@ def _rows_like(x: Tensor) -> Tensor:
     return y if y.stride(-1) == 1 else x.new_empty(x.shape)
 
 
+def _logits_like(t: Tensor, dtype: torch.dtype) -> Tensor:
+    """An uninitialised gradient for logits t, in t's order of dimensions."""
+    g = torch.empty_like(t, dtype=dtype)
+    _, _, U, P, _ = g.shape
+    return g if U == 1 or g.stride(2) == P * g.stride(3) else t.new_empty(t.shape, dtype=dtype)
+
+
 def _position_words(t: Tensor) -> tuple[Tensor, tuple[int, ...]]:
     """Positions and their strides in int32 words: an int64 position is read
     through its low word, which is what a cast to int32 keeps."""
@@ -230,24 +237,23 @@ def topk_addr_backward(idx: Tensor, val: Tensor, w_addr: Tensor, r_addr: Tensor,
     ev = (B, H, w_top_k + r_top_k, T)
     _check_shapes(op, idx=(idx, ev), val=(val, ev), D_val=(D_val, ev), w_addr=(w_addr, (B, H, U, P, T)),
                   r_addr=(r_addr, (B, H, U, P, T)), position_ids=(position_ids, (B, T)))
-    w_addr, r_addr = w_addr.to(dtype).contiguous(), r_addr.to(dtype).contiguous()
-    pos = position_ids.to(device=w_addr.device, dtype=torch.int32).contiguous()
-    gw = torch.empty((B, H, U, P, T), dtype=dtype, device=w_addr.device)
-    gr = torch.empty_like(gw)
+    gw, gr = _logits_like(w_addr, dtype), _logits_like(r_addr, dtype)
+    w_addr, r_addr = _logits(w_addr.to(dtype)), _logits(r_addr.to(dtype))
+    pos, pos_s = _position_words(position_ids.to(device=w_addr.device))
+    at = nat.strides(*w_addr.stride(), *r_addr.stride(), *gw.stride(), *gr.stride(), *pos_s)
     with nat.on_device(w_addr):
-        nat.call("ramnet_topk_addr_backward", idx.to(torch.int32).contiguous().data_ptr(),
+        nat.call("ramnet_topk_addr_backward_strided", idx.to(torch.int32).contiguous().data_ptr(),
                  val.to(torch.float32).contiguous().data_ptr(), w_addr.data_ptr(), r_addr.data_ptr(),
                  D_val.to(torch.float32).contiguous().data_ptr(), _code(w_addr), B, H, U, P, T, embed_num, A,
-                 pos.data_ptr(), w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), gw.data_ptr(), gr.data_ptr(),
-                 nat.stream_of(w_addr))
+                 pos.data_ptr(), w_top_k, r_top_k, float(w_re_norm), float(r_re_norm), at, gw.data_ptr(),
+                 gr.data_ptr(), nat.stream_of(w_addr))
     return gw, gr
 
 
 @topk_addr_backward.register_fake
 def _(idx, val, w_addr, r_addr, D_val, embed_num, position_ids, w_top_k, r_top_k, w_re_norm, r_re_norm, shape,
       dtype):
-    B, H, U, P, _, T = shape
-    return val.new_empty((B, H, U, P, T), dtype=dtype), val.new_empty((B, H, U, P, T), dtype=dtype)
+    return _logits_like(w_addr, dtype), _logits_like(r_addr, dtype)
 
 
 def _single_setup(ctx, inputs, output):
@@ -470,7 +476,11 @@ def topk_segment_forward_saved(addr_idx: Tensor, addr_val: Tensor, x: Tensor, ga
     op = "topk_segment_forward_saved"
     _require_gpu(op, addr_idx, addr_val, x, gamma, init_slot, init_mass, mask)
     B, H, T, C, A = _check_segment(op, addr_idx, addr_val, x, gamma, init_slot, init_mass, mask, w_top_k, r_top_k)
-    x, gamma, mask = _segment_args(x, gamma, mask)
+    y = _rows_like(x)
+    x = _rows(x)
+    gamma = gamma.to(dtype=x.dtype).contiguous()
+    if mask is not None:
+        mask = mask.to(device=x.device, dtype=torch.bool).contiguous()
     nbytes = _saved_bytes(op, B, H, T, A, C, w_top_k, r_top_k, x.dtype)
     addr_idx = addr_idx.to(torch.int32).contiguous()
     addr_val = addr_val.to(torch.float32).contiguous()
@@ -478,14 +488,14 @@ def topk_segment_forward_saved(addr_idx: Tensor, addr_val: Tensor, x: Tensor, ga
     init_mass = init_mass.to(torch.float32).contiguous()
     slot = torch.empty_like(init_slot)
     mass = torch.empty_like(init_mass)
-    y = torch.empty_like(x)
     ws = _workspace(x, B, H, T, A, C, w_top_k, r_top_k)
     saved = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     with nat.on_device(x):
-        nat.call("ramnet_topk_segment_forward_save", addr_idx.data_ptr(), addr_val.data_ptr(), x.data_ptr(),
+        nat.call("ramnet_topk_segment_forward_save_strided", addr_idx.data_ptr(), addr_val.data_ptr(), x.data_ptr(),
                  gamma.data_ptr(), _code(x), nat.ptr(mask), init_slot.data_ptr(), init_mass.data_ptr(),
                  slot.data_ptr(), mass.data_ptr(), y.data_ptr(), B, H, T, A, C, w_top_k, r_top_k, int(mass_aware),
-                 float(eps), ws.data_ptr(), ws.numel(), saved.data_ptr(), saved.numel(), nat.stream_of(x))
+                 float(eps), ws.data_ptr(), ws.numel(), saved.data_ptr(), saved.numel(),
+                 nat.strides(*x.stride()[:3], *y.stride()[:3]), nat.stream_of(x))
     return y, slot, mass, saved
 
 
@@ -494,17 +504,18 @@ def _(addr_idx, addr_val, x, gamma, init_slot, init_mass, mask, w_top_k, r_top_k
     B, H, T, C = x.shape
     A = init_slot.shape[2]
     nbytes = _saved_bytes("topk_segment_forward_saved", B, H, T, A, C, w_top_k, r_top_k, x.dtype)
-    return (x.new_empty(x.shape), init_slot.new_empty(init_slot.shape, dtype=torch.float32),
+    return (_rows_like(x), init_slot.new_empty(init_slot.shape, dtype=torch.float32),
             init_mass.new_empty(init_mass.shape, dtype=torch.float32), x.new_empty((nbytes,), dtype=torch.uint8))
 
 
 @torch.library.custom_op(f"{_NS}::topk_segment_backward_saved", mutates_args=(), device_types="cuda")
 def topk_segment_backward_saved(addr_val: Tensor, x: Tensor, gamma: Tensor, init_slot: Tensor, init_mass: Tensor,
                                 saved: Tensor, D_y: Tensor, D_post_slot: Tensor | None, D_post_mass: Tensor | None,
-                                w_top_k: int, r_top_k: int, mass_aware: bool,
-                                eps: float) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+                                w_top_k: int, r_top_k: int, mass_aware: bool, eps: float,
+                                typed_x: bool = False) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """Gradients of ``topk_segment_forward_saved`` from its ``saved`` rows;
-    outputs as ``topk_segment_backward``."""
+    outputs as ``topk_segment_backward``. With ``typed_x`` D_x comes in x's
+    dtype and order of dimensions."""
     op = "topk_segment_backward_saved"
     _require_given(op, addr_val=addr_val, x=x, gamma=gamma, init_slot=init_slot, init_mass=init_mass, saved=saved,
                    D_y=D_y)
@@ -515,41 +526,42 @@ def topk_segment_backward_saved(addr_val: Tensor, x: Tensor, gamma: Tensor, init
     _check_shapes(op, addr_val=(addr_val, (B, H, K, T)), gamma=(gamma, (B, H, T)), init_slot=(init_slot, (B, H, A, C)),
                   init_mass=(init_mass, (B, H, A)), D_y=(D_y, (B, H, T, C)), D_post_slot=(D_post_slot, (B, H, A, C)),
                   D_post_mass=(D_post_mass, (B, H, A)))
-    x, gamma, _ = _segment_args(x, gamma, None)
+    gamma = gamma.to(dtype=x.dtype).contiguous()
     nbytes = _saved_bytes(op, B, H, T, A, C, w_top_k, r_top_k, x.dtype)
     if saved.dtype != torch.uint8 or saved.numel() < nbytes or not saved.is_contiguous():
         raise RuntimeError(f"{op}: saved must be the contiguous uint8 tensor of topk_segment_forward_saved")
     addr_val = addr_val.to(torch.float32).contiguous()
     init_slot = init_slot.to(torch.float32).contiguous()
     init_mass = init_mass.to(torch.float32).contiguous()
-    D_y = D_y.to(dtype=x.dtype).contiguous()
+    D_y = _rows(D_y.to(dtype=x.dtype))
     if D_post_slot is not None:
         D_post_slot = D_post_slot.to(torch.float32).contiguous()
     if D_post_mass is not None:
         D_post_mass = D_post_mass.to(torch.float32).contiguous()
     f32 = dict(dtype=torch.float32, device=x.device)
     D_addr = torch.empty((B, H, K, T), **f32)
-    D_x = torch.empty((B, H, T, C), **f32)
+    D_x = _rows_like(x) if typed_x else torch.empty((B, H, T, C), **f32)
     D_gamma = torch.empty((B, H, T), **f32)
     D_slot = torch.empty_like(init_slot)
     D_mass = torch.empty_like(init_mass)
     ws = torch.empty(max(1, nat.segment_backward_saved_workspace_bytes(B, H, T, A, C, w_top_k, r_top_k)),
                      dtype=torch.uint8, device=x.device)
     with nat.on_device(x):
-        nat.call("ramnet_topk_segment_backward_saved", addr_val.data_ptr(), x.data_ptr(), gamma.data_ptr(), _code(x),
+        nat.call("ramnet_topk_segment_backward_saved_strided", addr_val.data_ptr(), x.data_ptr(), gamma.data_ptr(), _code(x),
                  init_slot.data_ptr(), init_mass.data_ptr(), D_y.data_ptr(), nat.ptr(D_post_slot),
                  nat.ptr(D_post_mass), D_addr.data_ptr(), D_x.data_ptr(), D_gamma.data_ptr(), D_slot.data_ptr(),
                  D_mass.data_ptr(), B, H, T, A, C, w_top_k, r_top_k, int(mass_aware), float(eps), saved.data_ptr(),
-                 saved.numel(), ws.data_ptr(), ws.numel(), nat.stream_of(x))
+                 saved.numel(), nat.strides(*D_y.stride()[:3], *D_x.stride()[:3]), int(typed_x), ws.data_ptr(), ws.numel(), nat.stream_of(x))
     return D_addr, D_x, D_gamma, D_slot, D_mass
 
 
 @topk_segment_backward_saved.register_fake
 def _(addr_val, x, gamma, init_slot, init_mass, saved, D_y, D_post_slot, D_post_mass, w_top_k, r_top_k, mass_aware,
-      eps):
+      eps, typed_x=False):
     B, H, T, C = x.shape
     f32 = torch.float32
-    return (x.new_empty((B, H, w_top_k + r_top_k, T), dtype=f32), x.new_empty(x.shape, dtype=f32),
+    return (x.new_empty((B, H, w_top_k + r_top_k, T), dtype=f32),
+            _rows_like(x) if typed_x else x.new_empty(x.shape, dtype=f32),
             x.new_empty((B, H, T), dtype=f32), init_slot.new_empty(init_slot.shape, dtype=f32),
             init_mass.new_empty(init_mass.shape, dtype=f32))
 
@@ -569,7 +581,8 @@ def _segment_saved_backward(ctx, D_y, D_slot, D_mass, D_saved):
     if D_y is None:
         D_y = torch.zeros_like(x)
     D_addr, D_x, D_gamma, D_s, D_m = topk_segment_backward_saved(addr_val, x, gamma, init_slot, init_mass, saved, D_y,
-                                                                 D_slot, D_mass, w_top_k, r_top_k, mass_aware, eps)
+                                                                 D_slot, D_mass, w_top_k, r_top_k, mass_aware, eps,
+                                                                 typed_x=True)
     need = ctx.needs_input_grad
     return (None,
             D_addr if need[1] else None,

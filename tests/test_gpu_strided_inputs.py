@@ -142,6 +142,42 @@ def test_decode_positions(P, Kw):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("order", list(ORDERS))
+@pytest.mark.parametrize("case", [c for c in CASES if c[4] > 1], ids=lambda c: "-".join(str(v).replace("torch.", "") for v in c))
+def test_strided_gradients(case, order):
+    """Gradients of logits and values in the inputs' layouts: bit for bit those
+    of contiguous inputs, fp32 sums rounded once to the inputs' type."""
+    B, H, U, P, T, C, Kw, Kr, dtype = case
+    d = _inputs(B, H, U, P, T, C, dtype, seed=1)
+    lay, ops = ORDERS[order], torch.ops.ramnet_ops
+    A = P ** U
+    pos = torch.arange(T, device=DEV).view(1, T) * 3 + torch.arange(B, device=DEV).view(B, 1) * 7 - 5
+    logits = lambda t: t.permute(0, 1, 3, 4, 2)
+    w, r = logits(d["w"]).contiguous(), logits(d["r"]).contiguous()
+    idx, val = ops.topk_addr_forward(w, r, H // 2, A, pos, Kw, Kr, 0.5, 0.25)
+    dval = torch.randn(val.shape, generator=torch.Generator(device=DEV).manual_seed(2), device=DEV)
+    tail = (dval, H // 2, pos, Kw, Kr, 0.5, 0.25, [B, H, U, P, A, T], dtype)
+    want = ops.topk_addr_backward(idx, val, w, r, *tail)
+    got = ops.topk_addr_backward(idx, val, logits(lay(d["w"])), logits(_store(d["r"], (0, 2, 1))), *tail)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    if nat.segment_saved_bytes(B, H, T, A, C, Kw, Kr, dtype) < 0:
+        return
+    seg = (d["gamma"], d["slot"], d["mass"])
+    y, slot, mass, saved = ops.topk_segment_forward_saved(idx, val, d["x"], *seg, d["mask"], Kw, Kr, True, 1e-6)
+    dy = torch.randn(y.shape, generator=torch.Generator(device=DEV).manual_seed(3), device=DEV).to(dtype)
+    want = ops.topk_segment_backward_saved(val, d["x"], *seg, saved, dy, None, None, Kw, Kr, True, 1e-6)
+    x = lay(d["x"])
+    y2, slot2, mass2, saved2 = ops.topk_segment_forward_saved(idx, val, x, *seg, d["mask"], Kw, Kr, True, 1e-6)
+    for a, b in zip((y2, slot2, mass2), (y, slot, mass)):
+        assert torch.equal(a, b)
+    for typed in (False, True):
+        got = ops.topk_segment_backward_saved(val, x, *seg, saved2, lay(dy), None, None, Kw, Kr, True, 1e-6, typed)
+        assert got[1].dtype == (dtype if typed else torch.float32)
+        for k, (a, b) in enumerate(zip(got, want)):
+            assert torch.equal(a, b.to(a.dtype)), k
+
+
 def test_refused_strides():
     """Steps the kernels cannot follow are refused by the native entry."""
     z = torch.zeros(64, device=DEV)
