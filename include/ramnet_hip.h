@@ -356,6 +356,16 @@ int ramnet_topk_autoregressive_steps_strided_(const void *w_addr, const void *r_
                                               float eps, const int64_t *strides, void *y, void *stream);
 
 /*
+ * Read-out of a layer: sigmoid(gate) * RMSNorm(y) per row of C elements
+ * (reference: ram_attn_block.py:326-334), computed in fp32 and rounded once.
+ *   y, gate, out    (rows, C) `dtype`;  weight (C) `dtype`
+ * A row takes at most 64 pieces: of 16 bytes where C is a multiple of them
+ * and every pointer is 16-byte aligned, else of one element.
+ */
+int ramnet_readout(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C, float eps,
+                   void *out, void *stream);
+
+/*
  * One fused decode step on a persistent state, updated in place.
  * Replaces ramnet_ops::topk_autoregressive_ (ram_attn_bind.cpp:92-101,
  * ram_attn_ops.cpp:349-394).

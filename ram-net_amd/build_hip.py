@@ -29,7 +29,7 @@ PROBE_SOURCE = "lds_probe.hip"
 
 SOURCES = ("topk_addr.hip", "segment_forward.hip", "segment_scan_f32.hip", "segment_scan_f16.hip",
            "segment_scan_bf16.hip", "segment_level_f32.hip", "segment_level_f16.hip", "segment_level_bf16.hip",
-           "segment_backward.hip", "autoregressive.hip", "capi.hip")
+           "segment_backward.hip", "autoregressive.hip", "readout.hip", "capi.hip")
 ARCH = "gfx950"
 
 

@@ -1097,6 +1097,19 @@ int ramnet_topk_autoregressive_steps_strided_(const void *w_addr, const void *r_
                           C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, pos, true, y, stream);
 }
 
+int ramnet_readout(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C, float eps,
+                   void *out, void *stream) {
+    RAMNET_REQUIRE(rows >= 0 && C > 0 && C < kIntMax, "readout shape must have rows >= 0 and C > 0");
+    RAMNET_REQUIRE(valid_dtype(dtype), "readout dtype must be float32, float16 or bfloat16");
+    if (rows == 0)
+        return RAMNET_OK;
+    RAMNET_REQUIRE(y && gate && weight && out, "null tensor pointer");
+    const ramnet::ReadoutJob job{y, gate, weight, out, dtype, rows, static_cast<int>(C), eps};
+    const char *why = nullptr;
+    const hipError_t err = ramnet::launch_readout(job, static_cast<hipStream_t>(stream), &why);
+    return finish(err, why, "readout launch");
+}
+
 // The query has no token count: it answers for a call of kPlanQueryTokens
 // tokens (the form can differ for much shorter calls, where the mass-wave
 // form's saving of the pre-pass launches decides).

@@ -250,6 +250,18 @@ struct PackJob {
     int B, H, T, A, Kw, Kr;
 };
 hipError_t launch_pack_records(const PackJob &job, hipStream_t stream, const char **why);
+
+// Normalised and gated read-out of a layer: rows of C elements in `dtype`.
+struct ReadoutJob {
+    const void *y, *gate;     // (rows, C)
+    const void *weight;       // (C)
+    void *out;                // (rows, C)
+    int dtype;
+    int64_t rows;
+    int C;
+    float eps;
+};
+hipError_t launch_readout(const ReadoutJob &job, hipStream_t stream, const char **why);
 hipError_t launch_autoregressive(const DecodeJob &job, hipStream_t stream, const char **why);
 // S consecutive decode steps; the inputs, y, position_ids and mask of a
 // DecodeJob carry a leading step dimension (S, ...).

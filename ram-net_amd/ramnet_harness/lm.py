@@ -31,6 +31,7 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from ramnet_ops import random_access_memory_attention
 
@@ -56,6 +57,14 @@ class HarnessConfig:
     @property
     def slots(self) -> int:
         return self.addr_radix ** self.addr_order
+
+
+def has_hooks(module: nn.Module) -> bool:
+    """Whether calling the module would run more than its forward."""
+    return any(getattr(module, n) for n in ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks",
+                                            "_backward_pre_hooks")) \
+        or any(getattr(nn.modules.module, n) for n in ("_global_forward_hooks", "_global_forward_pre_hooks",
+                                                       "_global_backward_hooks", "_global_backward_pre_hooks"))
 
 
 class RamLayer(nn.Module):
@@ -114,8 +123,25 @@ class RamLayer(nn.Module):
             top_k=self.cfg.top_k, eps=self.cfg.ram_eps, t_dim=1, inplace=inplace, impl_backend="cuda")
         if capture is not None:
             capture[-1]["y"] = y
+        gate = self.gate(x)
+        if self._fused_readout(y, gate):
+            return self.out(torch.ops.ramnet_ops.readout(y, gate, self.out_norm.weight, self.out_norm.eps)), new_state
         y = self.out_norm(y).flatten(-2)
-        return self.out(torch.sigmoid(self.gate(x)) * y), new_state
+        return self.out(torch.sigmoid(gate) * y), new_state
+
+    def _fused_readout(self, y: torch.Tensor, gate: torch.Tensor) -> bool:
+        """Whether the norm and the gate run as one kernel: eager calls that
+        want no derivative, with nothing attached to the norm. A layer call of
+        32768 tokens, 8 heads of 128 in bf16: 1022 us with torch's kernels,
+        841 with this one."""
+        norm = self.out_norm
+        if type(norm) is not nn.RMSNorm or norm.weight is None or norm.eps is None:
+            return False
+        from ramnet_ops.impl._ops import readout_fits  # (needs the built library, as y does)
+        wants_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (y, gate, norm.weight))
+        return (not wants_grad and not torch.compiler.is_compiling() and not torch.is_autocast_enabled("cuda")
+                and not has_hooks(norm)
+                and forward_ad.unpack_dual(gate).tangent is None and readout_fits(y, gate, norm.weight))
 
 
 class SwiGLU(nn.Module):

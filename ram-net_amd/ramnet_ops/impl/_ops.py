@@ -708,6 +708,43 @@ def _(w_addr, r_addr, x, gamma, slot, mass, mask, embed_num, position_ids, w_top
 
 
 # --------------------------------------------------------------------------
+# read-out of a layer
+
+def readout_fits(y: Tensor, gate: Tensor, weight: Tensor) -> bool:
+    """Whether ``readout`` takes these tensors: contiguous, one GPU dtype, and
+    a row of at most 64 pieces of 16 bytes."""
+    C = y.shape[-1]
+    return (y.is_cuda and y.dtype in nat.DTYPE_CODES and y.dtype == gate.dtype == weight.dtype
+            and y.device == gate.device == weight.device and y.is_contiguous() and gate.is_contiguous()
+            and weight.is_contiguous() and weight.shape == (C,) and gate.numel() == y.numel()
+            and C * y.element_size() % 16 == 0 and C * y.element_size() <= 64 * 16
+            and not any(t.data_ptr() % 16 for t in (y, gate, weight)))
+
+
+@torch.library.custom_op(f"{_NS}::readout", mutates_args=(), device_types="cuda")
+def readout(y: Tensor, gate: Tensor, weight: Tensor, eps: float) -> Tensor:
+    """``sigmoid(gate) * rms_norm(y, weight, eps)`` over y's last dimension, in
+    the shape of gate (no gradient)."""
+    op = "readout"
+    _require_gpu(op, y, gate, weight)
+    C = y.shape[-1]
+    _check_shapes(op, weight=(weight, (C,)))
+    if gate.numel() != y.numel() or not y.dtype == gate.dtype == weight.dtype:
+        raise RuntimeError(f"{op}: y, gate and weight must share dtype, y and gate their number of elements")
+    y, gate, weight = y.contiguous(), gate.contiguous(), weight.contiguous()
+    out = torch.empty_like(gate, memory_format=torch.contiguous_format)
+    with nat.on_device(y):
+        nat.call("ramnet_readout", y.data_ptr(), gate.data_ptr(), weight.data_ptr(), _code(y), y.numel() // C, C,
+                 float(eps), out.data_ptr(), nat.stream_of(y))
+    return out
+
+
+@readout.register_fake
+def _(y, gate, weight, eps):
+    return torch.empty_like(gate, memory_format=torch.contiguous_format)
+
+
+# --------------------------------------------------------------------------
 # fused decode step
 
 @torch.library.custom_op(f"{_NS}::topk_autoregressive_", mutates_args=("slot", "mass"), device_types="cuda")
