@@ -13,7 +13,7 @@ of ``topk_autoregressive_steps_``) under ``decode.multi_step``. Timings give
 the median, min and max over repetitions. Config 1 (fp32, one fused forward
 call) is reported under ``config1``.
 
-``roofline`` is for the dominant stage (the segment stage: mass pre-pass and
+``roofline`` is for the dominant stage (the segment stage: event schedule and
 segment scan, one C-ABI call), timed with HIP events on the stream it runs
 on: ``achieved`` / ``frac`` are its counter-measured HBM bytes per call
 (rocprofv3, ``--traffic-summary``) over that time against the HBM peak;
@@ -67,9 +67,9 @@ HBM_PEAK_GBS = 8000.0
 # built from other sources reports it as stale.
 TRAFFIC_FILE = os.path.join(REPO, "profiles", "segment_stage_traffic.json")
 TRAFFIC_SOURCES = ("segment_scan.hpp", "segment_scan_pair.hpp", "segment_forward.hip", "segment_scan_bf16.hip",
-                   "ramnet_kernels.hpp", "ramnet_device.hpp", "topk_addr.hip", "lane_search.hpp", "capi.hip")
-# the scan kernels of the segment stage (one-token, paired, slot-range forms)
-SCAN_KERNELS = ("segment_scan_kernel", "segment_scan_pair_kernel", "segment_scan_range_kernel")
+                   "segment_level.hpp", "segment_level_bf16.hip", "ramnet_kernels.hpp", "ramnet_device.hpp", "topk_addr.hip", "lane_search.hpp", "capi.hip")
+# the scan kernels of the segment stage (one-token, paired, slot-range, level forms)
+SCAN_KERNELS = ("segment_scan_kernel", "segment_scan_pair_kernel", "segment_scan_range_kernel", "segment_level_kernel")
 PROBE_LIB = os.path.join(REPO, "ram-net_amd", "ramnet_ops", "_lib", "libramnet_lds_probe.so")
 METRIC = "prefill tokens/s (T=4096) + decode tokens/s (B=64); % HBM roofline"
 
@@ -148,7 +148,7 @@ def traffic_summary(out_dir: str) -> int:
     --copy-probe 1024``. FETCH_SIZE and WRITE_SIZE (KiB per dispatch,
     medians) are scaled by what they read for the 1 GiB copy."""
     import statistics
-    stage_names = SCAN_KERNELS + ("segment_mass_kernel", "mass_chunk_map_kernel", "mass_chunk_scan_kernel")
+    stage_names = SCAN_KERNELS + ("segment_schedule_kernel", "segment_mass_kernel", "mass_chunk_map_kernel", "mass_chunk_scan_kernel")
 
     def counters(path):
         vals = {}
@@ -839,18 +839,19 @@ def main(argv=None) -> int:
                 "segment_length": 128,
             },
             "roofline": {
-                # The dominant stage is the segment stage (one C-ABI call: the
-                # mass pre-pass kernels, then segment_scan_kernel), timed live
+                # The dominant stage is the segment stage (one C-ABI call:
+                # segment_schedule_kernel, then segment_level_kernel, beside
+                # the launches of the crowded form, which exit), timed live
                 # with HIP events. achieved / frac: its HBM bytes per call as
                 # rocprofv3's FETCH_SIZE / WRITE_SIZE count them (calibrated on
                 # a copy), over that time, against the HBM peak. It does not
                 # bind: the slot state stays in LDS for the whole call, and
-                # the scan is bound by its per-token LDS round trips ("lds"
+                # the scan is bound by its LDS and vector instructions ("lds"
                 # below: the slot rows it moves through LDS against the LDS
                 # read peak measured in this run).
                 "bound": "lds",
                 "peak_resource": "hbm",
-                "kernel": "segment stage: mass pre-pass + segment_scan_kernel",
+                "kernel": "segment stage: segment_schedule_kernel + segment_level_kernel",
                 "achieved": hbm_gbs,
                 "peak": HBM_PEAK_GBS,
                 "unit": "GB/s",
