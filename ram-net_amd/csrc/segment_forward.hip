@@ -270,8 +270,8 @@ bool level_layout(int A, int T, int vec, int nw, int kmax, bool mass_aware, Plan
 // 8 heads, T = 2048, A = 1024, K = 8, one workgroup of one wave per CU: 88,
 // 87 and 107 us with 1, 2 and 4 channels per lane; 128 heads, T = 4096: 471
 // us with (4 channels, 4 waves), 609 with (2, 4); 32 heads, T = 8192, A =
-// 4096, K = 16: 936 us with (2, 2), 959 with (1, 4), 1733 with (2, 1), and
-// 3.8 ms with (4, 1), whose 16 events spill registers.
+// 4096, K = 16: 907 us with (1, 4), 932 with (2, 2), 1580 with (1, 2), 1733
+// with (2, 1), and 3.8 ms with (4, 1), whose 16 events spill registers.
 bool plan_level(int B, int H, int A, int C, int kmax, int n_cu, int T, bool mass_aware, Plan *out) {
     bool found = false;
     double best = 0;
