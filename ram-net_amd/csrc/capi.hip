@@ -502,6 +502,14 @@ static hipError_t pack_decoded(const ramnet::SegmentJob &job, const int32_t *add
     return ramnet::launch_pack_records(pack, s, why);
 }
 
+// A workspace that holds no read sums offers none to the launch, which then
+// refuses a scan in slot ranges instead of writing past its end.
+static void fit_workspace(ramnet::SegmentJob &job, int64_t workspace_bytes) {
+    const int64_t records = scan_workspace_bytes(job.B, job.H, job.T, job.Kw, job.Kr);
+    if (job.dtype != RAMNET_F32 && workspace_bytes < records + static_cast<int64_t>(job.B) * job.H * job.T * job.C * 4)
+        job.yacc = nullptr;
+}
+
 static int segment_from_decoded(const int32_t *addr_idx, const float *addr_val, const void *x, const void *gamma,
                                 int dtype, const uint8_t *mask, const float *init_slot, const float *init_mass,
                                 float *slot_out, float *mass_out, void *y, int64_t B, int64_t H, int64_t T, int64_t A,
@@ -515,6 +523,7 @@ static int segment_from_decoded(const int32_t *addr_idx, const float *addr_val, 
     RAMNET_REQUIRE(T == 0 || (addr_idx && addr_val), "null tensor pointer");
     ramnet::SegmentJob job = make_segment_job(x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C,
                                               w_top_k, r_top_k, mass_aware, eps, workspace);
+    fit_workspace(job, workspace_bytes);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const char *why = nullptr;
     if (T > 0) {
@@ -637,6 +646,7 @@ static int segment_scan(const void *x, int dtype, const float *init_slot, const 
         return RAMNET_OK;
     ramnet::SegmentJob job = make_segment_job(x, dtype, init_slot, init_mass, slot_out, mass_out, y, B, H, T, A, C,
                                               w_top_k, r_top_k, mass_aware, eps, workspace);
+    fit_workspace(job, workspace_bytes);
     RAMNET_REQUIRE(T == 0 || (stride_ok(at.x, {B, H, T}) && stride_dense(at.y, B, H, T, C)),
                    "x strides must be >= 0 and within int32, y's rows must fill B * H * T * C elements");
     std::copy_n(at.x, 3, job.x_stride);
@@ -1123,6 +1133,16 @@ int ramnet_segment_plan(int64_t B, int64_t H, int64_t A, int64_t C, int64_t w_to
     return ramnet::segment_plan(static_cast<int>(B), static_cast<int>(H), kPlanQueryTokens, static_cast<int>(A),
                                 static_cast<int>(C), static_cast<int>(w_top_k), static_cast<int>(r_top_k), dtype,
                                 slice_channels, lds_bytes, precomputed_gains);
+}
+
+int ramnet_segment_call_form(int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
+                             int dtype, int mass_aware, int *slot_ranges) {
+    if (B <= 0 || H <= 0 || T <= 0 || A <= 0 || A >= kAddressLimit || C <= 0 || w_top_k <= 0 || r_top_k <= 0 ||
+        !valid_dtype(dtype) || !fits_int({B * H * A * C, B * H * (A + 2), B * H * T * C}))
+        return -1;
+    return ramnet::segment_call_form(static_cast<int>(B), static_cast<int>(H), static_cast<int>(T), static_cast<int>(A),
+                                     static_cast<int>(C), static_cast<int>(w_top_k), static_cast<int>(r_top_k), dtype,
+                                     mass_aware ? 1 : 0, slot_ranges);
 }
 
 // ---- prefill forward without a workspace argument

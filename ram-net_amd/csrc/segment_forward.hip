@@ -1489,8 +1489,7 @@ static bool pick_plan(const SegmentJob &job, Plan *p, const char **why) {
     return true;
 }
 
-int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int *cs, int *lds_bytes, int *pre,
-                 int *ranges) {
+static SegmentJob plan_job(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int mass_aware) {
     SegmentJob job{};
     job.B = B;
     job.H = H;
@@ -1500,9 +1499,19 @@ int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, i
     job.Kw = Kw;
     job.Kr = Kr;
     job.dtype = dtype;
-    Plan p{};
+    job.mass_aware = mass_aware;
+    return job;
+}
+
+// The mass-aware level-scheduled form holds more LDS, so near the LDS limit
+// the two kinds of call can differ in form. The layout is that of a call
+// that is not mass-aware; `ranges` is the larger of the two, as the workspace
+// that it sizes serves both.
+int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int *cs, int *lds_bytes, int *pre,
+                 int *ranges) {
+    Plan p{}, q{};
     const char *why = nullptr;
-    if (!pick_plan(job, &p, &why))
+    if (!pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 0), &p, &why))
         return 0;
     if (cs)
         *cs = p.cs;
@@ -1511,8 +1520,18 @@ int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, i
     if (pre)
         *pre = p.pre ? 1 : 0;
     if (ranges)
-        *ranges = p.nr;
+        *ranges = pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 1), &q, &why) ? std::max(p.nr, q.nr) : p.nr;
     return 1;
+}
+
+int segment_call_form(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int mass_aware, int *ranges) {
+    Plan p{};
+    const char *why = nullptr;
+    if (!pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, mass_aware), &p, &why))
+        return -1;
+    if (ranges)
+        *ranges = p.nr;
+    return p.tp == kLevelPlan ? kFormLevel : p.tp == 2 ? kFormPaired : p.pre ? kFormGains : kFormMassWave;
 }
 
 bool segment_forward_can_save(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, const SavedRows &geo) {

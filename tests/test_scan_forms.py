@@ -1,0 +1,25 @@
+"""The segment forward's choice of form near the edges of LDS, without a GPU
+(``ramnet_segment_call_form`` and the size queries do no device work)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from ramnet_ops import _native as nat
+
+B, H, C = 4, 8, 64
+# around the widest slot spaces of the forms that hold them whole: 20**3 .. 23**3, 104**2 .. 116**2, and between
+SLOTS = sorted({20 ** 3, 21 ** 3, 22 ** 3, 23 ** 3, *(p * p for p in range(86, 117, 3)), *range(7600, 14000, 173)})
+
+
+@pytest.mark.parametrize("T", [9, 48, 64, 65, 128, 2048, 8192])
+@pytest.mark.parametrize("K", [4, 8, 16])
+def test_workspace_holds_every_call(K, T):
+    """The workspace size, which does not depend on mass_aware, holds the fp32
+    read sums of a call scanned in slot ranges, mass-aware or not."""
+    for A in SLOTS:
+        ws = nat.segment_workspace_bytes(B, H, T, A, C, K, K, torch.bfloat16)
+        for mass_aware in (False, True):
+            form, ranges = nat.segment_call_form(B, H, T, A, C, K, K, torch.bfloat16, mass_aware)
+            sums = B * H * T * C * 4 if ranges > 1 else 0
+            assert ws >= nat.scan_workspace_bytes(B, H, T, K, K) + sums, (A, mass_aware, form, ranges)
