@@ -450,11 +450,13 @@ int ramnet_segment_plan(int64_t B, int64_t H, int64_t A, int64_t C, int64_t w_to
  * The form that a segment forward of exactly these sizes takes (-1: not
  * supported): 0 one token a step with a mass wave, 1 one token a step with
  * precomputed gains, 2 two tokens a step, 3 level-scheduled chunks of 32
- * tokens. *slot_ranges (may be null): the ranges its slot space is scanned
- * in. Honours RAMNET_SCAN_LAYOUT like the launch does.
+ * tokens. *slot_ranges: the ranges its slot space is scanned in;
+ * *crowded_form: the form that takes the call where its addresses crowd a few
+ * slots, which the level-scheduled form finds out on the device (each may be
+ * null). Honours RAMNET_SCAN_LAYOUT like the launch does.
  */
 int ramnet_segment_call_form(int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
-                             int dtype, int mass_aware, int *slot_ranges);
+                             int dtype, int mass_aware, int *slot_ranges, int *crowded_form);
 
 #ifdef __cplusplus
 }

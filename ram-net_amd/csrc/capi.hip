@@ -1136,13 +1136,13 @@ int ramnet_segment_plan(int64_t B, int64_t H, int64_t A, int64_t C, int64_t w_to
 }
 
 int ramnet_segment_call_form(int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t w_top_k, int64_t r_top_k,
-                             int dtype, int mass_aware, int *slot_ranges) {
+                             int dtype, int mass_aware, int *slot_ranges, int *crowded_form) {
     if (B <= 0 || H <= 0 || T <= 0 || A <= 0 || A >= kAddressLimit || C <= 0 || w_top_k <= 0 || r_top_k <= 0 ||
         !valid_dtype(dtype) || !fits_int({B * H * A * C, B * H * (A + 2), B * H * T * C}))
         return -1;
     return ramnet::segment_call_form(static_cast<int>(B), static_cast<int>(H), static_cast<int>(T), static_cast<int>(A),
                                      static_cast<int>(C), static_cast<int>(w_top_k), static_cast<int>(r_top_k), dtype,
-                                     mass_aware ? 1 : 0, slot_ranges);
+                                     mass_aware ? 1 : 0, slot_ranges, crowded_form);
 }
 
 // ---- prefill forward without a workspace argument

@@ -275,9 +275,11 @@ hipError_t launch_autoregressive_steps(const DecodeJob &job, int S, hipStream_t 
 // current device.
 int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int *cs, int *lds_bytes, int *pre,
                  int *ranges = nullptr);
-// The form of one call (-1: not supported), and its slot ranges.
+// The form of one call (-1: not supported), its slot ranges, and the form
+// that takes it where its addresses are crowded.
 enum : int { kFormMassWave = 0, kFormGains = 1, kFormPaired = 2, kFormLevel = 3 };
-int segment_call_form(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int mass_aware, int *ranges);
+int segment_call_form(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int mass_aware, int *ranges,
+                      int *crowded);
 
 // Mass pre-pass in record-keeping mode: the records stay as they are and
 // `aux` receives the per-event quantities. `maps` holds the chunk maps

@@ -86,6 +86,7 @@ struct Plan {
                   // kLevelPlan = the level-scheduled scan (vec channels per lane)
     int km = 0;   // level-scheduled scan: padded events per token
     double us = 0;  // and its estimated time
+    bool alone = false;  // level-scheduled scan: takes crowded calls too
 };
 constexpr int kLevelPlan = 3;
 // Calls of at most this many tokens are never left to the one-token scan: its
@@ -301,6 +302,30 @@ bool plan_level(int B, int H, int A, int C, int kmax, int n_cu, int T, bool mass
     return found;
 }
 
+// The one-token layout that takes a crowded call from the level-scheduled
+// scan (estimated at `us`). Each launch that returns at once takes about 4
+// us, so the pre-pass form is for calls of kCrowdedPreUs and more, and for
+// those whose mass-wave form does not fit in LDS.
+constexpr double kCrowdedPreUs = 200;
+bool plan_crowded(int B, int H, int A, int C, int kmax, int elem, int n_cu, int T, double us, Plan *out) {
+    const SavedRows *none = nullptr;
+    int64_t cost = 0;
+    if (plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, true, us >= kCrowdedPreUs, out, &cost, none, false))
+        return true;
+    return us < kCrowdedPreUs && plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, false, true, out, &cost, none, false);
+}
+
+// Whether the planner's level-scheduled layout serves this call: alone, or
+// beside a one-token layout for crowded addresses. Slot spaces wider than
+// any of those (A > 10912) keep the scan in slot ranges.
+bool plan_level_call(int B, int H, int A, int C, int kmax, int elem, int n_cu, int T, bool mass_aware, Plan *out) {
+    Plan crowded{};
+    if (!plan_level(B, H, A, C, kmax, n_cu, T, mass_aware, out))
+        return false;
+    out->alone = T <= kLevelAlone;
+    return out->alone || plan_crowded(B, H, A, C, kmax, elem, n_cu, T, out->us, &crowded);
+}
+
 bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, int T, Plan *out,
                const SavedRows *sv = nullptr, bool mass_aware = true) {
     const int kmax = std::max(Kw, Kr);
@@ -313,8 +338,9 @@ bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, i
     // and 0.6x at 512 (T = 84), 1.5x at A = 1728 (K = 12).
     const int64_t writes = static_cast<int64_t>(kTile) * kmax;
     if (!sv && B > 0 && T > 1 && (kmax <= 8 ? 2 * writes <= 3 * static_cast<int64_t>(A) : 5 * writes <= 3 * static_cast<int64_t>(A)) &&
-        plan_level(B, H, A, C, kmax, n_cu, T, mass_aware, out))
+        plan_level_call(B, H, A, C, kmax, elem, n_cu, T, mass_aware, out))
         return true;
+    *out = Plan{};
     if (sv)  // saving rows: the precomputed-gain form over the whole slot space
         return A <= kMaxPrePassSlots && save_fits(*sv, T) &&
                plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, false, true, out, &cost, sv);
@@ -1428,7 +1454,9 @@ __global__ __launch_bounds__(256) void state_copy_kernel(float *dst, const float
 
 // RAMNET_SCAN_LAYOUT="vec,epp,np,nw[,pre[,tp]]" replaces the planner's
 // choice (tests sweep every compiled layout with it; also a tuning knob).
-// tp = 2 names a paired layout (pre = 1, np = 1; epp events per half wave).
+// tp = 2 names a paired layout (pre = 1, np = 1; epp events per half wave),
+// tp = 3 a level-scheduled one (pre = 1, np = 1, epp = 2), which then takes
+// crowded addresses too.
 // The layout must be compiled, cover max(Kw, Kr) events and fit in LDS.
 static int layout_override(const SegmentJob &job, Plan *p, const char **why) {
     const char *env = std::getenv("RAMNET_SCAN_LAYOUT");
@@ -1437,8 +1465,10 @@ static int layout_override(const SegmentJob &job, Plan *p, const char **why) {
     int vec = 0, epp = 0, np = 0, nw = 0, pre = 0, tp = 1;
     const int n = std::sscanf(env, "%d,%d,%d,%d,%d,%d", &vec, &epp, &np, &nw, &pre, &tp);
     if (n == 6 && tp == kLevelPlan && pre == 1 && np == 1 && epp == kWave / kTile &&
-        level_layout(job.A, job.T, vec, nw, std::max(job.Kw, job.Kr), job.mass_aware != 0, p))
+        level_layout(job.A, job.T, vec, nw, std::max(job.Kw, job.Kr), job.mass_aware != 0, p)) {
+        p->alone = true;
         return 1;
+    }
     const bool pair = n == 6 && tp == 2;
     const bool named = pair ? pre == 1 && np == 1 && scan_pair_layout_compiled(vec, epp, nw)
                             : (n >= 4 && n <= 6) && (pre == 0 || pre == 1) && tp == 1 &&
@@ -1524,14 +1554,24 @@ int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, i
     return 1;
 }
 
-int segment_call_form(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int mass_aware, int *ranges) {
-    Plan p{};
+static int form_of(const Plan &p) {
+    return p.tp == kLevelPlan ? kFormLevel : p.tp == 2 ? kFormPaired : p.pre ? kFormGains : kFormMassWave;
+}
+
+int segment_call_form(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int mass_aware, int *ranges,
+                      int *crowded) {
+    Plan p{}, q{};
     const char *why = nullptr;
     if (!pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, mass_aware), &p, &why))
         return -1;
     if (ranges)
         *ranges = p.nr;
-    return p.tp == kLevelPlan ? kFormLevel : p.tp == 2 ? kFormPaired : p.pre ? kFormGains : kFormMassWave;
+    if (crowded)
+        *crowded = p.tp == kLevelPlan && !p.alone &&
+                           plan_crowded(B, H, A, C, std::max(Kw, Kr), dtype_bytes(dtype), cu_count(), T, p.us, &q)
+                       ? form_of(q)
+                       : form_of(p);
+    return form_of(p);
 }
 
 bool segment_forward_can_save(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, const SavedRows &geo) {
@@ -1551,16 +1591,11 @@ static hipError_t launch_scan_layout(const SegmentJob &job, const ScanGeom &geo,
 // scan, whose waves return at once otherwise. It runs before the
 // level-scheduled scan: a pre-pass that is not needed leaves y and the final
 // masses alone, and one that is has read what it needs of the schedule
-// before the gain records replace it. Each launch that returns at once takes
-// about 4 us, so the pre-pass form is for calls of kCrowdedPreUs and more.
-constexpr double kCrowdedPreUs = 200;
+// before the gain records replace it.
 static hipError_t launch_crowded(const SegmentJob &job, double us, hipStream_t stream, const char **why) {
     Plan p{};
-    int64_t cost = 0;
     const int t_pad = scan_t_pad(job.T), n_cu = cu_count();
-    const SavedRows *none = nullptr;
-    if (!plan_layout(job.B, job.H, job.A, job.A, job.C, std::max(job.Kw, job.Kr), dtype_bytes(job.dtype), n_cu, job.T,
-                     true, us >= kCrowdedPreUs, &p, &cost, none, false)) {
+    if (!plan_crowded(job.B, job.H, job.A, job.C, std::max(job.Kw, job.Kr), dtype_bytes(job.dtype), n_cu, job.T, us, &p)) {
         *why = "segment forward: no one-token layout for a crowded call";
         return hipErrorInvalidValue;
     }
@@ -1610,7 +1645,7 @@ static hipError_t launch_level_scan(const SegmentJob &job, const Plan &p, hipStr
     geo.n_units = job.B * job.H * geo.n_slices;
     geo.t_pad = t_pad;
     geo.nw = p.nw;
-    geo.leave_crowded = job.T > kLevelAlone;
+    geo.leave_crowded = !p.alone;
     if (geo.leave_crowded) {
         if (const hipError_t err = launch_crowded(job, p.us, stream, why); err != hipSuccess)
             return err;

@@ -130,7 +130,7 @@ SIGNATURES: dict[str, tuple[type, list]] = {
     "ramnet_segment_plan": (_c_int, [
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int),
         ctypes.POINTER(_c_int)]),
-    "ramnet_segment_call_form": (_c_int, [_c_i64] * 7 + [_c_int, _c_int, ctypes.POINTER(_c_int)]),
+    "ramnet_segment_call_form": (_c_int, [_c_i64] * 7 + [_c_int, _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int)]),
 }
 
 _lock = threading.Lock()
@@ -182,12 +182,13 @@ def segment_plan(B: int, H: int, A: int, C: int, w_top_k: int, r_top_k: int,
 
 
 def segment_call_form(B: int, H: int, T: int, A: int, C: int, w_top_k: int, r_top_k: int, dtype: torch.dtype,
-                      mass_aware: bool) -> tuple[int, int] | None:
-    """(form, slot ranges) of a segment forward of these sizes, or None if unsupported."""
-    ranges = _c_int(0)
+                      mass_aware: bool) -> tuple[int, int, int] | None:
+    """(form, slot ranges, form for crowded addresses) of a segment forward of
+    these sizes, or None if unsupported."""
+    ranges, crowded = _c_int(0), _c_int(0)
     form = lib().ramnet_segment_call_form(B, H, T, A, C, w_top_k, r_top_k, DTYPE_CODES[dtype], int(mass_aware),
-                                          ctypes.byref(ranges))
-    return None if form < 0 else (form, ranges.value)
+                                          ctypes.byref(ranges), ctypes.byref(crowded))
+    return None if form < 0 else (form, ranges.value, crowded.value)
 
 
 def scan_workspace_bytes(B: int, H: int, T: int, w_top_k: int, r_top_k: int) -> int:

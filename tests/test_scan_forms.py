@@ -20,6 +20,22 @@ def test_workspace_holds_every_call(K, T):
     for A in SLOTS:
         ws = nat.segment_workspace_bytes(B, H, T, A, C, K, K, torch.bfloat16)
         for mass_aware in (False, True):
-            form, ranges = nat.segment_call_form(B, H, T, A, C, K, K, torch.bfloat16, mass_aware)
+            form, ranges, _ = nat.segment_call_form(B, H, T, A, C, K, K, torch.bfloat16, mass_aware)
             sums = B * H * T * C * 4 if ranges > 1 else 0
             assert ws >= nat.scan_workspace_bytes(B, H, T, K, K) + sums, (A, mass_aware, form, ranges)
+
+
+# what the planner answers where it takes no level-scheduled form: one token a step, in ranges or not
+ONE_TOKEN, LEVEL = (0, 1, 2), 3
+
+
+@pytest.mark.parametrize("mass_aware", [False, True])
+@pytest.mark.parametrize("K", [4, 8, 16, 24])
+def test_crowded_calls_have_a_form(K, mass_aware):
+    """Every call that may leave crowded addresses to another form has one, and
+    wider slot spaces than any whole one-token layout are scanned in ranges."""
+    for A in SLOTS:
+        for T in (65, 100, 300, 1024, 4096):
+            form, ranges, crowded = nat.segment_call_form(B, H, T, A, C, K, K, torch.bfloat16, mass_aware)
+            assert crowded in ONE_TOKEN, (A, T, form, ranges, crowded)
+            assert (ranges == 1) == (A <= 10912), (A, T, form, ranges)
