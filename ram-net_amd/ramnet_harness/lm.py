@@ -67,6 +67,14 @@ def has_hooks(module: nn.Module) -> bool:
                                                        "_global_backward_hooks", "_global_backward_pre_hooks"))
 
 
+def is_plain(t: torch.Tensor) -> bool:
+    """Whether an operator without derivative, batching or tracing rules loses
+    nothing of t: no gradient wanted, no forward-mode tangent, no subclass and
+    no tensor of a ``torch.func`` transform."""
+    return (type(t) in (torch.Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and not (torch.is_grad_enabled() and t.requires_grad) and forward_ad.unpack_dual(t).tangent is None)
+
+
 class RamLayer(nn.Module):
     """The operator's caller: projections, scaling, gamma, read-out norm and gate."""
 
@@ -138,10 +146,8 @@ class RamLayer(nn.Module):
         if type(norm) is not nn.RMSNorm or norm.weight is None or norm.eps is None:
             return False
         from ramnet_ops.impl._ops import readout_fits  # (needs the built library, as y does)
-        wants_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (y, gate, norm.weight))
-        return (not wants_grad and not torch.compiler.is_compiling() and not torch.is_autocast_enabled("cuda")
-                and not has_hooks(norm)
-                and forward_ad.unpack_dual(gate).tangent is None and readout_fits(y, gate, norm.weight))
+        return (not torch.compiler.is_compiling() and not torch.is_autocast_enabled("cuda") and not has_hooks(norm)
+                and all(is_plain(t) for t in (y, gate, norm.weight)) and readout_fits(y, gate, norm.weight))
 
 
 class SwiGLU(nn.Module):

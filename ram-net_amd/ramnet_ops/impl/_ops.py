@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from .. import _native as nat
 
@@ -724,9 +725,11 @@ def readout_fits(y: Tensor, gate: Tensor, weight: Tensor) -> bool:
 @torch.library.custom_op(f"{_NS}::readout", mutates_args=(), device_types="cuda")
 def readout(y: Tensor, gate: Tensor, weight: Tensor, eps: float) -> Tensor:
     """``sigmoid(gate) * rms_norm(y, weight, eps)`` over y's last dimension, in
-    the shape of gate (no gradient)."""
+    the shape of gate (no gradient; a forward-mode tangent is refused)."""
     op = "readout"
     _require_gpu(op, y, gate, weight)
+    if any(forward_ad.unpack_dual(t).tangent is not None for t in (y, gate, weight)):
+        raise NotImplementedError(f"{op}: no forward-mode derivative")
     C = y.shape[-1]
     _check_shapes(op, weight=(weight, (C,)))
     if gate.numel() != y.numel() or not y.dtype == gate.dtype == weight.dtype:

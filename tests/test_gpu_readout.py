@@ -94,3 +94,57 @@ def test_layer_choice():
     assert ((fused.double() - plain.double()).abs() <= 4.1 * UNIT[torch.bfloat16] * plain.double().abs()).all()
     out, _ = layer(x.clone().requires_grad_(), (None, None), pos, False)
     assert out.requires_grad and torch.equal(out, plain)
+
+
+def _small_layer():
+    from ramnet_harness import HarnessConfig
+    from ramnet_harness.lm import RamLayer
+    cfg = HarnessConfig(d_model=64, heads=4, value_chs=32, addr_order=2, addr_radix=8, top_k=4, embed_num=2)
+    torch.manual_seed(1)
+    layer = RamLayer(cfg)
+    layer.init_weights()
+    layer = layer.to(DEV).requires_grad_(False)
+    layer.out = torch.nn.Identity()
+    x = torch.randn(2, 9, 64, device=DEV)
+    pos = torch.arange(9, device=DEV).view(1, 9).expand(2, 9)
+    return layer, lambda weight: torch.func.functional_call(layer, {"out_norm.weight": weight},
+                                                            (x, (None, None), pos, False))[0]
+
+
+@pytest.mark.parametrize("grad_mode", [False, True])
+def test_layer_keeps_forward_mode(grad_mode):
+    """A tangent on the norm's weight alone reaches the output (which is linear
+    in the weight), through dual tensors and through torch.func.jvp."""
+    layer, call = _small_layer()
+    weight, tangent = layer.out_norm.weight.detach() + 0.5, torch.randn(32, device=DEV)
+    with torch.set_grad_enabled(grad_mode):
+        want = call(tangent)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(weight, tangent)
+            got = torch.autograd.forward_ad.unpack_dual(call(dual)).tangent
+        assert got is not None
+        torch.testing.assert_close(got, want, atol=1e-6, rtol=1e-5)
+        torch.testing.assert_close(torch.func.jvp(call, (weight,), (tangent,))[1], want, atol=1e-6, rtol=1e-5)
+
+
+def test_layer_keeps_vmap_and_grad_transforms():
+    """The norm's weight as a batch of torch.vmap, and as the argument of torch.func.grad."""
+    layer, call = _small_layer()
+    weights = torch.randn(3, 32, device=DEV)
+    with torch.no_grad():
+        got = torch.vmap(call)(weights)
+        torch.testing.assert_close(got, torch.stack([call(w) for w in weights]), atol=1e-6, rtol=1e-5)
+    up = torch.randn(2, 9, 128, device=DEV)
+    grad = torch.func.grad(lambda w: (call(w) * up).sum())(weights[0])
+    basis = torch.stack([(call(e) * up).sum() for e in torch.eye(32, device=DEV)])
+    torch.testing.assert_close(grad, basis, atol=1e-4, rtol=1e-4)
+
+
+def test_readout_refuses_tangents():
+    y, gate, weight = _make(4, 32, torch.float32)
+    for at in range(3):
+        with torch.autograd.forward_ad.dual_level():
+            args = [y, gate, weight]
+            args[at] = torch.autograd.forward_ad.make_dual(args[at], torch.ones_like(args[at]))
+            with pytest.raises(NotImplementedError, match="forward-mode"):
+                torch.ops.ramnet_ops.readout(*args, 1e-6)
