@@ -503,9 +503,14 @@ static hipError_t pack_decoded(const ramnet::SegmentJob &job, const int32_t *add
 }
 
 // A workspace that holds no read sums offers none to the launch, which then
-// refuses a scan in slot ranges instead of writing past its end.
+// refuses a scan in slot ranges instead of writing past its end; one that
+// holds the decoder records alone leaves it the mass-wave form.
 static void fit_workspace(ramnet::SegmentJob &job, int64_t workspace_bytes) {
     const int64_t records = scan_workspace_bytes(job.B, job.H, job.T, job.Kw, job.Kr);
+    if (workspace_bytes < records) {
+        job.gain = nullptr;
+        job.flags = nullptr;
+    }
     if (job.dtype != RAMNET_F32 && workspace_bytes < records + static_cast<int64_t>(job.B) * job.H * job.T * job.C * 4)
         job.yacc = nullptr;
 }
@@ -1198,10 +1203,13 @@ int ramnet_ram_attn_forward_noalloc(const void *w_addr, const void *r_addr, cons
                            fits_int({B * H * A * C, B * H * (A + 2), B * H * T * C,
                                      B * H * (T + ramnet::kScanPad) * (w_top_k + r_top_k)});
     if (plausible) {
+        // where the scratch holds the decoder records alone, the planner's
+        // choice among the forms that may need no more
+        const bool whole = scan_workspace_bytes(B, H, T, w_top_k, r_top_k) <= RAMNET_NOALLOC_SCRATCH_BYTES;
         int pre = 0;
         RAMNET_REQUIRE(ramnet::segment_plan(static_cast<int>(B), static_cast<int>(H), static_cast<int>(T),
                                             static_cast<int>(A), static_cast<int>(C), static_cast<int>(w_top_k),
-                                            static_cast<int>(r_top_k), dtype, nullptr, nullptr, &pre),
+                                            static_cast<int>(r_top_k), dtype, nullptr, nullptr, &pre, nullptr, whole),
                        "ram_attn_forward_noalloc: shape outside the LDS-resident scan (top_k <= 128)");
         // the decoder records; the precomputed-gain form adds the gain
         // records and, in slot ranges with 16-bit y, the fp32 read sums

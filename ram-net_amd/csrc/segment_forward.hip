@@ -327,7 +327,7 @@ bool plan_level_call(int B, int H, int A, int C, int kmax, int elem, int n_cu, i
 }
 
 bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, int T, Plan *out,
-               const SavedRows *sv = nullptr, bool mass_aware = true) {
+               const SavedRows *sv = nullptr, bool mass_aware = true, bool level_ok = true) {
     const int kmax = std::max(Kw, Kr);
     if (kmax > 2 * kWave || A < 1)
         return false;
@@ -337,7 +337,7 @@ bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, i
     // 1.07x at A = 144, 0.77x at A = 64; K = 16, 0.78x at A = 256 (T = 1500)
     // and 0.6x at 512 (T = 84), 1.5x at A = 1728 (K = 12).
     const int64_t writes = static_cast<int64_t>(kTile) * kmax;
-    if (!sv && B > 0 && T > 1 && (kmax <= 8 ? 2 * writes <= 3 * static_cast<int64_t>(A) : 5 * writes <= 3 * static_cast<int64_t>(A)) &&
+    if (level_ok && !sv && B > 0 && T > 1 && (kmax <= 8 ? 2 * writes <= 3 * static_cast<int64_t>(A) : 5 * writes <= 3 * static_cast<int64_t>(A)) &&
         plan_level_call(B, H, A, C, kmax, elem, n_cu, T, mass_aware, out))
         return true;
     *out = Plan{};
@@ -1492,8 +1492,9 @@ static int layout_override(const SegmentJob &job, Plan *p, const char **why) {
 
 // The layout a launch of this job uses: the override, else the planner's
 // choice for the job's B, H, dtype and this device's CU count. A job that
-// saves rows takes the override only where it can save them.
-static bool pick_plan(const SegmentJob &job, Plan *p, const char **why) {
+// saves rows takes the override only where it can save them. level_ok: the
+// workspace holds the level-scheduled form's schedule.
+static bool pick_plan(const SegmentJob &job, Plan *p, const char **why, bool level_ok = true) {
     if (job.save.w) {
         const SavedRows &sv = job.save;
         const int forced = layout_override(job, p, why);
@@ -1511,7 +1512,7 @@ static bool pick_plan(const SegmentJob &job, Plan *p, const char **why) {
     if (forced < 0)
         return false;
     if (!forced && !make_plan(job.B, job.H, job.A, job.C, job.Kw, job.Kr, dtype_bytes(job.dtype), cu_count(), job.T, p, nullptr,
-                              job.mass_aware != 0)) {
+                              job.mass_aware != 0, level_ok)) {
         *why = "segment forward: shape outside the LDS-resident scan (top_k <= 128; slot spaces wider than one "
                "resident slice are scanned in at most 4096 slot ranges)";
         return false;
@@ -1538,10 +1539,10 @@ static SegmentJob plan_job(int B, int H, int T, int A, int C, int Kw, int Kr, in
 // that is not mass-aware; `ranges` is the larger of the two, as the workspace
 // that it sizes serves both.
 int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int *cs, int *lds_bytes, int *pre,
-                 int *ranges) {
+                 int *ranges, bool level_ok) {
     Plan p{}, q{};
     const char *why = nullptr;
-    if (!pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 0), &p, &why))
+    if (!pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 0), &p, &why, level_ok))
         return 0;
     if (cs)
         *cs = p.cs;
@@ -1550,7 +1551,7 @@ int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, i
     if (pre)
         *pre = p.pre ? 1 : 0;
     if (ranges)
-        *ranges = pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 1), &q, &why) ? std::max(p.nr, q.nr) : p.nr;
+        *ranges = pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 1), &q, &why, level_ok) ? std::max(p.nr, q.nr) : p.nr;
     return 1;
 }
 
@@ -1672,7 +1673,7 @@ hipError_t launch_segment_forward(const SegmentJob &job, hipStream_t stream, con
     if (static_cast<int64_t>(job.B) * job.H == 0)
         return hipSuccess;
     Plan p{};
-    if (!pick_plan(job, &p, why))
+    if (!pick_plan(job, &p, why, job.gain && job.flags))
         return hipErrorInvalidValue;
     if (job.T == 0) {
         // no events: the final state is the initial state (a kernel, not a

@@ -39,3 +39,19 @@ def test_crowded_calls_have_a_form(K, mass_aware):
             form, ranges, crowded = nat.segment_call_form(B, H, T, A, C, K, K, torch.bfloat16, mass_aware)
             assert crowded in ONE_TOKEN, (A, T, form, ranges, crowded)
             assert (ranges == 1) == (A <= 10912), (A, T, form, ranges)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the calls would launch on pointers that are not memory")
+@pytest.mark.parametrize("T,C", [(3072, 32), (3072, 64), (4096, 64), (4096, 128)])
+def test_noalloc_takes_records_that_fit(T, C):
+    """Decoder records that fit the scratch where the other forms' do not: the
+    mass-wave form, which needs no more, takes the call (which here ends for
+    want of a device, not at the scratch check)."""
+    B, H, U, P, K = 8, 16, 2, 32, 16
+    assert nat.scan_workspace_bytes(B, H, T, K, K) > 192 << 20
+    fake = 0x1000
+    rc = nat.lib().ramnet_ram_attn_forward_noalloc(
+        fake, fake, fake, fake, 2, None, 8, fake, fake, fake + 64, fake + 128, fake + 192, fake + 256, B, H, U, P, T,
+        P ** U, C, K, K, 0.0, 0.0, 0, 1e-12, None)
+    message = nat.lib().ramnet_last_error().decode()
+    assert rc != nat.RAMNET_EINVAL and "scratch;" not in message, message

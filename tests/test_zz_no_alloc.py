@@ -173,3 +173,17 @@ def test_noalloc_refuses_shapes_beyond_the_scratch():
     assert rc == nat.RAMNET_EINVAL
     msg = nat.lib().ramnet_last_error().decode()
     assert "scratch" in msg and str(192 << 20) in msg, msg
+
+
+def test_noalloc_records_alone_fit():
+    """Decoder records that fit the scratch where the level-scheduled form's
+    schedule does not: the mass-wave form serves the call (its sums run in
+    another order than those of the workspace call)."""
+    nat = _nat()
+    B, H, U, P, T, C, K = 8, 16, 2, 32, 3072, 32, (16, 16)
+    assert nat.scan_workspace_bytes(B, H, T, *K) > 192 << 20
+    case = make_case(B, H, U, P, T, C, seed=11).to(DEV)
+    got, want = (_launch(nat, case, U, P, K, 8, (0.0, 0.0), False, noalloc) for noalloc in (True, False))
+    for name, a, b in zip(("y", "slot", "mass"), got, want):
+        err = ((a.double() - b.double()).norm() / b.double().norm()).item()
+        assert err <= 1e-5, f"{name} rel err {err:.3e}"
