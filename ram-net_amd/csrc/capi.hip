@@ -398,12 +398,12 @@ static int64_t scan_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t Kw,
 // them itself). `plan_ok` is false for shapes the scan does not take.
 static int64_t range_sum_bytes(int64_t B, int64_t H, int64_t T, int64_t A, int64_t C, int64_t Kw, int64_t Kr,
                                int dtype, bool *plan_ok = nullptr) {
-    int ranges = 1;
+    int ranges = 0;
     const bool ok = B > 0 && H > 0 && T >= 0 && A > 0 && A < kAddressLimit && C > 0 && Kw > 0 && Kr > 0 &&
                     valid_dtype(dtype) && fits_int({B * H * A * C, B * H * (A + 2), B * H * T * C}) &&
-                    ramnet::segment_plan(static_cast<int>(B), static_cast<int>(H), static_cast<int>(T),
-                                         static_cast<int>(A), static_cast<int>(C), static_cast<int>(Kw),
-                                         static_cast<int>(Kr), dtype, nullptr, nullptr, nullptr, &ranges);
+                    (ranges = ramnet::segment_ranges(static_cast<int>(B), static_cast<int>(H), static_cast<int>(T),
+                                                     static_cast<int>(A), static_cast<int>(C), static_cast<int>(Kw),
+                                                     static_cast<int>(Kr), dtype)) > 0;
     if (plan_ok)
         *plan_ok = ok;
     return ok && ranges > 1 && dtype != RAMNET_F32 ? B * H * T * C * 4 : 0;
@@ -1209,7 +1209,7 @@ int ramnet_ram_attn_forward_noalloc(const void *w_addr, const void *r_addr, cons
         int pre = 0;
         RAMNET_REQUIRE(ramnet::segment_plan(static_cast<int>(B), static_cast<int>(H), static_cast<int>(T),
                                             static_cast<int>(A), static_cast<int>(C), static_cast<int>(w_top_k),
-                                            static_cast<int>(r_top_k), dtype, nullptr, nullptr, &pre, nullptr, whole),
+                                            static_cast<int>(r_top_k), dtype, nullptr, nullptr, &pre, whole),
                        "ram_attn_forward_noalloc: shape outside the LDS-resident scan (top_k <= 128)");
         // the decoder records; the precomputed-gain form adds the gain
         // records and, in slot ranges with 16-bit y, the fp32 read sums

@@ -270,11 +270,13 @@ hipError_t launch_autoregressive(const DecodeJob &job, hipStream_t stream, const
 int stair_buffer(int P, int K, int NPD);
 hipError_t launch_autoregressive_steps(const DecodeJob &job, int S, hipStream_t stream, const char **why);
 
-// Channel-slice width, dynamic LDS bytes, form (1: precomputed gains) and
-// number of slot ranges that a segment-scan launch of this shape uses on the
-// current device. level_ok: its workspace holds more than the decoder records.
+// Channel-slice width, dynamic LDS bytes and form (1: precomputed gains) that
+// a segment-scan launch of this shape uses on the current device (0: not
+// supported). level_ok: its workspace holds more than the decoder records.
 int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int *cs, int *lds_bytes, int *pre,
-                 int *ranges = nullptr, bool level_ok = true);
+                 bool level_ok = true);
+// The slot ranges that calls of this shape may need (0: not supported).
+int segment_ranges(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype);
 // The form of one call (-1: not supported), its slot ranges, and the form
 // that takes it where its addresses are crowded.
 enum : int { kFormMassWave = 0, kFormGains = 1, kFormPaired = 2, kFormLevel = 3 };

@@ -35,6 +35,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 
@@ -85,12 +86,16 @@ struct Plan {
     int tp = 1;   // tokens per wave step: 2 = the paired scan (precomputed-gain form, one range);
                   // kLevelPlan = the level-scheduled scan (vec channels per lane)
     int km = 0;   // level-scheduled scan: padded events per token
-    double us = 0;  // and its estimated time
-    bool alone = false;  // level-scheduled scan: takes crowded calls too
+    double us = 0;  // its estimated time, in this many rounds of resident workgroups
+    int64_t rounds = 1;
+    bool alone = false;  // it takes crowded calls too; else those with more
+    double late = 0;     // late levels a chunk than this go to another form;
+    bool other_pre = false;     // the planner's choice among those: with a pre-pass,
+    int64_t other_cycles = 0;   // and its estimate
 };
 constexpr int kLevelPlan = 3;
-// Calls of at most this many tokens are never left to the one-token scan: its
-// launch costs more than their levels can.
+// Calls of at most this many tokens are never left to another form: its
+// launches cost more than their levels can.
 constexpr int kLevelAlone = 2 * kScanPad;
 
 // Cost model of one layout, in cycles per token of one round of resident
@@ -153,16 +158,21 @@ static bool save_layout_ok(const SavedRows *sv, int vec, int epp, int np, int cs
 
 // The best layout for slot ranges of AL slots (the whole space when AL == A);
 // forms: mass wave allowed (mass_ok), precomputed gains allowed (pre_ok);
-// sv: the layout saves rows in those slices.
+// sv: the layout saves rows in those slices. crowded: of layouts estimated
+// alike, the one that spreads over the most CUs, up to one workgroup each (the
+// lanes of crowded addresses meet in the same LDS rows; mass wave, 16 heads, T
+// = 2048, A = 1024, K = 16: 382 us with two state waves, 586 with four; 32
+// heads, T = 4096, K = 8: 488 with two on 256 CUs, 552 with one on half a CU
+// each, 521 with four).
 static bool plan_layout(int B, int H, int AL, int A_full, int C, int kmax, int elem, int n_cu, int T, bool mass_ok,
-                        bool pre_ok, Plan *out, int64_t *best_cost, const SavedRows *sv = nullptr, bool pair_ok = true) {
+                        bool pre_ok, Plan *out, int64_t *best_cost, const SavedRows *sv = nullptr, bool crowded = false) {
     const int64_t tt = std::max(1, T);
     const int epp0 = std::min(kWave, std::max(4, pow2_ceil(kmax)));
     bool found = false;
-    int64_t best = 0;
+    int64_t best = 0, best_spread = 0;
     // paired scan: the precomputed-gain form over the whole slot space, one
     // pass of events
-    if (!sv && pair_ok && pre_ok && AL == A_full && AL <= kMaxPairSlots && pair_records_fit(kmax, T)) {
+    if (!sv && pre_ok && AL == A_full && AL <= kMaxPairSlots && pair_records_fit(kmax, T)) {
         for (int epp = 2; epp <= kWave / 2; epp <<= 1) {
             if (epp < kmax)
                 continue;
@@ -227,11 +237,17 @@ static bool plan_layout(int B, int H, int AL, int A_full, int C, int kmax, int e
                         cost += tt * kPrePassCycles + kPrePassLaunchCycles;
                     // ties: fewer channels per lane (less work per wave), then
                     // more waves, then wider slices
+                    const bool idle = epp > std::max(8, epp0);  // event lanes without an event
+                    const int64_t spread = crowded && units <= n_cu && !idle ? 4 * units - np : 0;
                     const bool better =
                         !found || cost < best ||
-                        (cost == best && (vec < out->vec || (vec == out->vec && (nw > out->nw ||
-                                                                                 (nw == out->nw && cs > out->cs)))));
+                        (cost == best &&
+                         (vec < out->vec ||
+                          (vec == out->vec && (spread != best_spread
+                                                   ? spread > best_spread
+                                                   : nw > out->nw || (nw == out->nw && cs > out->cs)))));
                     if (better) {
+                        best_spread = spread;
                         *out = {vec, epp, np, nw, cs, lds, pre != 0};
                         out->tp = 1;
                         best = cost;
@@ -295,6 +311,7 @@ bool plan_level(int B, int H, int A, int C, int kmax, int n_cu, int T, bool mass
             if (!found || cost < best) {
                 *out = p;
                 out->us = best = cost;
+                out->rounds = rounds;
                 found = true;
             }
         }
@@ -302,28 +319,85 @@ bool plan_level(int B, int H, int A, int C, int kmax, int n_cu, int T, bool mass
     return found;
 }
 
-// The one-token layout that takes a crowded call from the level-scheduled
-// scan (estimated at `us`). Each launch that returns at once takes about 4
-// us, so the pre-pass form is for calls of kCrowdedPreUs and more, and for
-// those whose mass-wave form does not fit in LDS.
+// The layout that takes a crowded call from the level-scheduled scan
+// (estimated at `us`): the planner's choice among the other forms in calls of
+// kCrowdedPreUs and more. Each launch that returns at once takes about 4 us,
+// so shorter ones take the mass-wave form, which is one launch, unless its
+// estimate is beyond kCrowdedWaveCost of the pre-pass forms' (where it does
+// not hold a whole round in LDS: 16 heads, T = 2048, A = 4096, K = 8, crowded,
+// 580 us in the mass-wave form and 344 in the paired one), or it would also
+// scale the reads of a call that the planner gives to those forms (24 heads, T
+// = 1835, A = 1024, K = 6, mass-aware: 366 us, and 221 paired).
 constexpr double kCrowdedPreUs = 200;
-bool plan_crowded(int B, int H, int A, int C, int kmax, int elem, int n_cu, int T, double us, Plan *out) {
+constexpr double kCrowdedWaveCost = 1.1;
+bool plan_crowded(int B, int H, int A, int C, int kmax, int elem, int n_cu, int T, bool mass_aware, const Plan &level,
+                  Plan *out) {
     const SavedRows *none = nullptr;
-    int64_t cost = 0;
-    if (plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, true, us >= kCrowdedPreUs, out, &cost, none, false))
-        return true;
-    return us < kCrowdedPreUs && plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, false, true, out, &cost, none, false);
+    // (short calls of wide slot spaces are state copies, for which wide slices are best)
+    const bool spread = A <= 8 * static_cast<int64_t>(T);
+    int64_t cost = 0, all_cost = 0;
+    const bool any = level.us >= kCrowdedPreUs;
+    bool ok = plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, true, any, out, &cost, none, spread);
+    const double most = (mass_aware ? 1.0 : kCrowdedWaveCost) * static_cast<double>(level.other_cycles);
+    if (!any && level.other_pre && (!ok || static_cast<double>(cost) > most))
+        ok = plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, false, true, out, &all_cost, none, spread);
+    return ok;
 }
 
-// Whether the planner's level-scheduled layout serves this call: alone, or
-// beside a one-token layout for crowded addresses. Slot spaces wider than
-// any of those (A > 10912) keep the scan in slot ranges.
+// The mean number of late levels a chunk up to which the level-scheduled
+// layout p is faster than the other forms, whose best takes `cycles` by its
+// estimate: in proportion to their time for a chunk and round, with less of it
+// for a level the more events a token has. Crossing points measured, heads
+// alike, bf16 unless said (and the limit here): 128 heads T = 4096 A = 1024 K
+// = 8, 4.3 (4.2); 32 such heads, 4.2 (4.6); 32 heads T = 8192 A = 4096 K = 16,
+// 3.0 (2.7); 32 heads T = 2048 A = 256 K = 8, 5.2 (4.6), K = 4, 6.1 (6.8); 32
+// heads T = 1024 A = 1024 K = 10, 4.5 (4.4); 16 heads T = 512 K = 8, 4.6 (5.0),
+// T = 128, 5.0 (5.4); mass-aware 16 heads T = 1024 A = 4096 K = 16, 1.9 (1.9),
+// 18 heads T = 1237 A = 576 K = 6, 8.7 (7.6).
+double level_limit(const Plan &p, int B, int H, int A, int C, int kmax, int T, bool mass_aware, const Plan &other,
+                   int64_t cycles) {
+    // (a mass wave that also scales the reads takes 1.7 times as long; the
+    // others' state copy, which the level-scheduled scan makes in wide pieces,
+    // takes 0.5 us a MB more)
+    const double us = static_cast<double>(cycles) / 2400 * (mass_aware && !other.pre ? 1.7 : 1.0) +
+                      0.5e-6 * 4 * B * H * static_cast<double>(A) * C;
+    const double chunks = (T + kTile - 1) / kTile;
+    return us / chunks / static_cast<double>(p.rounds) * (0.8 + 5.8 / kmax) / (mass_aware ? 1.2 : 1.0);
+}
+
+// One head may have this many times the mean's limit: its levels are cheaper
+// while the other workgroups of its CU have finished (128 heads, K = 8: six
+// concentrated ones may have 5.7 to 6.4 late levels a chunk).
+constexpr double kCrowdedHead = 1.6;
+
+// Late levels a chunk of evenly spread addresses, by the writes per slot and
+// chunk: 1.3 to 1.4 at 1/16, 2.2 at 1/4, 2.6 to 3.2 at 1/2, 3.9 at 1.
+double spread_levels(int A, int kmax) { return 0.6 + 3.3 * std::sqrt(static_cast<double>(kTile) * kmax / A); }
+
+// Whether the planner's level-scheduled layout serves this call. A short call
+// runs it alone. A longer one launches another form beside it for crowded
+// addresses, and takes it where spread ones stay under its limit with some
+// room (64 heads, T = 2048, A = 1024, K = 16: 424 us, and 343 with the
+// one-token scan) and a whole layout of another form fits (A up to 10912:
+// wider slot spaces keep the scan in slot ranges).
 bool plan_level_call(int B, int H, int A, int C, int kmax, int elem, int n_cu, int T, bool mass_aware, Plan *out) {
-    Plan crowded{};
+    Plan other{};
+    int64_t cost = 0;
     if (!plan_level(B, H, A, C, kmax, n_cu, T, mass_aware, out))
         return false;
-    out->alone = T <= kLevelAlone;
-    return out->alone || plan_crowded(B, H, A, C, kmax, elem, n_cu, T, out->us, &crowded);
+    if (T <= kLevelAlone) {
+        // where a chunk's writes are many for the slots, levels pile up even
+        // for spread addresses: K = 8, 0.77x of the one-token forms at A = 64
+        // (T = 1500); K = 16, 0.6x at A = 512 (T = 84)
+        out->alone = true;
+        return 10 * kTile * kmax <= (kmax <= 8 ? 15 : 6) * static_cast<int64_t>(A);
+    }
+    if (!plan_layout(B, H, A, A, C, kmax, elem, n_cu, T, true, true, &other, &cost))
+        return false;
+    out->late = level_limit(*out, B, H, A, C, kmax, T, mass_aware, other, cost);
+    out->other_pre = other.pre;
+    out->other_cycles = cost;
+    return spread_levels(A, kmax) + 0.2 < out->late;
 }
 
 bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, int T, Plan *out,
@@ -332,12 +406,7 @@ bool make_plan(int B, int H, int A, int C, int Kw, int Kr, int elem, int n_cu, i
     if (kmax > 2 * kWave || A < 1)
         return false;
     int64_t cost = 0;
-    // Where a chunk's writes are many for the slots, levels pile up even for
-    // evenly spread addresses. Against the one-token forms: K = 8, T = 1500,
-    // 1.07x at A = 144, 0.77x at A = 64; K = 16, 0.78x at A = 256 (T = 1500)
-    // and 0.6x at 512 (T = 84), 1.5x at A = 1728 (K = 12).
-    const int64_t writes = static_cast<int64_t>(kTile) * kmax;
-    if (level_ok && !sv && B > 0 && T > 1 && (kmax <= 8 ? 2 * writes <= 3 * static_cast<int64_t>(A) : 5 * writes <= 3 * static_cast<int64_t>(A)) &&
+    if (level_ok && !sv && B > 0 && T > 1 &&
         plan_level_call(B, H, A, C, kmax, elem, n_cu, T, mass_aware, out))
         return true;
     *out = Plan{};
@@ -660,7 +729,7 @@ __device__ __forceinline__ void mass_fetch(const MassLanes<MP, HALF> &ln, const 
 // past the last (b, h) repeating it); LDS holds (a, b) per slot and unit.
 template<int MP, int NU = 1>
 __global__ __launch_bounds__(kWave) void mass_chunk_map_kernel(const SegmentJob job, float2 *maps, int t_pad,
-                                                              int chunk_len, int crowded) {
+                                                              int chunk_len, const int *decision) {
     static_assert(NU == 1 || MP == 1, "several units per wave: one pass of events");
     constexpr int HALF = kWave / NU / 2;
     using L = MassLanes<MP, HALF>;
@@ -672,7 +741,7 @@ __global__ __launch_bounds__(kWave) void mass_chunk_map_kernel(const SegmentJob 
     const int ck = blockIdx.y, nck = gridDim.y;
     const int lane = static_cast<int>(threadIdx.x);
     const int bh = min(static_cast<int>(blockIdx.x) * NU + lane / (2 * HALF), n_bh - 1);
-    if (crowded && !level_crowded(job.flags, n_bh, t_pad, job.T))
+    if (decision && *decision >= 0)
         return;
     const bool wlane = (lane / HALF) % 2 == 0;
     const int A = job.A, Kw = job.Kw, Kr = job.Kr;
@@ -753,13 +822,12 @@ __global__ __launch_bounds__(kWave) void mass_chunk_map_kernel(const SegmentJob 
 
 // Step 2: one thread per (b, h, slot); the map of chunk c is replaced by
 // (m_start of chunk c, unused).
-__global__ __launch_bounds__(256) void mass_chunk_scan_kernel(const SegmentJob job, float2 *maps, int nck, int crowded) {
+__global__ __launch_bounds__(256) void mass_chunk_scan_kernel(const SegmentJob job, float2 *maps, int nck,
+                                                              const int *decision) {
     const int A = job.A;
     const int64_t n = static_cast<int64_t>(job.B) * job.H * A;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (crowded && !level_crowded(job.flags, job.B * job.H, scan_t_pad(job.T), job.T))  // (by whole waves)
-        return;
-    if (i >= n)
+    if (i >= n || (decision && *decision >= 0))
         return;
     const int64_t bh = i / A;
     const int a = static_cast<int>(i - bh * A);
@@ -799,7 +867,8 @@ __global__ __launch_bounds__(256) void mass_chunk_scan_kernel(const SegmentJob j
 // (whose predecessor another chunk replays) is flagged.
 template<bool MA, int MP, int AUX = 0, int NU = 1, bool FL = false>
 __global__ __launch_bounds__(kWave) void segment_mass_kernel(const SegmentJob job, int t_pad, int chunk_len,
-                                                            const float2 *starts, const MassAux aux, int crowded = 0) {
+                                                            const float2 *starts, const MassAux aux,
+                                                            const int *decision) {
     static_assert(NU == 1 || (MP == 1 && !AUX), "several units per wave: one pass of events, no AUX");
     static_assert(!(FL && AUX), "flags: the forward pre-pass only");
     constexpr int HALF = kWave / NU / 2;
@@ -812,7 +881,7 @@ __global__ __launch_bounds__(kWave) void segment_mass_kernel(const SegmentJob jo
     const int lane = static_cast<int>(threadIdx.x);
     const int unit = lane / (2 * HALF);
     const int bh = min(static_cast<int>(blockIdx.x) * NU + unit, n_bh - 1);
-    if (AUX == 0 && crowded && !level_crowded(job.flags, n_bh, t_pad, job.T))
+    if (AUX == 0 && decision && *decision >= 0)
         return;
     const int hl = lane % HALF;
     const bool wlane = (lane / HALF) % 2 == 0;
@@ -1034,7 +1103,8 @@ __global__ __launch_bounds__(kWave) void segment_mass_kernel(const SegmentJob jo
                 rwm |= unit_hit || first ? 1u << j : 0u;
             }
             const int jj = min(hl, min(CH, t_end - t0) - 1);
-            gfl[t0 + jj] = static_cast<int>((rwm >> jj) & 1u);
+            // (the flags share their words with the decision's bit 31)
+            gfl[t0 + jj] = static_cast<int>(((rwm >> jj) & 1u) | (decision ? 0x80000000u : 0u));
         }
     };
     const int nc = (t_end - t_begin + CH - 1) / CH;
@@ -1111,19 +1181,20 @@ size_t mass_lds_bytes(int A, bool aux, int nu = 1, bool fl = false) {
 // groups of NU.
 template<bool MA, int MP, int AUX, int NU>
 void launch_replay_units(const SegmentJob &job, int t_pad, int len, int nck, const float2 *starts, const MassAux &aux,
-                         int crowded, hipStream_t stream) {
+                         const int *decision, hipStream_t stream) {
     const unsigned groups = static_cast<unsigned>((job.B * job.H + NU - 1) / NU);
-    const bool fl = !AUX && job.flags && !crowded;
+    const bool fl = !AUX && job.flags;
     const dim3 grid(groups, static_cast<unsigned>(nck));
     if constexpr (!AUX) {
         if (fl) {
             hipLaunchKernelGGL((segment_mass_kernel<MA, MP, AUX, NU, true>), grid, dim3(kWave),
-                               mass_lds_bytes(job.A, false, NU, true), stream, job, t_pad, len, starts, aux);
+                               mass_lds_bytes(job.A, false, NU, true), stream, job, t_pad, len, starts, aux,
+                               decision);
             return;
         }
     }
     hipLaunchKernelGGL((segment_mass_kernel<MA, MP, AUX, NU>), grid, dim3(kWave), mass_lds_bytes(job.A, AUX != 0, NU),
-                       stream, job, t_pad, len, starts, aux, crowded);
+                       stream, job, t_pad, len, starts, aux, decision);
 }
 
 // Units per replay wave: four when a token has at most 8 events and the
@@ -1134,38 +1205,38 @@ void launch_replay_units(const SegmentJob &job, int t_pad, int len, int nck, con
 // slower with the time chunks halved to keep the wave count.
 template<bool MA, int MP, int AUX>
 void launch_mass_replay_nu(const SegmentJob &job, int t_pad, int len, int nck, const float2 *starts,
-                           const MassAux &aux, int crowded, hipStream_t stream) {
+                           const MassAux &aux, const int *decision, hipStream_t stream) {
     if constexpr (MP == 1 && !AUX) {
         if (std::max(job.Kw, job.Kr) <= 8 && mass_lds_bytes(job.A, false, 4, job.flags != nullptr) <= 64 * 1024)
-            return launch_replay_units<MA, MP, AUX, 4>(job, t_pad, len, nck, starts, aux, crowded, stream);
+            return launch_replay_units<MA, MP, AUX, 4>(job, t_pad, len, nck, starts, aux, decision, stream);
     }
-    launch_replay_units<MA, MP, AUX, 1>(job, t_pad, len, nck, starts, aux, crowded, stream);
+    launch_replay_units<MA, MP, AUX, 1>(job, t_pad, len, nck, starts, aux, decision, stream);
 }
 
 // `maps` is scratch for the chunk maps (maps_bytes of it); the final masses
-// go to job.mass_out. crowded: only for a call that the level-scheduled scan
-// leaves to the one-token scan.
+// go to job.mass_out. decision: only for a call that the level-scheduled scan
+// leaves (a word whose bit 31 says so).
 template<bool MA, int MP, int AUX>
 hipError_t launch_mass_pass_mp(const SegmentJob &job, int t_pad, int n_cu, void *maps_buf, size_t maps_bytes,
-                               const MassAux &aux, hipStream_t stream, int crowded = 0) {
+                               const MassAux &aux, hipStream_t stream, const int *decision = nullptr) {
     int len = 0;
     const int nck = mass_chunks(job, maps_bytes, n_cu, &len);
     const unsigned bh = static_cast<unsigned>(job.B * job.H);
     if (nck <= 1) {
-        launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, job.T, 1, nullptr, aux, crowded, stream);
+        launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, job.T, 1, nullptr, aux, decision, stream);
         return hipGetLastError();
     }
     auto *maps = static_cast<float2 *>(maps_buf);
     if (MP == 1 && std::max(job.Kw, job.Kr) <= 8 && static_cast<size_t>(job.A + 2) * 8 * 4 <= 64 * 1024)
         hipLaunchKernelGGL((mass_chunk_map_kernel<1, 4>), dim3((bh + 3) / 4, nck), dim3(kWave),
-                           static_cast<size_t>(job.A + 2) * 8 * 4, stream, job, maps, t_pad, len, crowded);
+                           static_cast<size_t>(job.A + 2) * 8 * 4, stream, job, maps, t_pad, len, decision);
     else
         hipLaunchKernelGGL((mass_chunk_map_kernel<MP>), dim3(bh, nck), dim3(kWave),
-                           static_cast<size_t>(job.A + 2) * 8, stream, job, maps, t_pad, len, crowded);
+                           static_cast<size_t>(job.A + 2) * 8, stream, job, maps, t_pad, len, decision);
     const int64_t n = static_cast<int64_t>(bh) * job.A;
     hipLaunchKernelGGL(mass_chunk_scan_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, job,
-                       maps, nck, crowded);
-    launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, len, nck, maps, aux, crowded, stream);
+                       maps, nck, decision);
+    launch_mass_replay_nu<MA, MP, AUX>(job, t_pad, len, nck, maps, aux, decision, stream);
     return hipGetLastError();
 }
 
@@ -1534,13 +1605,9 @@ static SegmentJob plan_job(int B, int H, int T, int A, int C, int Kw, int Kr, in
     return job;
 }
 
-// The mass-aware level-scheduled form holds more LDS, so near the LDS limit
-// the two kinds of call can differ in form. The layout is that of a call
-// that is not mass-aware; `ranges` is the larger of the two, as the workspace
-// that it sizes serves both.
 int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, int *cs, int *lds_bytes, int *pre,
-                 int *ranges, bool level_ok) {
-    Plan p{}, q{};
+                 bool level_ok) {
+    Plan p{};
     const char *why = nullptr;
     if (!pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 0), &p, &why, level_ok))
         return 0;
@@ -1550,9 +1617,36 @@ int segment_plan(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype, i
         *lds_bytes = static_cast<int>(p.lds);
     if (pre)
         *pre = p.pre ? 1 : 0;
-    if (ranges)
-        *ranges = pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, 1), &q, &why, level_ok) ? std::max(p.nr, q.nr) : p.nr;
     return 1;
+}
+
+// Whether a one-token layout holds the whole slot space.
+static bool whole_layout_fits(int A, int kmax, int elem) {
+    for (int pre = 1; pre >= 0; --pre)
+        for (int epp = kWave; epp >= 4; epp >>= 1)
+            for (int nw = 1; nw <= 4; nw <<= 1) {
+                const int np = (kmax + epp - 1) / epp;
+                if (np <= 2 && scan_layout_compiled(1, epp, np, nw, pre) && (!pre || A <= kMaxPrePassSlots) &&
+                    static_cast<int64_t>(scan_lds_bytes(A, 1, epp, np, nw, elem, pre)) + kLdsGranule <= kLdsPerCu)
+                    return true;
+            }
+    return false;
+}
+
+// One where a whole one-token layout fits, whatever form a call takes. Where
+// none does, the mass-aware level-scheduled form, which holds more LDS, may
+// not fit while the other does: the larger answer, as the workspace that it
+// sizes serves both kinds of call.
+int segment_ranges(int B, int H, int T, int A, int C, int Kw, int Kr, int dtype) {
+    const char *env = std::getenv("RAMNET_SCAN_LAYOUT"), *why = nullptr;
+    Plan p{};
+    if (!(env && *env) && whole_layout_fits(A, std::max(Kw, Kr), dtype_bytes(dtype)))
+        return 1;
+    int ranges = 0;
+    for (int mass_aware = 0; mass_aware < 2; ++mass_aware)
+        if (pick_plan(plan_job(B, H, T, A, C, Kw, Kr, dtype, mass_aware), &p, &why))
+            ranges = std::max(ranges, p.nr);
+    return ranges;
 }
 
 static int form_of(const Plan &p) {
@@ -1569,7 +1663,8 @@ int segment_call_form(int B, int H, int T, int A, int C, int Kw, int Kr, int dty
         *ranges = p.nr;
     if (crowded)
         *crowded = p.tp == kLevelPlan && !p.alone &&
-                           plan_crowded(B, H, A, C, std::max(Kw, Kr), dtype_bytes(dtype), cu_count(), T, p.us, &q)
+                           plan_crowded(B, H, A, C, std::max(Kw, Kr), dtype_bytes(dtype), cu_count(), T,
+                                        mass_aware != 0, p, &q)
                        ? form_of(q)
                        : form_of(p);
     return form_of(p);
@@ -1588,18 +1683,66 @@ static hipError_t launch_scan_layout(const SegmentJob &job, const ScanGeom &geo,
     }
 }
 
-// A call that the level-scheduled scan leaves as too crowded: the one-token
-// scan, whose waves return at once otherwise. It runs before the
-// level-scheduled scan: a pre-pass that is not needed leaves y and the final
-// masses alone, and one that is has read what it needs of the schedule
-// before the gain records replace it.
-static hipError_t launch_crowded(const SegmentJob &job, double us, hipStream_t stream, const char **why) {
-    Plan p{};
-    const int t_pad = scan_t_pad(job.T), n_cu = cu_count();
-    if (!plan_crowded(job.B, job.H, job.A, job.C, std::max(job.Kw, job.Kr), dtype_bytes(job.dtype), n_cu, job.T, us, &p)) {
-        *why = "segment forward: no one-token layout for a crowded call";
-        return hipErrorInvalidValue;
+static hipError_t launch_pair_layout(const SegmentJob &job, const ScanGeom &geo, const Plan &p, hipStream_t stream) {
+    switch (job.dtype) {
+        case kF32: return launch_scan_pair_f32(job, geo, p.vec, p.epp, p.nw, stream);
+        case kF16: return launch_scan_pair_f16(job, geo, p.vec, p.epp, p.nw, stream);
+        default: return launch_scan_pair_bf16(job, geo, p.vec, p.epp, p.nw, stream);
     }
+}
+
+// The answer of a call of more chunks than a wave counts: one workgroup.
+__global__ __launch_bounds__(kWave *kCrowdWaves) void crowd_kernel(const CrowdRule rule) {
+    __shared__ int sums[kCrowdWaves], worst[kCrowdWaves];
+    const int wave = static_cast<int>(threadIdx.x) / kWave;
+    const CrowdSums mine = crowd_sums(rule, wave * kCrowdWave);
+    if (threadIdx.x % kWave == 0) {
+        sums[wave] = mine.sum;
+        worst[wave] = mine.worst;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    CrowdSums all{0, 0};
+    for (int w = 0; w < static_cast<int>(blockDim.x) / kWave; ++w) {
+        all.sum += sums[w];
+        all.worst = max(all.worst, worst[w]);
+    }
+    if (crowd_over(rule, all))
+        rule.flags[0] |= static_cast<int>(0x80000000u);
+}
+
+static CrowdRule crowd_rule(const SegmentJob &job, const Plan &level, bool pre) {
+    CrowdRule r{};
+    r.flags = job.flags;
+    r.heads = job.B * job.H;
+    r.chunks = (job.T + kTile - 1) / kTile;
+    r.t_pad = scan_t_pad(job.T);
+    r.per = r.chunks;
+    const bool all = static_cast<int64_t>(r.heads) * r.chunks <= kCrowdWave;
+    if (!all) {
+        const int most = std::max(1, std::min({r.chunks, kCrowdSamples / r.heads, std::max(16, kCrowdWave / r.heads)}));
+        r.per = pow2_ceil(most) == most ? most : pow2_ceil(most) / 2;
+    }
+    // the widest aligned window that every head holds whole
+    const int window = pow2_ceil(r.per) == r.per ? r.per : pow2_ceil((r.per + 1) / 2 + 1) / 2;
+    r.window = std::min(std::max(window, 4), kCrowdWave);
+    const double late = std::min(level.late, 2.0 * kTile);
+    r.mean16 = static_cast<int>(16 * late);
+    r.worst16 = static_cast<int>(16 * kCrowdedHead * late);
+    r.decided = !all || pre;  // (the pre-pass forms overwrite what the waves would count)
+    return r;
+}
+
+// The form that takes a crowded call, whose waves return at once otherwise.
+// It runs before the level-scheduled scan: a pre-pass that is not needed
+// leaves y and the final masses alone, and one that is has read what it needs
+// of the schedule before the gain records replace it.
+static hipError_t launch_crowded(const SegmentJob &job, const Plan &p, const CrowdRule &rule, hipStream_t stream) {
+    const int t_pad = scan_t_pad(job.T);
+    SegmentJob fj = job;
+    if (p.tp != 2)
+        fj.flags = nullptr;
     ScanGeom geo{};
     geo.n_slices = (job.C + p.cs - 1) / p.cs;
     geo.n_units = job.B * job.H * geo.n_slices;
@@ -1607,17 +1750,18 @@ static hipError_t launch_crowded(const SegmentJob &job, double us, hipStream_t s
     geo.t_pad = t_pad;
     geo.n_local = job.A;
     geo.last = 1;
-    geo.crowded = 1;
+    geo.crowd = rule;
     if (p.pre) {
         const size_t y_bytes = static_cast<size_t>(job.B) * job.H * job.T * job.C * dtype_bytes(job.dtype);
-        const MassAux none_aux{};
-        const hipError_t err = job.mass_aware
-                                   ? launch_mass_pass_mp<true, 1, 0>(job, t_pad, n_cu, job.y, y_bytes, none_aux, stream, 1)
-                                   : launch_mass_pass_mp<false, 1, 0>(job, t_pad, n_cu, job.y, y_bytes, none_aux, stream, 1);
+        const MassAux none{};
+        const int n = kReplayChunkFactor * cu_count();
+        const hipError_t err =
+            job.mass_aware ? launch_mass_pass_mp<true, 1, 0>(fj, t_pad, n, job.y, y_bytes, none, stream, rule.flags)
+                           : launch_mass_pass_mp<false, 1, 0>(fj, t_pad, n, job.y, y_bytes, none, stream, rule.flags);
         if (err != hipSuccess)
             return err;
     }
-    return launch_scan_layout(job, geo, p, stream);
+    return p.tp == 2 ? launch_pair_layout(fj, geo, p, stream) : launch_scan_layout(fj, geo, p, stream);
 }
 
 // Event schedule, then the scan.
@@ -1646,9 +1790,22 @@ static hipError_t launch_level_scan(const SegmentJob &job, const Plan &p, hipStr
     geo.n_units = job.B * job.H * geo.n_slices;
     geo.t_pad = t_pad;
     geo.nw = p.nw;
-    geo.leave_crowded = !p.alone;
-    if (geo.leave_crowded) {
-        if (const hipError_t err = launch_crowded(job, p.us, stream, why); err != hipSuccess)
+    if (!p.alone) {
+        Plan other{};
+        if (!plan_crowded(job.B, job.H, job.A, job.C, std::max(job.Kw, job.Kr), dtype_bytes(job.dtype), cu_count(),
+                          job.T, job.mass_aware != 0, p, &other)) {
+            *why = "segment forward: no other form for a crowded call";
+            return hipErrorInvalidValue;
+        }
+        geo.crowd = crowd_rule(job, p, other.pre);
+        if (geo.crowd.decided) {
+            const int samples = std::min(geo.crowd.heads, kCrowdSamples / geo.crowd.per) * geo.crowd.per;
+            hipLaunchKernelGGL(crowd_kernel, dim3(1), dim3(kWave * ((samples + kCrowdWave - 1) / kCrowdWave)), 0, stream,
+                               geo.crowd);
+            if (const hipError_t err = hipGetLastError(); err != hipSuccess)
+                return err;
+        }
+        if (const hipError_t err = launch_crowded(job, other, geo.crowd, stream); err != hipSuccess)
             return err;
     }
     // whole slices, and x and y aligned for VEC elements at a time
@@ -1736,13 +1893,8 @@ hipError_t launch_segment_forward(const SegmentJob &job, hipStream_t stream, con
         if (err != hipSuccess)
             return err;
     }
-    if (p.tp == 2) {
-        switch (job.dtype) {
-            case kF32: return launch_scan_pair_f32(pj, geo, p.vec, p.epp, p.nw, stream);
-            case kF16: return launch_scan_pair_f16(pj, geo, p.vec, p.epp, p.nw, stream);
-            default: return launch_scan_pair_bf16(pj, geo, p.vec, p.epp, p.nw, stream);
-        }
-    }
+    if (p.tp == 2)
+        return launch_pair_layout(pj, geo, p, stream);
     // slot ranges in order: each adds its read sums to the fp32 sums of the
     // ranges before it, and the last stores y
     const int al = (job.A + p.nr - 1) / p.nr;

@@ -76,7 +76,7 @@ struct LevelGeom {
     int n_slices;  // ceil(C / (nw * CSW))
     int t_pad;
     int nw;        // state waves (1, 2 or 4)
-    int leave_crowded;  // 1: a crowded call is left to the one-token scan
+    CrowdRule crowd;  // set: a crowded call is left to another form
 };
 
 // LDS of a workgroup: the state regions, the masses, the stage ring and the
@@ -90,7 +90,7 @@ inline size_t level_lds_bytes(int A, int vec, int nw, int km, bool ma) {
 inline size_t schedule_lds_bytes(int A) { return static_cast<size_t>(A) * 2 * 4; }
 
 // One wave per 64 tokens (two tiles) of one (b, h), one token per lane.
-// Bound by its record traffic (40 bytes per event and side).
+// Bound by its record traffic (24 bytes per write and 16 per read).
 template<int KM>
 __global__ __launch_bounds__(kWave) void segment_schedule_kernel(const SegmentJob job, int t_pad) {
     constexpr int L = kTile;
@@ -277,8 +277,8 @@ __global__ __launch_bounds__(kWave *(kLevelMaxWaves + 1)) void segment_level_ker
     const int bh = unit / geo.n_slices;
     const int c0 = (unit - bh * geo.n_slices) * CS;
     const int A = job.A, C = job.C, T = job.T, Kw = job.Kw, Kr = job.Kr, Tp = geo.t_pad;
-    if (geo.leave_crowded && level_crowded(job.flags, job.B * job.H, Tp, T))
-        return;  // left to the one-token scan
+    if (geo.crowd.flags && crowded(geo.crowd))
+        return;
     const int rs = (A + 2) * CSW;  // floats per wave region
     constexpr int SV = CSW % 4 == 0 ? 4 : 2;  // floats per state access
     auto region = [&](int c) { return lds + c / CSW * rs + c % CSW; };  // slice channel c in slot 0

@@ -27,6 +27,70 @@ namespace ramnet {
 
 constexpr int kChunk = kScanChunk;
 
+// Crowded addresses. Each late level costs the level-scheduled scan
+// (segment_level.hpp) a part of a chunk's level-0 pass however few events it
+// holds, so where addresses crowd a few slots another form is faster. A call
+// launches both, and they decide alike from the schedule's counts (word 0 of
+// a chunk's 32, bits 0..7: its late levels): the other form takes the call
+// where a chunk has more than `mean16` / 16 late levels on average, or where
+// one head's chunks have more than `worst16` / 16 -- a workgroup holds a head
+// to its end, so one concentrated head makes a call wait for its levels (128
+// heads of 4096 tokens, top-K 8, six of them concentrated: 2667 us, and 887
+// where the one-token scan takes the call).
+//
+// `per` chunks of each head are looked at: all of them while a call has at
+// most kCrowdWave chunks, which each wave counts for itself; else a power of
+// two, spread evenly -- 16 a head where that fits, or more for few heads -- by
+// crowd_kernel, which leaves the answer in bit 31 of word 0 (decided). A head's mean is taken over aligned windows of `window`
+// samples, of which each head holds a whole one.
+struct CrowdRule {
+    int *flags;  // the schedule's counts, (heads, t_pad); null: the call has one form
+    int heads, chunks, t_pad, per, window;
+    int mean16, worst16;
+    int decided;
+};
+constexpr int kCrowdWave = 4 * kWave;            // samples of a wave
+constexpr int kCrowdWaves = 16;                  // waves of crowd_kernel, at most
+constexpr int kCrowdSamples = kCrowdWave * kCrowdWaves;
+
+// Samples first .. first + kCrowdWave - 1 of a call: the sum of their late
+// levels, and the largest sum of a window. By whole waves.
+struct CrowdSums {
+    int sum, worst;
+};
+__device__ __forceinline__ CrowdSums crowd_sums(const CrowdRule &r, int first) {
+    const int lane = static_cast<int>(threadIdx.x % kWave);
+    const int heads = min(r.heads, kCrowdSamples / r.per), n = heads * r.per, step = r.heads / heads;
+    int levels[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int i = min(first + 4 * lane + j, n - 1), h = i / r.per, k = i - h * r.per;
+        const int c = k * (r.chunks / r.per) + k * (r.chunks % r.per) / r.per;
+        levels[j] = r.flags[static_cast<int64_t>(h) * step * r.t_pad + c * kScanPad] & 0xff;
+    }
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        sum += first + 4 * lane + j < n ? levels[j] : 0;
+    int worst = sum;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        worst = 4 * d <= r.window / 2 ? worst + __shfl_xor(worst, d) : max(worst, __shfl_xor(worst, d));
+        sum += __shfl_xor(sum, d);
+    }
+    return {__builtin_amdgcn_readfirstlane(sum), __builtin_amdgcn_readfirstlane(worst)};
+}
+__device__ __forceinline__ bool crowd_over(const CrowdRule &r, const CrowdSums &s) {
+    const int n = min(r.heads, kCrowdSamples / r.per) * r.per;
+    return s.sum * 16 > r.mean16 * n || s.worst * 16 > r.worst16 * r.window;
+}
+// Whether the other form takes the call.
+__device__ __forceinline__ bool crowded(const CrowdRule &r) {
+    if (r.decided)
+        return r.flags[0] < 0;
+    return crowd_over(r, crowd_sums(r, 0));
+}
+
 struct ScanGeom {
     int n_units;  // B * H * n_slices
     int n_slices; // ceil(C / CS)
@@ -40,46 +104,9 @@ struct ScanGeom {
     int r0;
     int n_local;
     int last;
-    // 1: only a call that the level-scheduled scan leaves to this one
-    int crowded = 0;
+    // set: only a call that the level-scheduled scan leaves to this one
+    CrowdRule crowd{};
 };
-
-// Whether a call's addresses are too concentrated for the level-scheduled
-// scan (segment_level.hpp): each of its levels costs it about a third of a
-// chunk's level-0 pass however few events it holds, and its slowest heads
-// decide, so beyond kCrowdedMean late levels per 32-token chunk on average,
-// or with more than one chunk in kCrowdedPart past kCrowdedLevels, the
-// one-token scan takes the call. Both are launched and decide alike from the
-// schedule's counts (in the flags of the workspace: word 0 of each chunk,
-// bits 0..7) of at most 256 chunks spread over the call. At config 2 sizes
-// with a mean of m late levels: 280 + 82 m us against 725 us (m = 2.3 on the
-// benchmark data). Called by whole waves.
-constexpr int kCrowdedMean = 5;
-constexpr int kCrowdedLevels = 14;
-constexpr int kCrowdedPart = 16;
-__device__ __forceinline__ bool level_crowded(const int *flags, int n_heads, int t_pad, int T) {
-    const int lane = static_cast<int>(threadIdx.x % kWave), nc = (T + kScanPad - 1) / kScanPad;
-    const int64_t total = static_cast<int64_t>(n_heads) * nc;
-    const int n = static_cast<int>(min(total, static_cast<int64_t>(4 * kWave)));
-    int levels[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t c = min(i * kWave + lane, n - 1) * total / n;
-        const int64_t bh = c / nc;
-        levels[i] = flags[bh * t_pad + (c - bh * nc) * kScanPad] & 0xff;
-    }
-    int sum = 0, many = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const bool in = i * kWave + lane < n;
-        sum += in ? levels[i] : 0;
-        many += __popcll(__ballot(in && levels[i] > kCrowdedLevels));
-    }
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1)
-        sum += __shfl_xor(sum, d);
-    return __builtin_amdgcn_readfirstlane(sum) > kCrowdedMean * n || many * kCrowdedPart > n;
-}
 
 // 1/d refined by one Newton step; gain = w / (m + eps) to ~1 ulp.
 __device__ __forceinline__ float scan_gain(float w, float d) {
@@ -465,7 +492,7 @@ __device__ __forceinline__ void segment_scan_body(const SegmentJob &job, const S
     const int bh = unit / geo.n_slices;
     const int c0 = (unit - bh * geo.n_slices) * CS;
     const int T = job.T, A = job.A, C = job.C, Kw = job.Kw, Kr = job.Kr, Tp = geo.t_pad;
-    if (geo.crowded && !level_crowded(job.flags, job.B * job.H, Tp, T))
+    if (geo.crowd.flags && !crowded(geo.crowd))
         return;
     const float eps = job.eps;
     // resident slot range: [r0, r0 + AL) (the whole space but in the

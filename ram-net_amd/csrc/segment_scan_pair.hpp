@@ -84,6 +84,8 @@ __global__ __launch_bounds__(kWave * NW) void segment_scan_pair_kernel(const Seg
     const int lane = tid % kWave;
     const int bh = unit / geo.n_slices;
     const int c0 = (unit - bh * geo.n_slices) * CS;
+    if (geo.crowd.flags && !crowded(geo.crowd))
+        return;
     const int T = job.T, A = job.A, C = job.C, Tp = geo.t_pad;
     const int EK = job.Kw > job.Kr ? job.Kw : job.Kr;
     constexpr int RS = scan_row_stride(VEC, CS);
@@ -139,7 +141,7 @@ __global__ __launch_bounds__(kWave * NW) void segment_scan_pair_kernel(const Seg
         int4 rec[NPS];  // {write slot, gain, read slot, read weight} of token 2 s + tp, event ev
         Bits x[XIW];
         int ov;  // overlap bits of token t0 + lane (decoder, write event 0), lanes < CH
-        int rw;  // 1 if token t0 + lane writes a slot that token t0 + lane - 1 reads (mass pre-pass)
+        int rw;  // bit 0: 1 if token t0 + lane writes a slot that token t0 + lane - 1 reads (mass pre-pass)
     };
     // the head's gain records through a buffer resource: a lane offset fixed
     // for the whole sequence plus a wave-uniform offset per pair (no 64-bit
@@ -183,7 +185,7 @@ __global__ __launch_bounds__(kWave * NW) void segment_scan_pair_kernel(const Seg
         // hazard masks, bit j = token t0 + j (see the file comment)
         uint64_t m_ser, m_ww, m_rel;
         {
-            const int fv = lane < CH && t0 + lane < T ? (f.ov & 7) | (f.rw << 3) : 0;
+            const int fv = lane < CH && t0 + lane < T ? (f.ov & 7) | ((f.rw & 1) << 3) : 0;
             const bool odd = (lane & 1) != 0;
             m_ser = __ballot(odd && (fv & 9) != 0);
             m_ww = __ballot(odd && (fv & 1) != 0);
