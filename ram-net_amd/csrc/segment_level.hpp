@@ -95,6 +95,7 @@ template<int KM>
 __global__ __launch_bounds__(kWave) void segment_schedule_kernel(const SegmentJob job, int t_pad) {
     constexpr int L = kTile;
     extern __shared__ __align__(16) uint32_t masks[];
+    __shared__ int late[4][L + 1];  // per tile: positions holding a read, a write of each level
     const int A = job.A, Kw = job.Kw, Kr = job.Kr;
     const int per_head = (t_pad + kWave - 1) / kWave;
     const int bh = static_cast<int>(blockIdx.x) / per_head;
@@ -104,6 +105,8 @@ __global__ __launch_bounds__(kWave) void segment_schedule_kernel(const SegmentJo
     const int tc = in ? t : t_pad - 1;
     for (int i = lane; i < 2 * A; i += kWave)
         masks[i] = 0;
+    for (int i = lane; i < 4 * (L + 1); i += kWave)
+        (&late[0][0])[i] = 0;
     // (every load issued up front, from clamped event indices)
     const WriteRec *gw = job.wrec + static_cast<int64_t>(bh) * Kw * t_pad + tc;
     const ReadRec *gr = job.rrec + static_cast<int64_t>(bh) * Kr * t_pad + tc;
@@ -171,29 +174,26 @@ __global__ __launch_bounds__(kWave) void segment_schedule_kernel(const SegmentJo
             }
         }
     }
-    // positions per level of each chunk, and its levels
-    uint32_t *cnt = out.counts + tc / L * L;
-    uint32_t levels = 0;
-    for (uint32_t l = 1; l <= L; ++l) {
-        uint32_t n = 0;
+    // positions per level of each chunk, and its levels (contiguous from 1: an
+    // event of a level waits for one of each level below). Through LDS
+    // maxima: 34 us for 128 heads, T = 4096, K = 8, spread or crowded; a
+    // butterfly over the lanes per level took 35 us on spread addresses and
+    // 61 on crowded ones, whose chunks have up to 32 levels.
+    const int half = lane / kTile * 2;
 #pragma unroll
-        for (int k = 0; k < KM; ++k) {
-            const uint32_t nr = rl[k] == l ? rp[k] + 1 : 0, nw = wl[k] == l ? wp[k] + 1 : 0;
-            n = max(n & 0xffu, nr) | max(n & 0xff00u, nw << 8);
-        }
-#pragma unroll
-        for (int d = 1; d < L; d <<= 1) {
-            const uint32_t o = __shfl_xor(n, d);
-            n = max(n & 0xffu, o & 0xffu) | max(n & 0xff00u, o & 0xff00u);
-        }
-        levels = n != 0 ? (l == L ? l | n << 8 : l) : levels;
-        if (in & (tt == 0) & (l < L))
-            cnt[l] = n;
-        if (__ballot(n != 0) == 0)
-            break;
+    for (int k = 0; k < KM; ++k) {
+        if ((rl[k] != 0) & (rl[k] != 255u))
+            atomicMax(&late[half][rl[k]], rp[k] + 1);
+        if ((wl[k] != 0) & (wl[k] != 255u))
+            atomicMax(&late[half + 1][wl[k]], wp[k] + 1);
     }
-    if (in & (tt == 0))
-        cnt[0] = levels;
+    __syncthreads();
+    // lane l of a tile: level l, and level L in word 0
+    const uint32_t n = late[half][tt] | late[half + 1][tt] << 8, last = late[half][L];
+    const uint32_t any = static_cast<uint32_t>(__ballot((tt > 0) & (n != 0)) >> (lane / kTile * kTile));
+    const uint32_t levels = last != 0 ? L | last << 8 : any != 0 ? 31 - __clz(static_cast<int>(any)) : 0;
+    if (in)
+        out.counts[tc] = tt == 0 ? levels : n;
 }
 
 // Orders LDS accesses of different lanes for the compiler (the hardware runs
