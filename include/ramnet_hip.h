@@ -364,6 +364,10 @@ int ramnet_topk_autoregressive_steps_strided_(const void *w_addr, const void *r_
  */
 int ramnet_readout(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C, float eps,
                    void *out, void *stream);
+/* ramnet_readout with the norm and the sigmoid each rounded to dtype before
+ * their product is (the values of three operators that store them). */
+int ramnet_readout_stepwise(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C,
+                            float eps, void *out, void *stream);
 
 /*
  * One fused decode step on a persistent state, updated in place.

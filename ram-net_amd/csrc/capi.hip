@@ -1112,17 +1112,27 @@ int ramnet_topk_autoregressive_steps_strided_(const void *w_addr, const void *r_
                           C, w_top_k, r_top_k, w_re_norm, r_re_norm, mass_aware, eps, pos, true, y, stream);
 }
 
-int ramnet_readout(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C, float eps,
-                   void *out, void *stream) {
+static int readout(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C, float eps,
+                   bool stepwise, void *out, void *stream) {
     RAMNET_REQUIRE(rows >= 0 && C > 0 && C < kIntMax, "readout shape must have rows >= 0 and C > 0");
     RAMNET_REQUIRE(valid_dtype(dtype), "readout dtype must be float32, float16 or bfloat16");
     if (rows == 0)
         return RAMNET_OK;
     RAMNET_REQUIRE(y && gate && weight && out, "null tensor pointer");
-    const ramnet::ReadoutJob job{y, gate, weight, out, dtype, rows, static_cast<int>(C), eps};
+    const ramnet::ReadoutJob job{y, gate, weight, out, dtype, rows, static_cast<int>(C), eps, stepwise};
     const char *why = nullptr;
     const hipError_t err = ramnet::launch_readout(job, static_cast<hipStream_t>(stream), &why);
     return finish(err, why, "readout launch");
+}
+
+int ramnet_readout(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C, float eps,
+                   void *out, void *stream) {
+    return readout(y, gate, weight, dtype, rows, C, eps, false, out, stream);
+}
+
+int ramnet_readout_stepwise(const void *y, const void *gate, const void *weight, int dtype, int64_t rows, int64_t C,
+                            float eps, void *out, void *stream) {
+    return readout(y, gate, weight, dtype, rows, C, eps, true, out, stream);
 }
 
 // The query has no token count: it answers for a call of kPlanQueryTokens

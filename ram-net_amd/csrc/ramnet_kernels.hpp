@@ -260,6 +260,7 @@ struct ReadoutJob {
     int64_t rows;
     int C;
     float eps;
+    bool stepwise;            // norm and gate rounded to dtype before their product
 };
 hipError_t launch_readout(const ReadoutJob &job, hipStream_t stream, const char **why);
 hipError_t launch_autoregressive(const DecodeJob &job, hipStream_t stream, const char **why);

@@ -7,8 +7,9 @@
 // one element where C or an address is not a multiple of the piece), so the
 // row sum is a butterfly over registers, without LDS; each lane takes kRows
 // rows at once, so their loads are in flight together. All in fp32, rounded
-// once. 262144 rows of 128 bf16: 192 us for torch's row norm alone (one
-// block a row), 30 for its sigmoid and 30 for its product; 45 us here.
+// once; or with the norm and the gate each rounded to the rows' type first
+// (stepwise), as three kernels that store them would. 262144 rows of 128 bf16: 192 us for torch's row norm alone (one
+// block a row), 30 for its sigmoid and 30 for its product; 45 us here, 38 stepwise.
 #include "ramnet_device.hpp"
 #include "ramnet_kernels.hpp"
 
@@ -31,7 +32,19 @@ __device__ __forceinline__ void load_piece(const Scalar *p, float (&out)[VEC]) {
     }
 }
 
-template<typename Scalar, int VEC>
+// v as it is stored in the rows' type (bf16 through the compiler's type, which
+// rounds to nearest even with one instruction for two values).
+template<typename Scalar>
+__device__ __forceinline__ float stored(float v) {
+    if constexpr (sizeof(Scalar) == 4)
+        return v;
+    else if constexpr (__is_same(Scalar, bf16_t))
+        return static_cast<float>(static_cast<__bf16>(v));
+    else
+        return static_cast<float>(static_cast<_Float16>(v));
+}
+
+template<typename Scalar, int VEC, bool STEPWISE>
 __global__ __launch_bounds__(256) void readout_kernel(const ReadoutJob job, int lpr_log) {
     const int lpr = 1 << lpr_log;
     const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
@@ -65,8 +78,15 @@ __global__ __launch_bounds__(256) void readout_kernel(const ReadoutJob job, int 
             continue;
         float o[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e)
-            o[e] = yv[i][e] * scale * w[e] / (1.f + expf(-gv[i][e]));
+        for (int e = 0; e < VEC; ++e) {
+            // (rounded to 16 bits next, the quotient takes the hardware's reciprocal, good to one unit of fp32)
+            const float d = 1.f + expf(-gv[i][e]);
+            if constexpr (STEPWISE)
+                o[e] = stored<Scalar>(yv[i][e] * scale * w[e]) *
+                       stored<Scalar>(sizeof(Scalar) == 4 ? 1.f / d : __builtin_amdgcn_rcpf(d));
+            else
+                o[e] = yv[i][e] * scale * w[e] / d;
+        }
         Scalar *dst = static_cast<Scalar *>(job.out) + row * job.C + c;
         if constexpr (VEC == 1) {
             store_f32(dst, o[0]);
@@ -75,8 +95,12 @@ __global__ __launch_bounds__(256) void readout_kernel(const ReadoutJob job, int 
                 Scalar v[VEC];
             } packed;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                store_f32(&packed.v[e], o[e]);
+            for (int e = 0; e < VEC; ++e) {
+                if constexpr (__is_same(Scalar, bf16_t))
+                    packed.v[e].bits = __builtin_bit_cast(uint16_t, static_cast<__bf16>(o[e]));
+                else
+                    store_f32(&packed.v[e], o[e]);
+            }
             *reinterpret_cast<Out *>(dst) = packed;
         }
     }
@@ -102,10 +126,14 @@ hipError_t launch_typed(const ReadoutJob &job, hipStream_t stream, const char **
         return hipErrorInvalidValue;
     }
     const dim3 grid(static_cast<unsigned>(blocks));
-    if (wide)
-        hipLaunchKernelGGL((readout_kernel<Scalar, V>), grid, dim3(256), 0, stream, job, log);
-    else
-        hipLaunchKernelGGL((readout_kernel<Scalar, 1>), grid, dim3(256), 0, stream, job, log);
+#define RAMNET_READOUT(VEC, STEPWISE)                  \
+    if (wide == (VEC > 1) && job.stepwise == STEPWISE) \
+        hipLaunchKernelGGL((readout_kernel<Scalar, VEC, STEPWISE>), grid, dim3(256), 0, stream, job, log)
+    RAMNET_READOUT(V, false);
+    RAMNET_READOUT(V, true);
+    RAMNET_READOUT(1, false);
+    RAMNET_READOUT(1, true);
+#undef RAMNET_READOUT
     return hipGetLastError();
 }
 

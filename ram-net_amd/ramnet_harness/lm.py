@@ -133,7 +133,10 @@ class RamLayer(nn.Module):
             capture[-1]["y"] = y
         gate = self.gate(x)
         if self._fused_readout(y, gate):
-            return self.out(torch.ops.ramnet_ops.readout(y, gate, self.out_norm.weight, self.out_norm.eps)), new_state
+            # (rounded as the operators below round, so that a call's values do not
+            # depend on whether it wants a derivative or has a hook)
+            return self.out(torch.ops.ramnet_ops.readout(y, gate, self.out_norm.weight, self.out_norm.eps,
+                                                         stepwise=True)), new_state
         y = self.out_norm(y).flatten(-2)
         return self.out(torch.sigmoid(gate) * y), new_state
 

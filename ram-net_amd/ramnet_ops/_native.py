@@ -96,6 +96,7 @@ SIGNATURES: dict[str, tuple[type, list]] = {
         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
         _c_int, _c_float, _c_ptr, _c_i64, _c_i64s, _c_int, _c_ptr, _c_i64, _c_ptr]),
     "ramnet_readout": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_i64, _c_i64, _c_float, _c_ptr, _c_ptr]),
+    "ramnet_readout_stepwise": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_i64, _c_i64, _c_float, _c_ptr, _c_ptr]),
     "ramnet_topk_autoregressive_strided_": (_c_int, [
         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_float, _c_float,

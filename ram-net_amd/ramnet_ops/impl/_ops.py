@@ -723,9 +723,11 @@ def readout_fits(y: Tensor, gate: Tensor, weight: Tensor) -> bool:
 
 
 @torch.library.custom_op(f"{_NS}::readout", mutates_args=(), device_types="cuda")
-def readout(y: Tensor, gate: Tensor, weight: Tensor, eps: float) -> Tensor:
+def readout(y: Tensor, gate: Tensor, weight: Tensor, eps: float, stepwise: bool = False) -> Tensor:
     """``sigmoid(gate) * rms_norm(y, weight, eps)`` over y's last dimension, in
-    the shape of gate (no gradient; a forward-mode tangent is refused)."""
+    the shape of gate (no gradient; a forward-mode tangent is refused). Rounded
+    once; with ``stepwise`` the norm and the sigmoid are each rounded to the
+    tensors' dtype first, as by the three torch operators."""
     op = "readout"
     _require_gpu(op, y, gate, weight)
     if any(forward_ad.unpack_dual(t).tangent is not None for t in (y, gate, weight)):
@@ -737,13 +739,13 @@ def readout(y: Tensor, gate: Tensor, weight: Tensor, eps: float) -> Tensor:
     y, gate, weight = y.contiguous(), gate.contiguous(), weight.contiguous()
     out = torch.empty_like(gate, memory_format=torch.contiguous_format)
     with nat.on_device(y):
-        nat.call("ramnet_readout", y.data_ptr(), gate.data_ptr(), weight.data_ptr(), _code(y), y.numel() // C, C,
-                 float(eps), out.data_ptr(), nat.stream_of(y))
+        nat.call("ramnet_readout_stepwise" if stepwise else "ramnet_readout", y.data_ptr(), gate.data_ptr(),
+                 weight.data_ptr(), _code(y), y.numel() // C, C, float(eps), out.data_ptr(), nat.stream_of(y))
     return out
 
 
 @readout.register_fake
-def _(y, gate, weight, eps):
+def _(y, gate, weight, eps, stepwise=False):
     return torch.empty_like(gate, memory_format=torch.contiguous_format)
 
 

@@ -148,3 +148,39 @@ def test_readout_refuses_tangents():
             args[at] = torch.autograd.forward_ad.make_dual(args[at], torch.ones_like(args[at]))
             with pytest.raises(NotImplementedError, match="forward-mode"):
                 torch.ops.ramnet_ops.readout(*args, 1e-6)
+
+
+# torch's own fp32 values differ by a few units (its sum's order, its root), about 2**-21 of a value, and
+# turn a rounding to 16 bits where they straddle a boundary: 2**-21 of the values' spacing, 2**-8 or 2**-11,
+# in each of two roundings (a product rounds with them): under 1 in 400 elements, one unit each and its product's
+@pytest.mark.parametrize("dtype", list(UNIT))
+@pytest.mark.parametrize("rows,C", [(3, 24), (1000, 128), (257, 256)])
+def test_readout_stepwise(rows, C, dtype):
+    """Rounded step by step, the kernel gives the values of torch's three operators."""
+    y, gate, weight = _make(rows, C, dtype)
+    out = torch.ops.ramnet_ops.readout(y, gate, weight, 1e-6, stepwise=True)
+    want = torch.sigmoid(gate) * torch.nn.functional.rms_norm(y, (C,), weight, 1e-6)
+    off = (out.double() - want.double()).abs()
+    assert (off <= (4 * UNIT[dtype] if dtype != torch.float32 else _bound(C, dtype)) * want.double().abs() + 2.0 ** -24).all()
+    if dtype != torch.float32:
+        assert (off != 0).double().mean() <= 1 / 400 + 1 / off.numel()
+
+
+def test_layer_values_do_not_depend_on_the_form():
+    """The layer's fused read-out against its separate operators, which a hook
+    or a wanted gradient selects: equal but for single roundings."""
+    from ramnet_harness import HarnessConfig
+    from ramnet_harness.lm import RamLayer
+    cfg = HarnessConfig(d_model=256, heads=8, value_chs=128, addr_order=2, addr_radix=16, top_k=8, embed_num=4)
+    torch.manual_seed(2)
+    layer = RamLayer(cfg)
+    layer.init_weights()
+    layer = layer.to(DEV, torch.bfloat16)
+    layer.out = torch.nn.Identity()
+    x = torch.randn(2, 64, 256, device=DEV).to(torch.bfloat16)
+    pos = torch.arange(64, device=DEV).view(1, 64).expand(2, 64)
+    with torch.no_grad():
+        fused, _ = layer(x, (None, None), pos, False)
+        layer.out_norm.register_forward_hook(lambda *a: None)
+        plain, _ = layer(x, (None, None), pos, False)
+    assert (fused != plain).double().mean() <= 1 / 400
