@@ -148,7 +148,8 @@ def traffic_summary(out_dir: str) -> int:
     --copy-probe 1024``. FETCH_SIZE and WRITE_SIZE (KiB per dispatch,
     medians) are scaled by what they read for the 1 GiB copy."""
     import statistics
-    stage_names = SCAN_KERNELS + ("segment_schedule_kernel", "segment_mass_kernel", "mass_chunk_map_kernel", "mass_chunk_scan_kernel")
+    stage_names = SCAN_KERNELS + ("segment_schedule_kernel", "crowd_kernel", "segment_mass_kernel",
+                                  "mass_chunk_map_kernel", "mass_chunk_scan_kernel")
 
     def counters(path):
         vals = {}

@@ -36,7 +36,9 @@ struct AddrSource {
 // the precomputed-gain scan (B*H, T_pad, max(Kw, Kr)) of GainRec, token-major
 // so that the events of one token, which the scan's lanes load together,
 // are contiguous, then the paired scan's flags (B*H, T_pad) of int. The
-// decoder records are never modified after they are written, so one set of
+// level-scheduled scan keeps its schedule where the gain records are and its
+// counts where the flags are; bit 31 of the first flag is then a call's
+// answer to being crowded (CrowdRule in segment_scan.hpp). The decoder records are never modified after they are written, so one set of
 // records can be scanned any number of times.
 constexpr int kScanChunk = 16;
 constexpr int kScanPad = 2 * kScanChunk;

@@ -8,8 +8,10 @@
 // row sum is a butterfly over registers, without LDS; each lane takes kRows
 // rows at once, so their loads are in flight together. All in fp32, rounded
 // once; or with the norm and the gate each rounded to the rows' type first
-// (stepwise), as three kernels that store them would. 262144 rows of 128 bf16: 192 us for torch's row norm alone (one
-// block a row), 30 for its sigmoid and 30 for its product; 45 us here, 38 stepwise.
+// (stepwise), as three kernels that store them would. 262144 rows of 128
+// bf16: 192 us for torch's row norm alone (one block a row), 30 for its
+// sigmoid and 30 for its product; 45 us here, 38 stepwise (which takes a
+// reciprocal for a division).
 #include "ramnet_device.hpp"
 #include "ramnet_kernels.hpp"
 

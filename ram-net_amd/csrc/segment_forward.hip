@@ -349,11 +349,12 @@ bool plan_crowded(int B, int H, int A, int C, int kmax, int elem, int n_cu, int 
 // estimate: in proportion to their time for a chunk and round, with less of it
 // for a level the more events a token has. Crossing points measured, heads
 // alike, bf16 unless said (and the limit here): 128 heads T = 4096 A = 1024 K
-// = 8, 4.3 (4.2); 32 such heads, 4.2 (4.6); 32 heads T = 8192 A = 4096 K = 16,
-// 3.0 (2.7); 32 heads T = 2048 A = 256 K = 8, 5.2 (4.6), K = 4, 6.1 (6.8); 32
-// heads T = 1024 A = 1024 K = 10, 4.5 (4.4); 16 heads T = 512 K = 8, 4.6 (5.0),
-// T = 128, 5.0 (5.4); mass-aware 16 heads T = 1024 A = 4096 K = 16, 1.9 (1.9),
-// 18 heads T = 1237 A = 576 K = 6, 8.7 (7.6).
+// = 8, 4.3 (4.2); 32 such heads, 4.2 (4.5); 32 heads T = 8192 A = 4096 K = 16,
+// 3.0 (2.7); 32 heads T = 2048 A = 256 K = 8, 5.2 (4.6), K = 4, 6.1 (6.9); 32
+// heads T = 1024 A = 1024 K = 10, 4.5 (4.6); 16 heads T = 512 K = 8, 4.6 (4.9),
+// T = 128, 5.0 (5.5), T = 2048 A = 4096, 3.6 (5.0), A = 2744 K = 16, 2.9 (3.7);
+// mass-aware 16 heads T = 1024 A = 4096 K = 16, 1.9 (1.9), 18 heads T = 1237 A
+// = 576 K = 6, 8.7 (7.7).
 double level_limit(const Plan &p, int B, int H, int A, int C, int kmax, int T, bool mass_aware, const Plan &other,
                    int64_t cycles) {
     // (a mass wave that also scales the reads takes 1.7 times as long; the
@@ -378,8 +379,8 @@ double spread_levels(int A, int kmax) { return 0.6 + 3.3 * std::sqrt(static_cast
 // runs it alone. A longer one launches another form beside it for crowded
 // addresses, and takes it where spread ones stay under its limit with some
 // room (64 heads, T = 2048, A = 1024, K = 16: 424 us, and 343 with the
-// one-token scan) and a whole layout of another form fits (A up to 10912:
-// wider slot spaces keep the scan in slot ranges).
+// one-token scan) and a whole layout of another form fits (A up to about
+// 10.9k: wider slot spaces keep the scan in slot ranges).
 bool plan_level_call(int B, int H, int A, int C, int kmax, int elem, int n_cu, int T, bool mass_aware, Plan *out) {
     Plan other{};
     int64_t cost = 0;

@@ -55,7 +55,8 @@ constexpr int kLevelRing = 4;             // chunks of gains the mass wave may b
 //   counts  per chunk, word 0: its late levels n (bits 0..7), and the event
 //           positions holding a read of level L (bits 8..15); word l = 1 ..
 //           n: the positions holding a read (bits 0..7) and a write (bits
-//           8..15) of level l < L
+//           8..15) of level l < L. Bit 31 of the call's first word: another
+//           form takes the call (crowd_kernel)
 struct LevelSchedule {
     uint32_t *write, *mass;
     uint2 *read;

@@ -102,10 +102,13 @@ __device__ __forceinline__ void write_records(const AddrJob &job, int which, int
 // offsets (the host checks that every offset fits). kLaneRow / kLaneRowPart:
 // each address's U * P logits adjacent and aligned, P == NP / P < NP, in
 // 16-byte loads. kLaneAny: any strides, P <= NP, through 64-bit pointers.
-// The search, not the loads, bounds all of them: B 8, H 16, T 4096, P 32,
-// top-K 8 in bf16 takes 81 us from (B, H, U, P, T) and 80 us from (B, T, H,
-// U, P) rows, where each lane's row is its own cache line; bringing two such
-// tensors into memory order first took 87 us each.
+// The search, not the loads, bounds the first three: B 8, H 16, T 4096, P 32,
+// top-K 8 in bf16 takes 73 to 81 us from (B, H, U, P, T) and 78 to 80 us from
+// (B, T, H, U, P) rows, where each lane's row is its own cache line; bringing
+// two such tensors into memory order first took 87 us each. Rows whose digits
+// are no whole pieces (P 20, 25, 30 in bf16) take 147 us logit by logit, 109
+// at P 10 with three digits; their copy into memory order and the search
+// there together 212 to 360.
 enum : int { kLaneAny = 0, kLaneBuffer = 1, kLaneRow = 2, kLaneRowPart = 3 };
 template<typename Scalar, int NP, int KM, int LAY>
 // Occupancy: the per-lane search holds its digit in registers (about 210

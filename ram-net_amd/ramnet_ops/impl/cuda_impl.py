@@ -88,8 +88,8 @@ def _cuda_ram_attn(
 
     assert w_addr.dtype == r_addr.dtype == xs.dtype == gamma.dtype, \
         f"Expected matching dtypes, got w={w_addr.dtype}, r={r_addr.dtype}, x={xs.dtype}, gamma={gamma.dtype}."
-    assert w_addr.device == r_addr.device == xs.device == gamma.device == init_slot.device == init_mass.device \
-        == xs.device, "Expected all inputs on one device."
+    assert w_addr.device == r_addr.device == xs.device == gamma.device == init_slot.device \
+        == init_mass.device, "Expected all inputs on one device."
     expected_shapes = (
         ("w_addr", w_addr, (B, H, U, P, T)),
         ("r_addr", r_addr, (B, H, U, P, T)),

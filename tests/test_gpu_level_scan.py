@@ -63,10 +63,10 @@ def test_level_scan_layouts(layout, partial, monkeypatch):
 @pytest.mark.parametrize("case", [(2, 4, 2, 16, 200, 8, 6, True, True), (1, 2, 2, 16, 5000, 8, 8, False, False)],
                          ids=["short", "long"])
 def test_level_scan_crowded(case):
-    """Addresses concentrated on a few slots leave the call to the one-token
-    scan, launched before the level-scheduled one (mass-wave form for short
-    calls, pre-pass form for long ones); spread ones do not. Either way the
-    state and y are those of the event loop."""
+    """Spread addresses, and addresses concentrated on a few slots, which leave
+    the call to the mass-wave form launched before the level-scheduled one:
+    either way the state and y are those of the event loop. (Which form ran, and
+    the pre-pass and paired ones: test_gpu_scan_forms.py.)"""
     B, H, U, P, T, Kw, Kr, masked, mass_aware = case
     import ramnet_ops  # noqa: F401
     ops = torch.ops.ramnet_ops
